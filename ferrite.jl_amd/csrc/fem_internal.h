@@ -38,7 +38,7 @@ struct DevError {
   int detj_cell;     // cell id (0-based) with det(J) <= 0, INT_MAX if none
   int pattern_cell;  // cell id with a nonzero value for a missing pattern entry
   int pattern_entry; // local entry (col * nb + row) of that cell (valid when pattern_cell set)
-  int pad;
+  int pad;        // 1: the resident CG gave up waiting for another block
 };
 
 struct SolverWork;
@@ -59,12 +59,15 @@ struct Scal {
   int restart;    // breakdown happened: the next reseed restarts p = r̂
   int fresh;      // p, s = Â p and α were just set by a reseed: the next step only moves x̂, r̂
   int sfresh;     // (record written by k_cg_scal) the step k_cg_move runs now is such a step
-  int pad;
+  int pad;        // 1: the resident CG gave up waiting for another block
   // x̂ moves every other step: k_cg_move adds xa0 p_old + xa1 p_new (both 0: x̂ is not touched
   // and α p of this step is pending); pend = the α whose step's p is not yet in x̂ (k_fold
   // adds it)
   double xa0, xa1, pend;
   double rz0;     // γ at the last reseed (the host's batch-length choice)
+  // resident CG: products run, and (time_kernels) the 100 MHz clock ticks block 0 spent in them
+  long long prod_ticks;
+  int prods, pad2;
 };
 
 }  // namespace fem

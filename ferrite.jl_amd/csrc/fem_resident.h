@@ -1,0 +1,43 @@
+// Resident CG (fem_resident.hip): one launch runs the whole recurrence between two hand-overs
+// with the operator's rows, the vectors and the scalars on chip.
+#pragma once
+#include "fem_internal.h"
+
+namespace fem {
+
+// Where the rows of the scaled operator Â come from.  src 0: the columns of K's CSC arrays
+// (= rows, K is symmetric) scaled by sc; 1: lattice value planes; 2: the cell form (one
+// coefficient per cell, masked scaling t, class values f).  1 and 2 number the rows by the
+// padded lattice (dofp: the dof of a padded row, −1 on padding).
+struct ResSource {
+  int src = 0;
+  int64_t n = 0;                 // rows: dofs (0) or padded lattice rows (1, 2)
+  int dim = 0;                   // 1, 2: lattice dimension
+  int32_t px = 0, pxy = 0;
+  int64_t npad = 0;
+  const int32_t* dofp = nullptr;
+  const void* val = nullptr;     // 1: planes [s][npad]
+  const double* kc = nullptr;    // 2: k_c at the padded row of each cell's first corner
+  const void* t = nullptr;       // 2: masked scaling (X precision; 0 on prescribed rows and padding)
+  double f[8] = {};              // 2: K¹ per corner-offset class
+};
+
+struct ResOp;
+
+// Ready to run on `s` in FP32 or FP64 (structure once per pattern, values when K or the scaling
+// changed); *ok = false when the rows do not fit (the caller keeps the separate kernels).
+int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok);
+
+// One stretch of the recurrence: (re)seeded from the FP64 residual `res` (p, sv: the last
+// direction and Â times it), iterated until the hand-over or `lim` steps, x̂ folded into u.
+// dofp: the dof of a lattice row, or null.  The scalar record s goes in (rr, rzp, restart) and
+// out; s->pad = 1: gave up waiting for
+// another block (nothing was folded).  *launched = false: the device did not take the launch.
+template <typename X>
+int resident_run(fem_ctx* c, ResOp* op, const double* res, const double* sc, X* p, X* sv, double* u, Scal* s,
+                 const int32_t* dofp, double hold_factor2, double tol2, int restart, int lim,
+                 bool* launched);
+
+void resident_free(ResOp** op);
+
+}  // namespace fem

@@ -1,0 +1,1207 @@
+// Resident CG: the Chronopoulos–Gear recurrence of fem_solve.hip (same scalars, same hand-over
+// rule, same reseed) in one cooperative launch per stretch between two hand-overs.
+//
+// What bounds the separate kernels on systems of up to a few hundred thousand rows is not their
+// bytes but two launches per iteration.  Here every block (one per CU) owns a compact part of
+// the mesh and keeps on chip, for the whole stretch, its rows' operator entries (registers and
+// LDS, with 16-bit positions into the block's part of r̂), r̂ for its rows and for the rows they
+// couple to (LDS), and p, ŝ = Âp, x̂ (registers).  One exchange per iteration is left: a block publishes
+// w = Âr̂ of its rows and its partials of γ = r̂·r̂ and δ = r̂·w, and reads the others' partials
+// and the w of its coupled rows; with those it also moves the coupled rows' ŝ and r̂ itself
+// (the same operations on the same values as their owner, so they stay equal bit for bit), and
+// the next product needs no second exchange.
+//
+// The exchange has no barrier and no fence.  Every published value travels in 8-byte words of
+// 32 data bits and the exchange's 32-bit number, written and read with agent-scope accesses
+// (which reach the memory all XCDs share); a reader polls the words it needs until
+// they carry the number.  Two buffers alternate: a block writes exchange e + 2 only after it
+// holds every block's partials of e + 1, which they publish after reading all of e.  Partials
+// are summed in block order, so every block holds the same scalars and results are bitwise
+// reproducible.  Waits are bounded (kSpinLimit): a block that gives up reports it and stops
+// publishing, so every other block gives up too, and the host runs the separate kernels.
+//
+// Measured, µs per iteration, separate kernels → here: 100×100 Q1 quads FP64 11.7 → 3.0 (21
+// blocks); 24×20×17 distorted hexes FP64 17.4 → 3.6 (24); 64³ hexes FP64 33 → 6.1 (250); 512×256
+// Q1² quads FP64 26.5 → 3.95 (180); 301×227 Q1 quads FP32 cell form 13.3 → 4.0 and 47×53×61 hexes
+// FP32 planes 16.2 → 6.6 (both with their hand-overs).  At 100×100 an iteration is about 0.3 µs of
+// products, 0.3 µs of sums inside the block, 1.3 µs until the other blocks' values are there and
+// 0.5 µs of scalars and vector moves.
+#include <algorithm>
+#include <cmath>
+
+#include "fem_cell.h"
+#include "fem_resident.h"
+
+namespace fem {
+
+constexpr int kResT = 512;              // threads per block
+constexpr int kResWaves = kResT / 64;
+constexpr int kResMaxBlocks = 256;      // one per CU
+constexpr int kResCopies = 8;           // copies of a block's record
+constexpr uint32_t kSpinLimit = 1u << 22;
+constexpr int kResRows = 256;           // least rows per block when there are several
+
+constexpr size_t kRecWords = (size_t)2 * kResCopies * 2 * kResMaxBlocks * 4;
+
+struct ResOp {
+  int state = 0;                        // 1 usable, −1 does not fit
+  int64_t n = 0;                        // rows of the numbering
+  // parts: one block each; own rows (those other parts read first, each class ascending),
+  // coupled rows (ascending), published slots
+  int nb = 0, Rmax = 0, Rp = 0, nz = 0, nlocmax = 0, nhmax = 0, nslots = 0;
+  int32_t* oofs = nullptr;              // [nb + 1] ranges of orow
+  int32_t* orow = nullptr;              // own rows of each part
+  int32_t* pofs = nullptr;              // [nb + 1] published slots: one per row other parts read
+  int32_t* hoff = nullptr;              // [nb + 1] ranges of hrow, hslot
+  int32_t* hrow = nullptr;              // coupled rows of each part
+  int32_t* hslot = nullptr;             // ... and their published slots
+  uint32_t* ai = nullptr;               // [nb][nz2][Rp] positions of two entries each
+  // values per precision: [nb][nz][Rp]
+  float* val32 = nullptr;
+  double* val64 = nullptr;
+  uint64_t ver[2] = {0, 0}, aux[2] = {0, 0};
+  int jac[2] = {-1, -1}, vsrc[2] = {-1, -1};
+  // exchange buffers and the number of the last exchange handed out
+  uint32_t* wx = nullptr;               // [2][nslots] values (8 or 16 bytes each)
+  uint32_t* rec = nullptr;              // [2][kResCopies][2][kResMaxBlocks] values of 16 bytes
+  uint32_t epoch = 0;
+};
+
+void resident_free(ResOp** op) {
+  if (!*op) return;
+  ResOp* o = *op;
+  dev_free(&o->oofs); dev_free(&o->orow); dev_free(&o->pofs); dev_free(&o->hoff); dev_free(&o->hrow);
+  dev_free(&o->hslot); dev_free(&o->ai); dev_free(&o->val32); dev_free(&o->val64); dev_free(&o->wx); dev_free(&o->rec);
+  delete o;
+  *op = nullptr;
+}
+
+// ---- row access ---------------------------------------------------------------------------
+struct ResRows {
+  int src, dim;
+  int64_t n, npad;
+  int32_t px, pxy;
+  const int32_t *colptr, *rowval, *dofp;
+  const double *nzval, *sc, *kc;
+  const void *val, *t;
+  double f[8];
+};
+
+// Column of entry k of a row, −1 when the row has no such entry.  Lattice rows: entry k is the
+// neighbour with code k (3D, (dx + 1) + 3 (dy + 1) + 9 (dz + 1)) or 9 + k (2D).
+__device__ __forceinline__ int32_t res_col(const ResRows& a, int32_t row, int k) {
+  if (a.src == 0) {
+    const int32_t p = a.colptr[row] + k;
+    return p < a.colptr[row + 1] ? a.rowval[p] : -1;
+  }
+  if (a.dofp[row] < 0) return -1;
+  const int code = a.dim == 3 ? k : 9 + k;
+  const int32_t q = row + (code % 3 - 1) + a.px * ((code / 3) % 3 - 1) + (a.dim == 3 ? a.pxy * (code / 9 - 1) : 0);
+  return a.dofp[q] >= 0 ? q : -1;
+}
+
+// ---- parts --------------------------------------------------------------------------------
+// The rows are cut into sx × sy × sz compact parts of nearly equal size by nested quantiles of
+// their positions: slabs along x, each slab along y, each of those along z.  Compact parts read
+// few rows of others (a part of 1,000 rows of a 2D grid about 130, where a range of consecutive
+// rows reads 1,000): what the parts publish and read per iteration is what bounds it.
+constexpr int kResBins = 4096;
+
+// Bin of a row along each axis.  Lattice rows: their lattice index.  Others: the position of a
+// node of the row's first cell, scaled by the bounding box.
+struct ResPos {
+  int src, dim;
+  int64_t n;
+  int32_t px, pxy;
+  const int32_t *dofp, *node;        // node: [n]
+  const double* x[3];
+  double lo[3], inv[3];              // (x − lo) inv in [0, kResBins)
+};
+__device__ __forceinline__ bool res_pos(const ResPos& a, int32_t row, double (&x)[3]) {
+  x[1] = x[2] = 0.0;
+  if (a.src != 0) {
+    if (a.dofp[row] < 0) return false;
+    const int32_t z = a.dim == 3 ? row / a.pxy : 0, r = row - z * a.pxy, y = r / a.px;
+    x[0] = r - y * a.px;
+    x[1] = y;
+    x[2] = z;
+    return true;
+  }
+  const int32_t nd = a.node[row];
+  for (int d = 0; d < a.dim; ++d) x[d] = a.x[d][nd];
+  return true;
+}
+__device__ __forceinline__ int res_bin(const ResPos& a, const double (&x)[3], int d) {
+  return max(0, min(kResBins - 1, (int)((x[d] - a.lo[d]) * a.inv[d])));
+}
+
+// One block: bounding box of the rows (out[0..2], out[3..5]), their number (out[9]), and per axis
+// the mean over sampled rows of the largest distance to a row they couple to (out[6..8]): the
+// spacing of the rows.
+__global__ __launch_bounds__(1024) void k_res_geom(ResPos g, ResRows a, int nz, double* __restrict__ out) {
+  __shared__ double sh[10][16];
+  double v[10] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300, 0.0, 0.0, 0.0, 0.0};
+  for (int64_t row = threadIdx.x; row < g.n; row += 1024) {
+    double x[3];
+    if (!res_pos(g, (int32_t)row, x)) continue;
+    for (int d = 0; d < 3; ++d) {
+      v[d] = fmin(v[d], x[d]);
+      v[3 + d] = fmax(v[3 + d], x[d]);
+    }
+    v[9] += 1.0;
+  }
+  const int32_t s = (int32_t)(((int64_t)threadIdx.x * g.n) / 1024);
+  double xs[3], hs = 0.0;
+  if (res_pos(g, s, xs)) {
+    double far[3] = {0.0, 0.0, 0.0};
+    for (int k = 0; k < nz; ++k) {
+      const int32_t q = res_col(a, s, k);
+      double x[3];
+      if (q < 0 || !res_pos(g, q, x)) continue;
+      for (int d = 0; d < 3; ++d) far[d] = fmax(far[d], fabs(x[d] - xs[d]));
+    }
+    for (int d = 0; d < 3; ++d) v[6 + d] = far[d];
+    hs = 1.0;
+  }
+  for (int i = 0; i < 10; ++i)
+    for (int o = 32; o > 0; o >>= 1) {
+      const double u = __shfl_down(v[i], o, 64);
+      v[i] = i < 3 ? fmin(v[i], u) : i < 6 ? fmax(v[i], u) : v[i] + u;
+    }
+  for (int o = 32; o > 0; o >>= 1) hs += __shfl_down(hs, o, 64);
+  __shared__ double hsum[16];
+  if ((threadIdx.x & 63) == 0) {
+    for (int i = 0; i < 10; ++i) sh[i][threadIdx.x >> 6] = v[i];
+    hsum[threadIdx.x >> 6] = hs;
+  }
+  __syncthreads();
+  if (threadIdx.x < 10) {
+    const int i = threadIdx.x;
+    double r = sh[i][0], h = hsum[0];
+    for (int w = 1; w < 16; ++w) {
+      const double u = sh[i][w];
+      r = i < 3 ? fmin(r, u) : i < 6 ? fmax(r, u) : r + u;
+      h += hsum[w];
+    }
+    out[i] = i >= 6 && i < 9 ? r / fmax(h, 1.0) : r;
+  }
+}
+
+// One level of the cut along axis d: rows per (slab, bin), the finer slab of each (slab, bin),
+// the rows' finer slabs.  part starts as 0 (level 0).
+__global__ __launch_bounds__(256) void k_res_hist(ResPos g, int d, const int32_t* __restrict__ part,
+                                                  int32_t* __restrict__ hist) {
+  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < g.n; row += (int64_t)gridDim.x * 256) {
+    double x[3];
+    if (res_pos(g, (int32_t)row, x)) atomicAdd(&hist[(int64_t)part[row] * kResBins + res_bin(g, x, d)], 1);
+  }
+}
+__global__ __launch_bounds__(256) void k_res_cut(int s, int32_t* __restrict__ hist) {   // one block per slab
+  __shared__ int32_t sum[256];
+  int32_t* h = hist + (int64_t)blockIdx.x * kResBins;
+  constexpr int PER = kResBins / 256;
+  int32_t c[PER], all = 0;
+  for (int i = 0; i < PER; ++i) all += c[i] = h[threadIdx.x * PER + i];
+  sum[threadIdx.x] = all;
+  __syncthreads();
+  for (int o = 1; o < 256; o <<= 1) {
+    const int32_t v = (int)threadIdx.x >= o ? sum[threadIdx.x - o] : 0;
+    __syncthreads();
+    sum[threadIdx.x] += v;
+    __syncthreads();
+  }
+  const int64_t total = sum[255];
+  int64_t before = sum[threadIdx.x] - all;
+  for (int i = 0; i < PER; ++i) {   // the slab that holds the bin's middle row
+    const int64_t f = total > 0 ? (2 * before + c[i]) * s / (2 * total) : 0;
+    before += c[i];
+    h[threadIdx.x * PER + i] = (int32_t)min<int64_t>(f, s - 1);
+  }
+}
+__global__ __launch_bounds__(256) void k_res_split(ResPos g, int d, int s, const int32_t* __restrict__ hist,
+                                                   int32_t* __restrict__ part) {
+  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < g.n; row += (int64_t)gridDim.x * 256) {
+    double x[3];
+    if (!res_pos(g, (int32_t)row, x)) {
+      part[row] = -1;
+      continue;
+    }
+    const int32_t p = part[row];
+    part[row] = p * s + hist[(int64_t)p * kResBins + res_bin(g, x, d)];
+  }
+}
+
+// Rows that another part's rows name; the size of each part.
+__global__ __launch_bounds__(256) void k_res_shared(ResRows a, int nz, const int32_t* __restrict__ part,
+                                                    uint8_t* __restrict__ flag, int32_t* __restrict__ size) {
+  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < a.n; row += (int64_t)gridDim.x * 256) {
+    const int32_t p = part[row];
+    if (p < 0) continue;
+    atomicAdd(&size[p], 1);
+    for (int k = 0; k < nz; ++k) {
+      const int32_t q = res_col(a, (int32_t)row, k);
+      if (q >= 0 && part[q] != p) flag[q] = 1;
+    }
+  }
+}
+
+// The rows of each part, then (one block per part) sorted: rows other parts read first, each
+// class ascending; rank[row] = the row's place, shared[b] = how many other parts read.
+__global__ __launch_bounds__(256) void k_res_gather(int64_t n, const int32_t* __restrict__ part,
+                                                    const uint8_t* __restrict__ flag, const int32_t* __restrict__ oofs,
+                                                    int32_t* __restrict__ fill, int32_t* __restrict__ orow) {
+  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < n; row += (int64_t)gridDim.x * 256) {
+    const int32_t p = part[row];
+    if (p >= 0) orow[oofs[p] + atomicAdd(&fill[p], 1)] = (int32_t)row | (flag[row] ? 0 : 1 << 30);
+  }
+}
+__global__ __launch_bounds__(1024) void k_res_sort(int pow2, const int32_t* __restrict__ oofs,
+                                                   int32_t* __restrict__ orow, int32_t* __restrict__ rank,
+                                                   int32_t* __restrict__ shared) {
+  extern __shared__ int32_t res_key[];
+  __shared__ int ns;
+  const int32_t o0 = oofs[blockIdx.x], m = oofs[blockIdx.x + 1] - o0;
+  if (threadIdx.x == 0) ns = 0;
+  for (int i = threadIdx.x; i < pow2; i += 1024) res_key[i] = i < m ? orow[o0 + i] : INT_MAX;
+  __syncthreads();
+  for (int k = 2; k <= pow2; k <<= 1)
+    for (int j = k >> 1; j > 0; j >>= 1) {
+      for (int i = threadIdx.x; i < pow2; i += 1024) {
+        const int l = i ^ j;
+        if (l > i) {
+          const int32_t x = res_key[i], y = res_key[l];
+          if ((x > y) == ((i & k) == 0)) {
+            res_key[i] = y;
+            res_key[l] = x;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  int mine = 0;
+  for (int i = threadIdx.x; i < m; i += 1024) {
+    const int32_t v = res_key[i], row = v & ~(1 << 30);
+    mine += !(v & (1 << 30));
+    orow[o0 + i] = row;
+    rank[row] = i;
+  }
+  atomicAdd(&ns, mine);
+  __syncthreads();
+  if (threadIdx.x == 0) shared[blockIdx.x] = ns;
+}
+
+// A part's bitmap of the rows of other parts that its rows name, in LDS.
+__device__ __forceinline__ void res_mark(const ResRows& a, int nz, const int32_t* __restrict__ part,
+                                         const int32_t* __restrict__ own, int m, uint32_t* bm, int words) {
+  for (int i = threadIdx.x; i < words; i += blockDim.x) bm[i] = 0u;
+  __syncthreads();
+  for (int i = threadIdx.x; i < m; i += blockDim.x)
+    for (int k = 0; k < nz; ++k) {
+      const int32_t q = res_col(a, own[i], k);
+      if (q >= 0 && part[q] != (int32_t)blockIdx.x) atomicOr(&bm[q >> 5], 1u << (q & 31));
+    }
+  __syncthreads();
+}
+
+__global__ __launch_bounds__(256) void k_res_count(ResRows a, int nz, const int32_t* __restrict__ part,
+                                                   const int32_t* __restrict__ oofs,
+                                                   const int32_t* __restrict__ orow, int32_t* __restrict__ cnt) {
+  extern __shared__ uint32_t res_bm[];
+  __shared__ int tot;
+  const int words = (int)((a.n + 31) / 32);
+  if (threadIdx.x == 0) tot = 0;
+  res_mark(a, nz, part, orow + oofs[blockIdx.x], oofs[blockIdx.x + 1] - oofs[blockIdx.x], res_bm, words);
+  int all = 0;
+  for (int i = threadIdx.x; i < words; i += blockDim.x) all += __popc(res_bm[i]);
+  atomicAdd(&tot, all);
+  __syncthreads();
+  if (threadIdx.x == 0) cnt[blockIdx.x] = tot;
+}
+
+// The coupled rows of each part with their slots, and the entries' positions in its local
+// numbering: own rows by rank, then the coupled rows.
+__global__ __launch_bounds__(256) void k_res_fill(ResRows a, int nz, int Rp, const int32_t* __restrict__ part,
+                                                  const int32_t* __restrict__ rank, const int32_t* __restrict__ oofs,
+                                                  const int32_t* __restrict__ orow, const int32_t* __restrict__ pofs,
+                                                  const int32_t* __restrict__ hoff, int32_t* __restrict__ hrow,
+                                                  int32_t* __restrict__ hslot, uint32_t* __restrict__ ai) {
+  extern __shared__ uint32_t res_bm[];
+  const int words = (int)((a.n + 31) / 32);
+  const int ng = (words + 7) / 8;
+  uint32_t* pre = res_bm + words;    // [ng] rows before each group of 8 words
+  const int32_t o0 = oofs[blockIdx.x], m = oofs[blockIdx.x + 1] - o0, h0 = hoff[blockIdx.x];
+  res_mark(a, nz, part, orow + o0, m, res_bm, words);
+  for (int g = threadIdx.x; g < ng; g += blockDim.x) {
+    uint32_t c = 0;
+    for (int i = 8 * g; i < min(words, 8 * g + 8); ++i) c += __popc(res_bm[i]);
+    pre[g] = c;
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {            // exclusive scan by one wave
+    uint32_t base = 0;
+    for (int g0 = 0; g0 < ng; g0 += 64) {
+      const int g = g0 + (int)threadIdx.x;
+      const uint32_t v = g < ng ? pre[g] : 0u;
+      uint32_t s = v;
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t up = __shfl_up(s, o, 64);
+        if ((int)threadIdx.x >= o) s += up;
+      }
+      if (g < ng) pre[g] = base + s - v;
+      base += __shfl(s, 63, 64);
+    }
+  }
+  __syncthreads();
+  auto coupled = [&](int32_t q) {    // place of a marked row
+    const int w = q >> 5, g = w >> 3;
+    uint32_t l = pre[g];
+    for (int i = 8 * g; i < w; ++i) l += __popc(res_bm[i]);
+    return l + __popc(res_bm[w] & ((1u << (q & 31)) - 1u));
+  };
+  for (int i = threadIdx.x; i < words; i += blockDim.x) {
+    uint32_t bits = res_bm[i];
+    while (bits) {
+      const int32_t q = i * 32 + __ffs(bits) - 1;
+      bits &= bits - 1;
+      const int32_t h = h0 + (int32_t)coupled(q);
+      hrow[h] = q;
+      hslot[h] = pofs[part[q]] + rank[q];
+    }
+  }
+  const int nz2 = (nz + 1) / 2;
+  for (int32_t i = threadIdx.x; i < Rp; i += blockDim.x) {
+    const int32_t row = i < m ? orow[o0 + i] : -1;
+    for (int k2 = 0; k2 < nz2; ++k2) {
+      uint32_t pk = 0;
+      for (int h = 0; h < 2; ++h) {
+        const int32_t q = row >= 0 && 2 * k2 + h < nz ? res_col(a, row, 2 * k2 + h) : -1;
+        if (q >= 0) pk |= (part[q] == (int32_t)blockIdx.x ? (uint32_t)rank[q] : (uint32_t)m + coupled(q)) << (16 * h);
+      }
+      ai[((int64_t)blockIdx.x * nz2 + k2) * Rp + i] = pk;
+    }
+  }
+}
+
+// Values of the rows' entries in X precision (0 where an entry is missing).
+template <typename X>
+__global__ __launch_bounds__(256) void k_res_vals(ResRows a, int nz, int Rp, int nb, const int32_t* __restrict__ oofs,
+                                                  const int32_t* __restrict__ orow, X* __restrict__ val) {
+  for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < (int64_t)nb * Rp; g += (int64_t)gridDim.x * 256) {
+    const int b = (int)(g / Rp), i = (int)(g - (int64_t)b * Rp);
+    const int32_t o0 = oofs[b];
+    const bool in = i < oofs[b + 1] - o0;
+    const int64_t row = in ? orow[o0 + i] : 0;
+    X* out = val + (int64_t)b * nz * Rp + i;
+    if (a.src == 0) {
+      const int32_t p0 = in ? a.colptr[row] : 0, len = in ? a.colptr[row + 1] - p0 : 0;
+      const double sr = in ? a.sc[row] : 0.0;
+      for (int k0 = 0; k0 < nz; k0 += 9) {   // nz is a multiple of 9
+        double v[9], sj[9];
+#pragma unroll
+        for (int u = 0; u < 9; ++u) {
+          const bool real = k0 + u < len;
+          v[u] = real ? a.nzval[p0 + k0 + u] : 0.0;
+          sj[u] = real ? a.sc[a.rowval[p0 + k0 + u]] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < 9; ++u) out[(int64_t)(k0 + u) * Rp] = (X)(v[u] * (sr * sj[u]));
+      }
+      continue;
+    }
+    const bool real = in && a.dofp[row] >= 0;
+    if (a.src == 1) {
+      const X* val0 = static_cast<const X*>(a.val);
+      for (int k = 0; k < nz; ++k) {
+        const int32_t q = real ? res_col(a, (int32_t)row, k) : -1;
+        const int code = a.dim == 3 ? k : 9 + k;
+        X v = X(0);
+        if (q >= 0) v = code >= 13 ? val0[(int64_t)(code - 13) * a.npad + row] : val0[(int64_t)(13 - code) * a.npad + q];
+        out[(int64_t)k * Rp] = v;
+      }
+      continue;
+    }
+    // cell form: s_P s_Q f[class] Σ k over the cells that hold both corners, in FP64 and rounded
+    // once (Â stays symmetric to the last bit); a prescribed row (t = 0) keeps its unit diagonal
+    const X* tt = static_cast<const X*>(a.t);
+    const bool free_p = real && tt[row] != X(0);
+    const double sp = free_p ? a.sc[a.dofp[row]] : 0.0;
+    double k8[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const bool on = real && (a.dim == 3 || e < 4);
+      k8[e] = on ? a.kc[row - (e & 1) - (int64_t)a.px * ((e >> 1) & 1) - (int64_t)a.pxy * (e >> 2)] : 0.0;
+    }
+    for (int k = 0; k < nz; ++k) {
+      const int32_t q = real ? res_col(a, (int32_t)row, k) : -1;
+      const int code = a.dim == 3 ? k : 9 + k;
+      const int dx = code % 3 - 1, dy = (code / 3) % 3 - 1, dz = code / 9 - 1;
+      double ks = 0.0;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const bool both = (dx == 0 || (e & 1) == (dx < 0)) && (dy == 0 || ((e >> 1) & 1) == (dy < 0)) &&
+                          (dz == 0 || (e >> 2) == (dz < 0));
+        ks += both ? k8[e] : 0.0;
+      }
+      double v = 0.0;
+      if (q >= 0) {
+        if (free_p && tt[q] != X(0)) v = a.f[(dx != 0) + 2 * (dy != 0) + 4 * (dz != 0)] * ks * (sp * a.sc[a.dofp[q]]);
+        if (!free_p && q == row) v = 1.0;
+      }
+      out[(int64_t)k * Rp] = (X)v;
+    }
+  }
+}
+
+// ---- the recurrence -----------------------------------------------------------------------
+template <typename X>
+struct ResArgs {
+  int Rp, nb, nslots;
+  int nl, rl0;                // rows whose entries LDS holds; elements of r̂, ŝ and w there
+  int nhmax;
+  const int32_t *oofs, *orow, *pofs, *hoff, *hrow, *hslot;
+  const uint32_t* ai;
+  const X* val;
+  const int32_t* dofp;        // dof of a row (lattice rows), or null: the same index
+  const double *res, *sc;
+  X *p, *sv;
+  double* u;
+  Scal* s;
+  uint32_t *wx, *rec;
+  double hold2, tol2;
+  uint32_t epoch;
+  int restart, lim, time;
+};
+
+typedef unsigned int U4 __attribute__((ext_vector_type(4)));
+typedef unsigned int U2 __attribute__((ext_vector_type(2)));
+
+// Published values: an FP64 value as 16 bytes (low half, tag, high half, tag), an FP32 value as
+// 8 (bits, tag); each 8-byte word carries its own tag, so a reader may see the words of one
+// value at different times.  The buffer forms with sc1 are the agent-scope relaxed accesses
+// (write-through, and a read of what all XCDs share), 16 bytes wide.
+constexpr int kAgent = 16;              // sc1
+__device__ __forceinline__ void ll_put(__amdgpu_buffer_rsrc_t r, uint32_t at, double v, uint32_t tag) {
+  const long long bits = __double_as_longlong(v);
+  U4 q = {(uint32_t)bits, tag, (uint32_t)((unsigned long long)bits >> 32), tag};
+  __builtin_amdgcn_raw_buffer_store_b128(q, r, (int)(at * 16u), 0, kAgent);
+}
+__device__ __forceinline__ void ll_put(__amdgpu_buffer_rsrc_t r, uint32_t at, float v, uint32_t tag) {
+  U2 q = {__float_as_uint(v), tag};
+  __builtin_amdgcn_raw_buffer_store_b64(q, r, (int)(at * 8u), 0, kAgent);
+}
+template <typename X>
+struct LL;
+template <>
+struct LL<double> {
+  typedef U4 W;
+  static __device__ __forceinline__ W get(__amdgpu_buffer_rsrc_t r, uint32_t at) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, (int)(at * 16u), 0, kAgent);
+  }
+  static __device__ __forceinline__ bool ok(W v, uint32_t tag) { return v[1] == tag && v[3] == tag; }
+  static __device__ __forceinline__ double val(W v) {
+    return __longlong_as_double((long long)(((unsigned long long)v[2] << 32) | v[0]));
+  }
+};
+template <>
+struct LL<float> {
+  typedef U2 W;
+  static __device__ __forceinline__ W get(__amdgpu_buffer_rsrc_t r, uint32_t at) {
+    return __builtin_amdgcn_raw_buffer_load_b64(r, (int)(at * 8u), 0, kAgent);
+  }
+  static __device__ __forceinline__ bool ok(W v, uint32_t tag) { return v[1] == tag; }
+  static __device__ __forceinline__ float val(W v) { return __uint_as_float(v[0]); }
+};
+
+// Sum over the wave by DPP row shifts and broadcasts, valid in lane 63 (fixed order).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return v + __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double wave_sum63(double v) {
+  v = dpp_add<0x111, 0xf>(v);   // row_shr:1, 2, 4, 8: sums of 16 lanes in the row's last lane
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// Element of an LDS array at a byte offset.
+template <typename X>
+__device__ __forceinline__ X at_lds(const X* base, uint32_t boff) {
+  return *reinterpret_cast<const X*>(reinterpret_cast<const char*>(base) + boff);
+}
+
+// The kernel's argument block, through a pointer the compiler cannot trace.
+__device__ __forceinline__ const void* res_kernargs() {
+  const void* p = (const void*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+__device__ __forceinline__ void res_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Rows per thread RT; the entries (NZ per row) of the first RRES stay in registers, those of the
+// block's other rows (a.nl of them) in LDS.  LDS: r̂ of
+// the rows the block reads (own, coupled, and a zero slot for the threads' unused rows); ŝ, w and
+// the slots of the coupled rows; the entries of a.nl rows.
+template <typename X, int NZ, int RRES, int RT>
+__global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
+  constexpr int NZ2 = (NZ + 1) / 2;
+  constexpr int QS = NZ2 | 1;                 // a row's words in LDS (odd: no bank conflicts)
+  constexpr int H = sizeof(X) == 4 ? 8 : 4;   // coupled rows a thread polls at once
+  extern __shared__ __align__(16) unsigned char res_lds[];
+  __shared__ double red[2][2][kResWaves];    // wave sums, alternating
+  __shared__ double tot[2][2][4];            // sums of 64 blocks' partials each
+  __shared__ int gaveup;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const int b = blockIdx.x;
+  const int32_t o0 = a.oofs[b], nown = a.oofs[b + 1] - o0;
+  const int32_t p0 = a.pofs[b], npub = a.pofs[b + 1] - p0;
+  const int32_t h0 = a.hoff[b], nh = a.hoff[b + 1] - h0;
+  X* rl = reinterpret_cast<X*>(res_lds);
+  X* sl = rl + a.rl0;
+  X* wl = sl + a.nhmax;
+  X* lv = wl + a.nhmax;
+  uint32_t* lq = reinterpret_cast<uint32_t*>(lv + (size_t)NZ * a.nl);
+  int32_t* hl = reinterpret_cast<int32_t*>(lq + (size_t)QS * a.nl);
+  const int zero = nown + nh;
+  const double rzp0 = a.s->rzp, rr0 = a.s->rr;
+  const bool keep0 = !a.restart && !a.s->restart && rzp0 > 0.0;
+  if (t == 0) {
+    gaveup = 0;
+    rl[zero] = X(0);
+  }
+
+  // operator rows
+  X av[RRES][NZ];
+  uint32_t ai[RRES][NZ2];
+  const X* vb = a.val + (int64_t)b * NZ * a.Rp;
+  const uint32_t* ib = a.ai + (int64_t)b * NZ2 * a.Rp;
+#pragma unroll
+  for (int k = 0; k < RRES; ++k) {
+    const int i = t + k * kResT;
+    const bool in = i < nown;
+#pragma unroll
+    for (int j = 0; j < NZ; ++j) av[k][j] = in ? vb[(int64_t)j * a.Rp + i] : X(0);
+#pragma unroll
+    for (int j = 0; j < NZ2; ++j) ai[k][j] = in ? ib[(int64_t)j * a.Rp + i] * (uint32_t)sizeof(X) : 0u;   // byte offsets
+  }
+  // the seed r̂ = S res, the last direction and Â times it
+  auto seed = [&](int32_t q) {
+    const int32_t d = a.dofp ? a.dofp[q] : q;
+    return d >= 0 ? (X)(a.sc[d] * a.res[d]) : X(0);
+  };
+  X p[RT], sv[RT], x[RT], w[RT];
+  int il[RT];                                // this thread's rows in rl
+#pragma unroll
+  for (int k = 0; k < RT; ++k) {
+    const int i = t + k * kResT;
+    const bool in = i < nown;
+    il[k] = in ? i : zero;
+    p[k] = sv[k] = x[k] = X(0);
+    if (in) {
+      const int32_t row = a.orow[o0 + i];
+      rl[i] = seed(row);
+      if (keep0) {
+        p[k] = a.p[row];
+        sv[k] = a.sv[row];
+      }
+    }
+  }
+  for (int h = t; h < nh; h += kResT) {
+    const int32_t q = a.hrow[h0 + h];
+    hl[h] = a.hslot[h0 + h];
+    sl[h] = keep0 ? a.sv[q] : X(0);
+    rl[nown + h] = seed(q);
+  }
+  for (int i = t; i < a.nl; i += kResT) {
+    const int row = RRES * kResT + i;
+    const bool in = row < nown;
+    for (int j = 0; j < NZ; ++j) lv[i * NZ + j] = in ? vb[(int64_t)j * a.Rp + row] : X(0);
+    for (int j = 0; j < NZ2; ++j) lq[i * QS + j] = in ? ib[(int64_t)j * a.Rp + row] * (uint32_t)sizeof(X) : 0u;
+  }
+  res_barrier();
+
+  uint32_t ep = a.epoch;
+  const __amdgpu_buffer_rsrc_t rw = buf_rsrc(a.wx, (uint32_t)(2 * sizeof(typename LL<X>::W)) * (uint32_t)a.nslots);
+  const __amdgpu_buffer_rsrc_t rr = buf_rsrc(a.rec, (uint32_t)(2 * kResCopies * 2 * 16) * kResMaxBlocks);
+  // Publishes w of the rows other parts read: the first npub of the part, whose slots are
+  // consecutive; the resource ends there, so the stores of the other rows are dropped.
+  auto publish = [&]() {
+    typedef typename LL<X>::W W;
+    const __amdgpu_buffer_rsrc_t ro =
+        buf_rsrc(reinterpret_cast<const W*>(a.wx) + ((size_t)(ep & 1u) * a.nslots + p0), (uint32_t)(sizeof(W) * npub));
+#pragma unroll
+    for (int k = 0; k < RT; ++k)
+      if (k * kResT < npub) ll_put(ro, (uint32_t)(t + k * kResT), w[k], ep);
+  };
+  double rzp = 0.0, alpha = 0.0, irz = 0.0, ira = 0.0;   // γ and α of the last step; 1 / γ, 1 / (γ α)
+  // Sums g0, g1 over all blocks; with `halo`, reads the coupled rows' w into wl.  Every thread
+  // returns the same sums; false when a wait was given up.
+  auto exchange = [&](double& g0, double& g1, bool halo) {
+    const int par = (int)(ep & 1u);
+    const double v0 = wave_sum63(g0), v1 = wave_sum63(g1);
+    if (lane == 63) {
+      red[par][0][wave] = v0;
+      red[par][1][wave] = v1;
+    }
+    res_barrier();
+    if (a.nb == 1) {
+      irz = 1.0 / rzp;
+      ira = 1.0 / (rzp * alpha);
+      g0 = g1 = 0.0;
+#pragma unroll
+      for (int i = 0; i < kResWaves; ++i) {
+        g0 += red[par][0][i];
+        g1 += red[par][1][i];
+      }
+      ++ep;
+      return true;
+    }
+    // the block's record: its two sums, one copy per group of readers (blocks ≡ b mod 8), so
+    // that the reads of all blocks spread over the memory channels
+    const uint32_t rec = (uint32_t)(par * kResCopies * 2 * kResMaxBlocks);
+    if (t < 2 * kResCopies) {
+      double sum = 0.0;
+#pragma unroll
+      for (int i = 0; i < kResWaves; ++i) sum += red[par][t & 1][i];
+      ll_put(rr, rec + (uint32_t)(t * kResMaxBlocks + b), sum, ep);
+    }
+    const uint32_t rin = rec + (uint32_t)((b % kResCopies) * 2 * kResMaxBlocks + t);
+    if (halo) {   // reciprocals of the last step's scalars, while the values travel
+      irz = 1.0 / rzp;
+      ira = 1.0 / (rzp * alpha);
+    }
+    const bool reader = t < a.nb;      // thread t reads block t's record
+    bool lost = false, need = reader;
+    U4 q0 = {}, q1 = {};
+    if (halo) {                        // the coupled rows' w, and the records along with them
+      const uint32_t wi = (ep & 1u) * (uint32_t)a.nslots;
+      for (int base = 0; base < nh; base += H * kResT) {
+        typename LL<X>::W hv[H];
+        uint32_t at[H];
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+          at[k] = wi + (uint32_t)hl[min(base + k * kResT + t, nh - 1)];   // (spare threads repeat the last row)
+        }
+        for (uint32_t spin = 0;; ++spin) {
+          asm volatile("" ::: "memory");
+          bool ok = true;
+          if (need) {
+            q0 = LL<double>::get(rr, rin);
+            q1 = LL<double>::get(rr, rin + kResMaxBlocks);
+          }
+#pragma unroll
+          for (int k = 0; k < H; ++k)
+            if (base + k * kResT < nh) hv[k] = LL<X>::get(rw, at[k]);
+#pragma unroll
+          for (int k = 0; k < H; ++k)
+            if (base + k * kResT < nh) ok = ok && LL<X>::ok(hv[k], ep);
+          if (need) need = !(LL<double>::ok(q0, ep) && LL<double>::ok(q1, ep));
+          if (ok) break;
+          if (spin >= kSpinLimit) { lost = true; break; }
+        }
+#pragma unroll
+        for (int k = 0; k < H; ++k)
+          if (base + k * kResT + t < nh) wl[base + k * kResT + t] = LL<X>::val(hv[k]);
+      }
+    }
+    if (wave < (kResMaxBlocks + 63) / 64) {
+      for (uint32_t spin = 0; need; ++spin) {
+        asm volatile("" ::: "memory");
+        q0 = LL<double>::get(rr, rin);
+        q1 = LL<double>::get(rr, rin + kResMaxBlocks);
+        need = !(LL<double>::ok(q0, ep) && LL<double>::ok(q1, ep));
+        if (spin >= kSpinLimit) { lost = true; break; }
+      }
+      const double s0 = wave_sum63(reader ? LL<double>::val(q0) : 0.0);
+      const double s1 = wave_sum63(reader ? LL<double>::val(q1) : 0.0);
+      if (lane == 63) {
+        tot[par][0][wave] = s0;
+        tot[par][1][wave] = s1;
+      }
+    }
+    if (lost) gaveup = 1;
+    res_barrier();
+    g0 = (tot[par][0][0] + tot[par][0][1]) + (tot[par][0][2] + tot[par][0][3]);
+    g1 = (tot[par][1][0] + tot[par][1][1]) + (tot[par][1][2] + tot[par][1][3]);
+    ++ep;
+    return gaveup == 0;
+  };
+
+  double rz = 0.0, rz0 = 0.0, gstop = 0.0, beta = 0.0, gam = 0.0, pq = 0.0;
+  long long ticks = 0;
+  int done = 0, restart = 0, prods = 0, it = 0;
+  bool first = true, ok = true;
+  for (;;) {
+    // w = Â r̂ on the block's rows; γ = r̂·r̂ and δ = r̂·w (in a reseed r̂·p instead)
+    const long long c0 = a.time ? wall_clock64() : 0;
+#pragma unroll
+    for (int k = 0; k < RT; ++k) {
+      w[k] = X(0);
+      if (k * kResT < nown) {
+        X acc = X(0);
+        if constexpr (RRES > 0)
+          if (k < RRES) {
+            const int kk = k < RRES ? k : 0;
+#pragma unroll
+            for (int m = 0; m < NZ2; ++m) {
+              asm volatile("" : "+v"(ai[kk][m]));   // keeps packed positions, not LDS addresses, in registers
+              const uint32_t q = ai[kk][m];
+              acc += av[kk][2 * m] * at_lds(rl, q & 0xffffu);
+              if (2 * m + 1 < NZ) acc += av[kk][2 * m + 1 < NZ ? 2 * m + 1 : 0] * at_lds(rl, q >> 16);
+            }
+          }
+        if (k >= RRES) {
+          const int rest = t + (k - RRES) * kResT;
+          if (rest < a.nl) {
+#pragma unroll
+            for (int m = 0; m < NZ2; ++m) {
+              const uint32_t q = lq[rest * QS + m];
+              acc += lv[rest * NZ + 2 * m] * at_lds(rl, q & 0xffffu);
+              if (2 * m + 1 < NZ) acc += lv[rest * NZ + 2 * m + 1] * at_lds(rl, q >> 16);
+            }
+          }
+        }
+        w[k] = acc;      // 0 on unused rows: their entries are 0
+      }
+    }
+    if (a.nb > 1) publish();
+    double g0 = 0.0, g1 = 0.0;
+#pragma unroll
+    for (int k = 0; k < RT; ++k)
+      if (k * kResT < nown) {
+        const X r = rl[il[k]];
+        g0 += (double)r * (double)r;
+        g1 += (double)r * (double)(first ? p[k] : w[k]);
+      }
+    if (a.time) ticks += wall_clock64() - c0;
+    ++prods;
+    ok = exchange(g0, g1, true);
+    if (!ok) break;
+    if (first) {
+      // reseed: p made orthogonal to the new residual and extended, α = γ / p·ŝ
+      const bool keep = keep0 && g0 > 0.0;
+      gam = g0 > 0.0 ? g1 / g0 : 0.0;
+      rz = rz0 = g0;
+      const double conv = rr0 > 0.0 ? a.tol2 / rr0 : 0.0;
+      gstop = g0 * (a.hold2 > conv ? a.hold2 : conv);
+      const X be = (X)(keep ? g0 / rzp0 : 0.0), ga = (X)gam;
+      double none = 0.0;
+      pq = 0.0;
+#pragma unroll
+      for (int k = 0; k < RT; ++k) {
+        const X r = rl[il[k]];
+        p[k] = keep ? r + be * (p[k] - ga * r) : r;
+        sv[k] = keep ? w[k] + be * (sv[k] - ga * w[k]) : w[k];
+        pq += (double)p[k] * (double)sv[k];
+      }
+      for (int h = t; h < nh; h += kResT) sl[h] = keep ? wl[h] + be * (sl[h] - ga * wl[h]) : wl[h];
+      ok = exchange(pq, none, false);
+      if (!ok) break;
+      alpha = pq > 0.0 ? rz / pq : 0.0;
+      if (!(pq > 0.0)) {          // p vanished (r̂ already zero): nothing to step
+        done = restart = 1;
+        break;
+      }
+      rzp = rz;                   // the first step moves x̂ and r̂ along the reseed's p, ŝ
+    } else {
+      const double be = g0 * irz;
+      const double den = g1 - g0 * g0 * ira;
+      const bool stop = g0 <= gstop;
+      const bool brk = !(rzp > 0.0) || !(alpha != 0.0) || !(den > 0.0);
+      rz = g0;
+      if (stop || brk) {          // hand over: x̂, p and ŝ of the last step
+        done = 1;
+        restart = stop ? 0 : 1;
+        break;
+      }
+      if (it >= a.lim) break;
+      alpha = g0 / den;
+      beta = be;
+      rzp = g0;
+    }
+    ++it;
+    const X al = (X)alpha, be = (X)beta;
+#pragma unroll
+    for (int k = 0; k < RT; ++k)
+      if (k * kResT < nown) {
+        const X r = rl[il[k]];
+        if (!first) {
+          p[k] = r + be * p[k];
+          sv[k] = w[k] + be * sv[k];
+        }
+        x[k] += al * p[k];
+        rl[il[k]] = r - al * sv[k];
+      }
+    for (int base = t; base < nh; base += 4 * kResT) {   // four rows' LDS reads in flight
+      X sn[4], rn[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int h = base + k * kResT;
+        if (h < nh) {
+          sn[k] = first ? sl[h] : wl[h] + be * sl[h];
+          rn[k] = rl[nown + h];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int h = base + k * kResT;
+        if (h < nh) {
+          sl[h] = sn[k];
+          rl[nown + h] = rn[k] - al * sn[k];
+        }
+      }
+    }
+    first = false;
+    res_barrier();
+  }
+  // the arguments read again: kept in scalar registers across the loop they would crowd it
+  const ResArgs<X>& z = *reinterpret_cast<const ResArgs<X>*>(res_kernargs());
+  if (!ok) {
+    if (t == 0) z.s->pad = 1;
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < RT; ++k) {
+    const int i = t + k * kResT;
+    if (i < nown) {
+      const int32_t row = z.orow[o0 + i];
+      z.p[row] = p[k];
+      z.sv[row] = sv[k];
+      const int32_t d = z.dofp ? z.dofp[row] : row;
+      if (d >= 0) z.u[d] += z.sc[d] * (double)x[k];
+    }
+  }
+  if (b == 0 && t == 0) {
+    Scal* o = z.s;                // all but pad, which a block that gave up sets
+    o->rz = rz;
+    o->rz0 = rz0;
+    o->rzp = rzp;
+    o->gstop = gstop;
+    o->alpha = alpha;
+    o->beta = beta;
+    o->gam = gam;
+    o->pq = pq;
+    o->done = done;
+    o->restart = restart;
+    o->fresh = 0;
+    o->pend = 0.0;
+    o->iters += it;
+    o->prods += prods;
+    o->prod_ticks += ticks;
+  }
+}
+
+// ---- host ---------------------------------------------------------------------------------
+// Most rows per block of the instantiated kernels (FP64 with 27 entries: what LDS holds besides).
+static int res_most_rows(int nz, bool fp32) {
+  return fp32 ? (nz == 9 ? 4096 : nz == 18 ? 2560 : 2048) : (nz == 9 ? 2048 : nz == 18 ? 1536 : 1400);
+}
+
+// The instantiated kernel for nz entries per row and R rows per block (null: too many).
+// Resident rows are what the 256 VGPRs of a thread hold beside the vectors (512 threads, two
+// waves per SIMD); the entries of further rows are in LDS.
+template <typename X>
+static const void* res_kernel(int nz, int R) {
+  const int need = (R + kResT - 1) / kResT;
+#define FEM_RES(NZ, RRES, RT) \
+  if (nz == NZ && need <= RT) return (const void*)k_resident<X, NZ, RRES, RT>
+  if constexpr (sizeof(X) == 4) {
+    FEM_RES(9, 8, 8);
+    FEM_RES(18, 5, 5);
+    FEM_RES(27, 3, 4);
+  } else {
+    FEM_RES(9, 4, 4);
+    FEM_RES(18, 3, 3);
+    FEM_RES(27, 2, 3);
+  }
+#undef FEM_RES
+  return nullptr;
+}
+
+// LDS of a block with nl rows' entries in it: r̂ (and a zero slot), ŝ, w and the slots of the
+// coupled rows, the entries
+static size_t res_lds_bytes(const ResOp* o, size_t xb, int nl) {
+  const size_t nz2 = (size_t)((o->nz + 1) / 2 | 1);
+  return ((size_t)o->nlocmax + 1 + 2 * (size_t)o->nhmax + (size_t)o->nz * nl) * xb + 4 * (nz2 * nl + (size_t)o->nhmax);
+}
+
+// Register rows of the instantiated kernels (kResT threads).
+static int res_register_rows(int nz, bool fp32) {
+  return kResT * (fp32 ? (nz == 9 ? 8 : nz == 18 ? 5 : 3) : (nz == 9 ? 4 : nz == 18 ? 3 : 2));
+}
+
+// Parts along each axis for nx × ny × nz positions of `per` rows each and at most `most` parts.
+// An iteration's cost in cycles, fitted to timed stretches (2D and 3D, 18 to 256 parts): every
+// kResT rows of the largest part begun (more where their entries are in LDS), its coupled rows,
+// and every part's record read by all; parts too large for FP64 values only where nothing else
+// is left.
+static void res_triple(const double* ext, int dim, double per, int nz, int most, int* out) {
+  double best = 1e300;
+  const double regs = kResT * (nz == 9 ? 4 : nz == 18 ? 3 : 2), cap = nz == 27 ? regs + 360.0 : regs;
+  for (int x = 1; x <= most; ++x)
+    for (int y = 1; x * y <= most; ++y) {
+      if (dim < 2 && y > 1) break;
+      for (int z = 1; x * y * z <= most; ++z) {
+        if (dim < 3 && z > 1) break;
+        const double bx = std::ceil(ext[0] / x - 1e-9), by = std::ceil(ext[1] / y - 1e-9),
+                     bz = std::ceil(ext[2] / z - 1e-9);
+        if (bx < 1 || by < 1 || bz < 1) continue;
+        const double own = bx * by * bz;
+        const double all = (x > 1 ? bx + 2 : bx) * (y > 1 ? by + 2 : by) * (z > 1 ? bz + 2 : bz);
+        const double rounds = std::ceil(per * own / kResT);
+        const double cost = rounds * (250.0 + 30.0 * nz) + (per * own > regs ? 1500.0 : 0.0) +
+                            0.5 * per * (all - own) + 0.1 * per * own + 8.0 * x * y * z +
+                            1e4 * std::max(0.0, per * own - cap);
+        if (cost < best) {
+          best = cost;
+          out[0] = x;
+          out[1] = y;
+          out[2] = z;
+        }
+      }
+    }
+}
+
+static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& rows, int nz, int most_rows) {
+  int ncu = 0, maxlds = 0, coop = 0;
+  (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device);
+  (void)hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device);
+  (void)hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device);
+  const int64_t n = rows.n;
+  o->state = -1;
+  o->n = n;
+  o->nz = nz;
+  const int words = (int)((n + 31) / 32), ng = (words + 7) / 8;
+  const int lds = 4 * (words + ng);
+  if (lds > maxlds - 1024) return FEM_OK;   // a bitmap of the rows (more than a million): far too many anyway
+
+  struct Scratch {                          // freed on every way out
+    int32_t *node = nullptr, *part = nullptr, *hist = nullptr, *size = nullptr, *rank = nullptr, *cnt = nullptr;
+    uint8_t* flag = nullptr;
+    double* geom = nullptr;
+    ~Scratch() {
+      dev_free(&node); dev_free(&part); dev_free(&hist); dev_free(&size); dev_free(&rank); dev_free(&cnt);
+      dev_free(&flag); dev_free(&geom);
+    }
+  } w;
+  int rc;
+  ResPos g{};
+  g.src = s.src;
+  g.n = n;
+  g.px = s.px;
+  g.pxy = s.pxy;
+  g.dofp = s.dofp;
+  g.dim = s.src ? s.dim : c->sdim;
+  if (s.src == 0) {   // a node of each dof's first cell (its own node for a Q1 field)
+    const int64_t nc = c->ncells, nd = c->ndpc, npc = c->npc;
+    if (nd <= 0 || npc <= 0 || (int64_t)c->h_cell_dofs.size() != nc * nd || (int64_t)c->h_cell_nodes.size() != nc * npc)
+      return FEM_OK;
+    std::vector<int32_t> node(n, 0), at(nd);
+    std::vector<uint8_t> seen(n, 0);
+    for (int64_t a = 0; a < nd; ++a) at[a] = (int32_t)(a * npc / nd);
+    for (int64_t e = 0; e < nc; ++e)
+      for (int64_t a = 0; a < nd; ++a) {
+        const int32_t d = c->h_cell_dofs[e * nd + a];
+        if (!seen[d]) {
+          seen[d] = 1;
+          node[d] = c->h_cell_nodes[e * npc + at[a]];
+        }
+      }
+    if ((rc = dev_alloc(c, &w.node, n))) return rc;
+    FEM_HIP(c, hipMemcpy(w.node, node.data(), 4 * n, hipMemcpyHostToDevice));
+    g.node = w.node;
+    for (int d = 0; d < 3; ++d) g.x[d] = c->d_x[d];
+  }
+  double geom[10];
+  if ((rc = dev_alloc(c, &w.geom, 10))) return rc;
+  k_res_geom<<<1, 1024, 0, c->stream>>>(g, rows, nz, w.geom);
+  FEM_HIP(c, hipGetLastError());
+  FEM_HIP(c, hipMemcpyAsync(geom, w.geom, sizeof geom, hipMemcpyDeviceToHost, c->stream));
+  FEM_HIP(c, hipStreamSynchronize(c->stream));
+  const double count = geom[9];
+  double ext[3] = {1.0, 1.0, 1.0}, cells = 1.0;
+  for (int d = 0; d < 3; ++d) {
+    const double len = geom[3 + d] - geom[d];
+    const bool flat = d >= g.dim || !(len > 0.0);
+    g.lo[d] = geom[d];
+    g.inv[d] = flat ? 0.0 : (kResBins - 0.5) / len;
+    if (!flat && geom[6 + d] > 0.0) ext[d] = std::max(1.0, std::floor(len / geom[6 + d] + 1.5));
+    cells *= ext[d];
+  }
+  const int most = (int)std::max<double>(
+      1.0, std::min<double>(std::min(ncu, kResMaxBlocks), std::ceil(count / kResRows)));
+  if ((most > 1 && !coop) || count > (double)most * most_rows) return FEM_OK;
+  int cut[3] = {1, 1, 1};
+  res_triple(ext, g.dim, count / cells, nz, most, cut);
+  const int nb = cut[0] * cut[1] * cut[2];
+  o->nb = nb;
+  const int grid = (int)std::min<int64_t>(2048, (n + 255) / 256);
+  if ((rc = dev_alloc(c, &w.part, n)) || (rc = dev_alloc(c, &w.hist, (size_t)kResBins * nb)) ||
+      (rc = dev_alloc(c, &w.flag, n)) || (rc = dev_alloc(c, &w.size, 2 * nb)) || (rc = dev_alloc(c, &w.rank, n)) ||
+      (rc = dev_alloc(c, &w.cnt, nb)) || (rc = dev_alloc(c, &o->oofs, nb + 1)) ||
+      (rc = dev_alloc(c, &o->pofs, nb + 1)) || (rc = dev_alloc(c, &o->hoff, nb + 1)))
+    return rc;
+  FEM_HIP(c, hipMemsetAsync(w.part, 0, 4 * n, c->stream));
+  FEM_HIP(c, hipMemsetAsync(w.flag, 0, n, c->stream));
+  FEM_HIP(c, hipMemsetAsync(w.size, 0, 8 * nb, c->stream));
+  int slabs = 1;
+  for (int d = 0; d < 3; ++d) {
+    if (cut[d] == 1 && !(d == 2)) continue;   // the last level also marks the rows without a place
+    FEM_HIP(c, hipMemsetAsync(w.hist, 0, (size_t)4 * kResBins * slabs, c->stream));
+    k_res_hist<<<grid, 256, 0, c->stream>>>(g, d, w.part, w.hist);
+    k_res_cut<<<slabs, 256, 0, c->stream>>>(cut[d], w.hist);
+    k_res_split<<<grid, 256, 0, c->stream>>>(g, d, cut[d], w.hist, w.part);
+    slabs *= cut[d];
+  }
+  k_res_shared<<<grid, 256, 0, c->stream>>>(rows, nz, w.part, w.flag, w.size);
+  FEM_HIP(c, hipGetLastError());
+  std::vector<int32_t> h(nb), off(nb + 1, 0);
+  FEM_HIP(c, hipMemcpyAsync(h.data(), w.size, 4 * nb, hipMemcpyDeviceToHost, c->stream));
+  FEM_HIP(c, hipStreamSynchronize(c->stream));
+  o->Rmax = 0;
+  for (int b = 0; b < nb; ++b) {
+    off[b + 1] = off[b] + h[b];
+    o->Rmax = std::max(o->Rmax, h[b]);
+  }
+  if (o->Rmax > 8192) return FEM_OK;
+  int pow2 = 2;
+  while (pow2 < o->Rmax) pow2 *= 2;
+  o->Rp = (o->Rmax + 63) / 64 * 64;
+  FEM_HIP(c, hipMemcpyAsync(o->oofs, off.data(), 4 * (nb + 1), hipMemcpyHostToDevice, c->stream));
+  if ((rc = dev_alloc(c, &o->orow, off[nb]))) return rc;
+  k_res_gather<<<grid, 256, 0, c->stream>>>(n, w.part, w.flag, o->oofs, w.size + nb, o->orow);
+  k_res_sort<<<nb, 1024, 4 * pow2, c->stream>>>(pow2, o->oofs, o->orow, w.rank, w.cnt);
+  FEM_HIP(c, hipGetLastError());
+  std::vector<int32_t> pub(nb + 1, 0), hof(nb + 1, 0);
+  FEM_HIP(c, hipMemcpyAsync(h.data(), w.cnt, 4 * nb, hipMemcpyDeviceToHost, c->stream));
+  FEM_HIP(c, hipStreamSynchronize(c->stream));
+  for (int b = 0; b < nb; ++b) pub[b + 1] = pub[b] + h[b];
+  o->nslots = pub[nb];
+  (void)hipFuncSetAttribute((const void*)k_res_count, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * words);
+  (void)hipFuncSetAttribute((const void*)k_res_fill, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  k_res_count<<<nb, 256, 4 * words, c->stream>>>(rows, nz, w.part, o->oofs, o->orow, w.cnt);
+  FEM_HIP(c, hipGetLastError());
+  FEM_HIP(c, hipMemcpyAsync(h.data(), w.cnt, 4 * nb, hipMemcpyDeviceToHost, c->stream));
+  FEM_HIP(c, hipStreamSynchronize(c->stream));
+  o->nlocmax = o->nhmax = 0;
+  for (int b = 0; b < nb; ++b) {
+    hof[b + 1] = hof[b] + h[b];
+    o->nhmax = std::max(o->nhmax, h[b]);
+    o->nlocmax = std::max(o->nlocmax, off[b + 1] - off[b] + h[b]);
+  }
+  o->nlocmax += o->nlocmax & 1;             // keeps what follows r̂ and its zero slot apart
+  if (o->nlocmax > 65535) return FEM_OK;    // positions are 16 bits (and byte offsets: res_lds_rows)
+  const int nz2 = (nz + 1) / 2;
+  if ((rc = dev_alloc(c, &o->hrow, hof[nb])) || (rc = dev_alloc(c, &o->hslot, hof[nb])) ||
+      (rc = dev_alloc(c, &o->ai, (size_t)nb * nz2 * o->Rp)) || (rc = dev_alloc(c, &o->wx, (size_t)8 * o->nslots)) ||
+      (rc = dev_alloc(c, &o->rec, kRecWords)))
+    return rc;
+  FEM_HIP(c, hipMemcpyAsync(o->pofs, pub.data(), 4 * (nb + 1), hipMemcpyHostToDevice, c->stream));
+  FEM_HIP(c, hipMemcpyAsync(o->hoff, hof.data(), 4 * (nb + 1), hipMemcpyHostToDevice, c->stream));
+  FEM_HIP(c, hipMemsetAsync(o->wx, 0, (size_t)32 * o->nslots, c->stream));
+  FEM_HIP(c, hipMemsetAsync(o->rec, 0, 4 * kRecWords, c->stream));
+  k_res_fill<<<nb, 256, lds, c->stream>>>(rows, nz, o->Rp, w.part, w.rank, o->oofs, o->orow, o->pofs, o->hoff, o->hrow,
+                                          o->hslot, o->ai);
+  FEM_HIP(c, hipGetLastError());
+  FEM_HIP(c, hipStreamSynchronize(c->stream));   // host vectors and scratch go
+  o->epoch = 0;
+  o->state = 1;
+  return FEM_OK;
+}
+
+// Rows whose entries LDS holds: those beyond the register rows; −1 when they do not fit.
+static int res_lds_rows(const ResOp* o, bool fp32, int maxlds) {
+  const size_t xb = fp32 ? 4 : 8, base = res_lds_bytes(o, xb, 0), per = o->nz * xb + 4 * ((o->nz + 1) / 2 | 1);
+  const size_t cap = (size_t)maxlds - 1024;
+  if (base > cap || (o->nlocmax + 1) * xb > 65536) return -1;   // 16-bit byte offsets into r̂
+  const int rest = std::max(0, o->Rmax - res_register_rows(o->nz, fp32));
+  return base + rest * per > cap ? -1 : rest;
+}
+
+int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok) {
+  *ok = false;
+  if (!*op) *op = new ResOp();
+  ResOp* o = *op;
+  if (o->state == -1) return FEM_OK;
+  ResRows rows{s.src, s.dim, s.n, s.npad, s.px, s.pxy, c->d_colptr, c->d_rowval, s.dofp, c->d_nzval, sc, s.kc, s.val,
+               s.t, {}};
+  for (int i = 0; i < 8; ++i) rows.f[i] = s.f[i];
+  int rc;
+  if (o->state == 0) {
+    const int widest = s.src == 0 ? c->max_row_nnz : s.dim == 3 ? 27 : 9;
+    const int nz = widest <= 9 ? 9 : widest <= 18 ? 18 : 27, most = res_most_rows(nz, fp32);
+    // clearly too large in this precision (lattice rows include some padding): nothing is built
+    if (widest > 27 || s.n < 1 || s.n > (int64_t)kResMaxBlocks * most * 5 / 4) return FEM_OK;
+    o->state = -1;
+    if ((rc = res_build(c, o, s, rows, nz, res_most_rows(nz, true)))) return rc;
+    if (o->state == -1) return FEM_OK;
+  }
+  int maxlds = 0;
+  (void)hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device);
+  if (!(fp32 ? res_kernel<float>(o->nz, o->Rmax) : res_kernel<double>(o->nz, o->Rmax)) ||
+      res_lds_rows(o, fp32, maxlds) < 0)
+    return FEM_OK;
+  const int pi = fp32 ? 0 : 1;
+  const size_t len = (size_t)o->nb * o->nz * o->Rp;
+  if (fp32 && !o->val32 && (rc = dev_alloc(c, &o->val32, len))) return rc;
+  if (!fp32 && !o->val64 && (rc = dev_alloc(c, &o->val64, len))) return rc;
+  if (o->ver[pi] != c->nzval_version + 1 || o->aux[pi] != c->aux_version + 1 || o->jac[pi] != jacobi ||
+      o->vsrc[pi] != s.src) {
+    const int g = (int)std::min<int64_t>(8192, ((int64_t)o->nb * o->Rp + 255) / 256);
+    if (fp32) k_res_vals<float><<<g, 256, 0, c->stream>>>(rows, o->nz, o->Rp, o->nb, o->oofs, o->orow, o->val32);
+    else k_res_vals<double><<<g, 256, 0, c->stream>>>(rows, o->nz, o->Rp, o->nb, o->oofs, o->orow, o->val64);
+    FEM_HIP(c, hipGetLastError());
+    o->ver[pi] = c->nzval_version + 1;
+    o->aux[pi] = c->aux_version + 1;
+    o->jac[pi] = jacobi;
+    o->vsrc[pi] = s.src;
+  }
+  *ok = true;
+  return FEM_OK;
+}
+
+template <typename X>
+int resident_run(fem_ctx* c, ResOp* o, const double* res, const double* sc, X* p, X* sv, double* u, Scal* s,
+                 const int32_t* dofp, double hold_factor2, double tol2, int restart, int lim, bool* launched) {
+  *launched = false;
+  // exchange numbers: one per product and one more per reseed; started over long before 2³²
+  const uint32_t need = (uint32_t)lim + 8u;
+  if (o->epoch > 0xf0000000u - need) {
+    FEM_HIP(c, hipMemsetAsync(o->wx, 0, (size_t)32 * o->nslots, c->stream));
+    FEM_HIP(c, hipMemsetAsync(o->rec, 0, 4 * kRecWords, c->stream));
+    o->epoch = 0;
+  }
+  int maxlds = 0;
+  FEM_HIP(c, hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
+  const int nl = res_lds_rows(o, sizeof(X) == 4, maxlds);
+  ResArgs<X> a{o->Rp, o->nb, o->nslots, nl, o->nlocmax + 1, o->nhmax, o->oofs, o->orow, o->pofs, o->hoff, o->hrow,
+               o->hslot, o->ai,
+               sizeof(X) == 4 ? reinterpret_cast<const X*>(o->val32) : reinterpret_cast<const X*>(o->val64),
+               dofp, res, sc, p, sv, u, s, o->wx, o->rec, hold_factor2, tol2, o->epoch + 1u, restart, lim,
+               c->tune.time_kernels};
+  o->epoch += need;
+  const void* k = res_kernel<X>(o->nz, o->Rmax);
+  const size_t lds = res_lds_bytes(o, sizeof(X), nl);
+  FEM_HIP(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  void* args[] = {&a};
+  const hipError_t e = o->nb == 1 ? hipLaunchKernel(k, dim3(1), dim3(kResT), args, lds, c->stream)
+                                  : hipLaunchCooperativeKernel(k, dim3(o->nb), dim3(kResT), args, (unsigned)lds,
+                                                               c->stream);
+  *launched = e == hipSuccess;
+  if (e != hipSuccess) (void)hipGetLastError();   // not as many blocks at once as the device should hold
+  return FEM_OK;
+}
+
+template int resident_run<float>(fem_ctx*, ResOp*, const double*, const double*, float*, float*, double*, Scal*,
+                                 const int32_t*, double, double, int, int, bool*);
+template int resident_run<double>(fem_ctx*, ResOp*, const double*, const double*, double*, double*, double*, Scal*,
+                                  const int32_t*, double, double, int, int, bool*);
+
+}  // namespace fem

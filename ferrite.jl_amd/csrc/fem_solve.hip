@@ -27,7 +27,9 @@
 //
 // Reductions are fence-free and fixed-order: blocks write partials that the next kernel
 // sums (by default one block, k_cg_scal), in the same order every time, so results are
-// bitwise reproducible and the host never sits in the iteration.  A batch of iterations is
+// bitwise reproducible and the host never sits in the iteration.  Systems whose rows fit the
+// chip's registers and LDS run the whole recurrence in one launch per hand-over instead
+// (fem_resident.hip).  Otherwise a batch of iterations is
 // captured once into a hipGraph and replayed; kernels launched past a hand-over return at
 // once on the device flag.
 #include <cmath>
@@ -35,6 +37,7 @@
 
 #include "fem_internal.h"
 #include "fem_cell.h"
+#include "fem_resident.h"
 
 namespace fem {
 
@@ -165,6 +168,9 @@ struct SolverWork {
   bool use_elem = false;       // the current solve runs on the stored element matrices
   ElemOp* eop = nullptr;       // their per-solve vectors (fem_elemop.hip)
   int elem_grid = 0;
+  ResOp *res_csc = nullptr, *res_lat = nullptr;   // resident CG on K's rows, on the lattice's rows
+  ResOp* res_op = nullptr;     // the one the current solve runs on, or null
+  bool res_off = false;        // a resident launch was not taken or gave up: not tried again
   int64_t cap32 = 0, cap64 = 0;   // length of the recurrence vectors
   int sell_grid = 0;           // blocks of the SELL SpMV (fixed: its partial count)
   SpmvShape sh64;              // CSR-stream FP64 residual
@@ -206,6 +212,8 @@ void free_solver(fem_ctx* c) {
   dev_free(&l.map); dev_free(&l.dofp); dev_free(&l.val32); dev_free(&l.val64); dev_free(&l.cnt);
   dev_free(&l.mir32); dev_free(&l.mir64);
   elem_op_free(&w->eop);
+  resident_free(&w->res_csc);
+  resident_free(&w->res_lat);
   CellOp& cl = w->cells;
   dev_free(&cl.corg); dev_free(&cl.kc64); dev_free(&cl.kc32); dev_free(&cl.t64); dev_free(&cl.t32);
   dev_free(&cl.cnt); dev_free(&cl.up64); dev_free(&cl.yp64); dev_free(&cl.tm64); dev_free(&cl.s0);
@@ -2268,17 +2276,28 @@ static int spmv_hat(fem_ctx* c, SolverWork* w, const X* x, X* y, const Scal* sc)
   return g;
 }
 
-// The scaling S and the scaled operator in X precision, ready for spmv_hat: the lattice
-// planes when the dofs form a lattice and K is symmetric (the mixed solver by default; the
-// FP64 solver with tuning lattice = 1), otherwise the sliced copy.  Returns the length of
-// the recurrence vectors in *nv.
+// Whether the tuning leaves the iteration's kernels at their defaults: an explicit launch shape
+// of the separate SpMV and vector kernels asks for those kernels.
+static bool resident_allowed(const fem_ctx* c, const SolverWork* w) {
+  const fem_tuning& t = c->tune;
+  return !w->res_off && t.cg_elems == 0 && t.sell_unroll == 0 && t.sell_map == 0 && t.sell_nt == 0 &&
+         t.sell_compress == 0 && t.lattice_blocks == 0 && t.cell_blocks == 0 && t.cell_rows == 0;
+}
+
+// The scaling S and the scaled operator in X precision: the lattice forms when the dofs form a
+// lattice and the form's check passes (the mixed solver by default; the FP64 solver with tuning
+// lattice = 1 / cell_operator = 1), the stored element matrices, otherwise K's own rows.  With
+// `resident`, the resident CG is prepared on that form where it fits (w->res_op); otherwise the
+// form (for K's rows the sliced copy) is ready for spmv_hat.  Returns the length of the
+// recurrence vectors in *nv.
 template <typename X>
-static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv) {
+static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv, bool resident = false) {
   int rc;
   k_scale<<<kMaxVecBlocks, kBlock, 0, c->stream>>>(c->n, c->d_diag, c->d_nzval, jacobi, w->sc);
   w->use_lat = false;
   w->use_cells = false;
   w->use_elem = false;
+  w->res_op = nullptr;
   const bool want = sizeof(X) == 4 ? c->tune.lattice != -1 : c->tune.lattice == 1;
   const bool want_cells = sizeof(X) == 4 ? c->tune.cell_operator != -1 : c->tune.cell_operator == 1;
   if (want || want_cells) {
@@ -2305,6 +2324,31 @@ static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv) 
   }
   *nv = w->use_lat ? w->lat.npad : c->n;
   if ((rc = ensure_vecs<X>(c, w, *nv))) return rc;
+  if (resident && !w->use_elem && resident_allowed(c, w)) {
+    const LatOp& l = w->lat;
+    const CellOp& cl = w->cells;
+    ResSource s;
+    s.src = w->use_cells ? 2 : w->use_lat ? 1 : 0;
+    s.n = *nv;
+    if (w->use_lat) {
+      s.dim = l.ns == 14 ? 3 : 2;
+      s.px = (int32_t)l.px;
+      s.pxy = (int32_t)l.pxy;
+      s.npad = l.npad;
+      s.dofp = l.dofp;
+      s.val = sizeof(X) == 4 ? (const void*)l.val32 : (const void*)l.val64;
+      s.kc = cl.kc64;
+      s.t = sizeof(X) == 4 ? (const void*)cl.t32 : (const void*)cl.t64;
+      for (int i = 0; i < 8; ++i) s.f[i] = cl.f[i];
+    }
+    ResOp** op = w->use_lat ? &w->res_lat : &w->res_csc;
+    bool ok = false;
+    if ((rc = resident_prepare(c, op, s, w->sc, jacobi, sizeof(X) == 4, &ok))) return rc;
+    if (ok) {
+      w->res_op = *op;
+      return FEM_OK;
+    }
+  }
   if (w->use_lat || w->use_elem) return FEM_OK;
   if ((rc = ensure_sell(c, w))) return rc;
   return ensure_sell_vals<X>(c, w, jacobi);
@@ -2557,6 +2601,82 @@ static int cg_run(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double bnorm2, 
   return converged ? FEM_OK : FEM_ERR_NOCONV;
 }
 
+// The same with the resident CG: one launch per stretch (reseed, iterations, fold into u), then
+// the FP64 residual, and one read of the record by the host.  *gave_up: the device did not take a
+// launch, or one stopped waiting for its blocks (nothing of it was folded); the caller starts over
+// with the separate kernels.
+template <typename X>
+static int cg_run_resident(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double bnorm2, double tol2,
+                           double hold_factor2, int maxit, int* iters, int* handovers, double* ms, bool* gave_up) {
+  zero_vec<double>(c, c->d_u, c->n);
+  k_cg_init_scal<<<1, 1, 0, c->stream>>>(w->s, bnorm2);
+  const int64_t most = ((int64_t)maxit + kBatch - 1) / kBatch * kBatch;   // as the batches round it up
+  const int32_t* dofp = w->use_lat ? w->lat.dofp : nullptr;
+  const double* res = c->d_f;
+  int rc, nho = 0, stall = 0;
+  bool converged = false;
+  double prev_true = bnorm2;
+  Scal h{};
+  FEM_HIP(c, hipEventRecord(c->ev0, c->stream));
+  for (;;) {
+    const int lim = (int)std::min<int64_t>(1 << 24, most - h.iters);
+    bool launched = false;
+    if ((rc = resident_run<X>(c, w->res_op, res, w->sc, v.p, v.sv, c->d_u, w->s, dofp, hold_factor2, tol2,
+                              res == c->d_f ? 1 : 0, lim, &launched)))
+      return rc;
+    if (!launched) {
+      *gave_up = true;
+      return FEM_OK;
+    }
+    residual(c, w);
+    FEM_HIP(c, hipGetLastError());
+    if ((rc = read_scal(c, w, &h))) return rc;
+    if (h.pad) {
+      *gave_up = true;
+      return FEM_OK;
+    }
+    if (h.done) ++nho;
+    if (h.rr <= tol2) { converged = true; break; }
+    if (h.iters >= most) break;
+    stall = h.rr > 0.81 * prev_true ? stall + 1 : 0;
+    if (stall >= kMaxStall) break;
+    prev_true = std::min(prev_true, h.rr);
+    res = w->res;
+  }
+  FEM_HIP(c, hipEventRecord(c->ev1, c->stream));
+  *ms += event_ms(c);
+  if (c->tune.time_kernels) {   // 100 MHz clock
+    c->timings.spmv_ms += 1e-5 * (double)h.prod_ticks;
+    c->timings.spmv_launches += h.prods;
+  }
+  *iters = h.iters;
+  *handovers = nho;
+  return converged ? FEM_OK : FEM_ERR_NOCONV;
+}
+
+// The solve in X precision on whichever form prepare_operator chose.
+template <typename X>
+static int cg_solve(fem_ctx* c, SolverWork* w, int jacobi, double bnorm2, double tol2, double hold_factor2, int maxit,
+                    int* iters, int* handovers, double* ms) {
+  int64_t nv = 0;
+  int rc = prepare_operator<X>(c, w, jacobi, &nv, true);
+  if (rc) return rc;
+  auto vecs = [&]() {
+    const int32_t* map = w->use_lat ? w->lat.map : nullptr;
+    if constexpr (sizeof(X) == 4) return CgVecs<X>{w->x32, w->r32, w->wv32, w->p32, w->sv32, nv, map};
+    else return CgVecs<X>{w->x, w->r, w->wv, w->p, w->sv, nv, map};
+  };
+  if (w->res_op) {
+    bool gave_up = false;
+    rc = cg_run_resident<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, iters, handovers, ms, &gave_up);
+    if (!gave_up) return rc;
+    w->res_off = true;
+    if ((rc = prepare_operator<X>(c, w, jacobi, &nv))) return rc;
+  }
+  return cg_run<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, sizeof(X) == 4 ? w->g32 : w->g64, iters, handovers,
+                   ms);
+}
+
 }  // namespace fem
 
 using namespace fem;
@@ -2591,17 +2711,12 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
   }
   const double tol2 = cfg->rtol * cfg->rtol * bnorm2;
   int iters = 0, handovers = 0;
-  int64_t nv = 0;
   if (!mixed) {
-    if ((rc = prepare_operator<double>(c, w, cfg->precond, &nv))) return rc;
-    const CgVecs<double> v{w->x, w->r, w->wv, w->p, w->sv, nv, w->use_lat ? w->lat.map : nullptr};
-    rc = cg_run<double>(c, w, v, bnorm2, tol2, 0.0, maxit, w->g64, &iters, &handovers, &cg_ms);
+    rc = cg_solve<double>(c, w, cfg->precond, bnorm2, tol2, 0.0, maxit, &iters, &handovers, &cg_ms);
   } else {
     // the FP32 recurrence hands over whenever its residual has fallen by δ (inner_rtol)
-    if ((rc = prepare_operator<float>(c, w, cfg->precond, &nv))) return rc;
     const double delta = cfg->inner_rtol > 0 ? cfg->inner_rtol : 0.1;
-    const CgVecs<float> v{w->x32, w->r32, w->wv32, w->p32, w->sv32, nv, w->use_lat ? w->lat.map : nullptr};
-    rc = cg_run<float>(c, w, v, bnorm2, tol2, delta * delta, maxit, w->g32, &iters, &handovers, &cg_ms);
+    rc = cg_solve<float>(c, w, cfg->precond, bnorm2, tol2, delta * delta, maxit, &iters, &handovers, &cg_ms);
   }
   if (rc && rc != FEM_ERR_NOCONV) return rc;
   out.iterations = iters;

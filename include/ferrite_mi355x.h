@@ -205,9 +205,11 @@ typedef struct {
   int32_t asm_block;                 /* cells per workgroup of the element kernels (0 = default) */
   int32_t asm_mode;                  /* scalar Q1 Poisson assembly: 0 = owner-computes gather when
                                         supported (default), 1 = colored scatter, 2 = gather only */
-  int32_t time_kernels;              /* 1: the solver launches its CG kernels directly (no graph
-                                        replay) with HIP events around every SpMV
-                                        (fem_timings.spmv_ms / spmv_launches) */
+  int32_t time_kernels;              /* 1: the solver times its SpMVs (fem_timings.spmv_ms /
+                                        spmv_launches): separate kernels are launched directly (no
+                                        graph replay) with HIP events around every SpMV; where the
+                                        whole recurrence runs in one launch, its products are timed
+                                        on the device's clock and counted */
   int32_t sell_unroll;               /* sliced-ELL SpMV: entries loaded per lane before their x
                                         gathers, 4 / 8 / 16 (0 = default: 8 FP32, 4 FP64) */
   int32_t sell_map;                  /* solver SpMV rows to blocks: 1 = grid-stride, 2 = contiguous,
@@ -254,8 +256,8 @@ typedef struct {
   double assemble_kernel_ms;   /* element + scatter kernels, summed over colors */
   double fill_ms;              /* start_assemble zero fill */
   double apply_ms;             /* all apply! kernels */
-  double spmv_ms;              /* solver SpMV launches of the last solve, summed (with time_kernels) */
-  int32_t spmv_launches;       /* number of those launches (0 without time_kernels) */
+  double spmv_ms;              /* SpMVs of the last solve, summed (with time_kernels) */
+  int32_t spmv_launches;       /* their number (0 without time_kernels) */
   int32_t assemble_launches;
   double solve_ms;             /* the CG loop of the last solve (HIP events) */
   double element_ms;           /* two-phase (owner-computes) assembly: the element-matrix phase */

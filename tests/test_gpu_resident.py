@@ -1,0 +1,98 @@
+"""The resident CG (one launch per stretch between hand-overs) against the separate kernels.
+
+Sizes at the edges of its parts: one block (up to a few hundred rows), one row more than a
+block's 512 threads, several rows per thread, rows whose entries lie in LDS (FP64, 27 entries,
+more than 1,024 rows per block); every source of rows (K's columns, lattice planes, cell form),
+9, 18 and 27 entries per row.  An explicit launch shape of the separate kernels (cg_elems)
+selects those.  Both solve to a true residual of 1e-12, so their u differ by a few times
+cond · 1e-12: 1e-8, the bar the other solver tests use."""
+import numpy as np
+import pytest
+
+from conftest import gpu_available
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
+
+import ferrite_amd as fa  # noqa: E402
+
+
+def _move(g, nel, seed):
+    """Interior nodes moved by up to a fifth of the cell size."""
+    rng = np.random.default_rng(seed)
+    inner = np.all((g.nodes > g.nodes.min(0) + 1e-12) & (g.nodes < g.nodes.max(0) - 1e-12), axis=1)
+    h = (g.nodes.max(0) - g.nodes.min(0)) / np.array(nel)
+    g.nodes[inner] += rng.uniform(-0.2, 0.2, (int(inner.sum()), g.sdim)) * h
+    return g
+
+
+def _poisson(nel, distort, **tune):
+    ct = "Hexahedron" if len(nel) == 3 else "Quadrilateral"
+    g = fa.generate_grid(ct, nel, (0.0,) * len(nel), (1.0,) * len(nel))
+    if distort:
+        _move(g, nel, 5)
+    ip = fa.Lagrange(g.refshape, 1)
+    dh = fa.DofHandler(g).add("u", ip).close()
+    K = fa.allocate_matrix(fa.MI355XCSC, dh)
+    f = fa.allocate_vector(K)
+    fa.set_tuning(K, **tune)
+    cv = fa.CellValues(fa.QuadratureRule(g.refshape, 2), ip)
+    k = np.exp(np.random.default_rng(3).normal(0.0, 0.5, g.ncells))
+    fa.assemble_global(fa.start_assemble(K, f), cv, fa.create_coloring(g), fa.PoissonElement(k=k, source=1.0))
+    ch = fa.ConstraintHandler(dh)
+    ch.add(fa.Dirichlet("u", g.facetsets["left"], lambda x, t: 1.0 + x[1])).close()
+    fa.apply(K, f, ch)
+    return K, f
+
+
+def _check(K, f, mode, operator):
+    A, b = K.to_scipy(), f.to_numpy()
+    one = fa.solve(K, f, mode=mode, rtol=1e-12)
+    two = fa.solve(K, f, mode=mode, rtol=1e-12)
+    assert one.operator == operator
+    assert np.array_equal(one.u, two.u) and one.iterations == two.iterations
+    assert np.linalg.norm(b - A @ one.u) <= 2e-12 * np.linalg.norm(b)
+    fa.set_tuning(K, cg_elems=8)
+    sep = fa.solve(K, f, mode=mode, rtol=1e-12)
+    assert sep.operator == operator
+    assert np.linalg.norm(one.u - sep.u) <= 1e-8 * np.linalg.norm(sep.u)
+
+
+@pytest.mark.parametrize("nel", [(3, 2), (15, 15), (22, 22), (30, 33), (71, 69), (5, 400), (7, 7, 7), (9, 8, 7),
+                                 (2, 2, 200), (23, 19, 17), (63, 64, 65)])
+def test_rows_of_K(nel):
+    print("case resident rows of K", nel, flush=True)
+    K, f = _poisson(nel, True, lattice=-1, cell_operator=-1)
+    _check(K, f, "cg", "sell")
+    if len(nel) == 2 or nel[0] < 60:
+        fa.set_tuning(K, cg_elems=0)
+        _check(K, f, "mixed", "sell")
+
+
+@pytest.mark.parametrize("nel", [(15, 15), (24, 21), (71, 69), (7, 7, 7), (13, 12, 11), (40, 38, 36)])
+@pytest.mark.parametrize("operator", ["lattice", "cells"])
+def test_lattice_rows(nel, operator):
+    print("case resident lattice rows", nel, operator, flush=True)
+    forms = dict(lattice=1, cell_operator=-1) if operator == "lattice" else dict(lattice=0, cell_operator=1)
+    K, f = _poisson(nel, operator == "lattice", **forms)
+    for mode in ("mixed", "cg"):
+        fa.set_tuning(K, cg_elems=0)
+        _check(K, f, mode, operator)
+
+
+@pytest.mark.parametrize("nel", [(11, 11), (40, 23), (130, 64)])
+def test_vector_field(nel):
+    print("case resident vector field", nel, flush=True)
+    g = _move(fa.generate_grid("Quadrilateral", nel, (0.0, 0.0), (2.0, 1.0)), nel, 6)
+    ip = fa.Lagrange("RefQuadrilateral", 1) ** 2
+    dh = fa.DofHandler(g).add("u", ip).close()
+    K = fa.allocate_matrix(fa.MI355XCSC, dh)
+    f = fa.allocate_vector(K)
+    cv = fa.CellValues(fa.QuadratureRule("RefQuadrilateral", 2), ip)
+    fa.assemble_global(fa.start_assemble(K, f), cv, fa.create_coloring(g), fa.ElasticityElement(nu=0.3))
+    fa.add_point_load(K, f, [dh.ndofs], [-1.0])
+    ch = fa.ConstraintHandler(dh)
+    ch.add(fa.Dirichlet("u", g.facetsets["left"] + g.facetsets["right"], lambda x, t: [0.0, 0.0])).close()
+    fa.apply(K, f, ch)
+    for mode in ("cg", "mixed"):
+        fa.set_tuning(K, cg_elems=0)
+        _check(K, f, mode, "sell")
