@@ -6,7 +6,7 @@
  * every problem of a set, each with its own Grid, DofHandler, create_sparsity_pattern
  * (src/Dofs/sparsity_pattern.jl), create_coloring (src/Grid/coloring.jl) and
  * ConstraintHandler.  Here all problems live in one device context; assembly is one
- * persistent kernel draining a (problem, colour, chunk) work queue, captured in a
+ * launch per colour over every problem's (colour, chunk) items, captured in a
  * hipGraph; the solve is one batched mixed-precision CG with per-problem scalars.
  *
  * Conventions are those of ferrite_mi355x.h: 1-based indices in the host arrays,
@@ -33,7 +33,7 @@ typedef struct {
 } fem_batch_cfg;
 
 typedef struct {
-  double assemble_ms;        /* persistent assembly graph (zero + kernel) */
+  double assemble_ms;        /* assembly graph (zero + one launch per colour) */
   double apply_ms;           /* batched apply! (meandiag, zero rows/cols, diagonal) */
   double solve_ms;           /* batched CG until the last problem converged */
   double total_ms;           /* whole run, start of assembly to the last convergence */
@@ -77,7 +77,7 @@ int32_t fem_batch_run(fem_batch* b, const fem_batch_cfg* cfg, fem_batch_info* in
  * iterations; arrays of length nproblems. */
 int32_t fem_batch_problem_stats(const fem_batch* b, double* completion_ms, int32_t* iterations);
 
-/* Assembly only (zero + persistent kernel), timed with HIP events: *ms. */
+/* Assembly only (zero + one launch per colour), timed with HIP events: *ms. */
 int32_t fem_batch_assemble_only(fem_batch* b, int32_t precision, int32_t cells_per_wg, int32_t chunk, double* ms);
 
 /* Copy problem `prob` (0-based) back: K.nzval[nnz], f[ndofs], u[ndofs]; NULL skips. */
