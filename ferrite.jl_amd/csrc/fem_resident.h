@@ -40,4 +40,18 @@ int resident_run(fem_ctx* c, ResOp* op, const double* res, const double* sc, X* 
 
 void resident_free(ResOp** op);
 
+// The same on the 3D cell form in FP32, for lattices too large for the rows' entries
+// (fem_resident_cells.hip).
+struct BrickSource {
+  int32_t px = 0, pxy = 0;
+  const float *t = nullptr, *kc = nullptr;   // masked scaling and coefficients on the padded rows
+  const int32_t* dofp = nullptr;
+  double f[8] = {};
+};
+struct BrickOp;
+int brick_prepare(fem_ctx* c, BrickOp** op, int nx, int ny, int nz, bool* ok);
+int brick_run(fem_ctx* c, BrickOp* op, const BrickSource& s, const double* res, const double* sc, float* p, float* sv,
+              double* u, Scal* scal, double hold_factor2, double tol2, int restart, int lim, bool* launched);
+void brick_free(BrickOp** op);
+
 }  // namespace fem

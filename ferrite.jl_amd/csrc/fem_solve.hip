@@ -170,6 +170,8 @@ struct SolverWork {
   int elem_grid = 0;
   ResOp *res_csc = nullptr, *res_lat = nullptr;   // resident CG on K's rows, on the lattice's rows
   ResOp* res_op = nullptr;     // the one the current solve runs on, or null
+  BrickOp* bricks = nullptr;   // resident CG on the 3D cell form
+  bool use_bricks = false;     // the current solve runs on it
   bool res_off = false;        // a resident launch was not taken or gave up: not tried again
   int64_t cap32 = 0, cap64 = 0;   // length of the recurrence vectors
   int sell_grid = 0;           // blocks of the SELL SpMV (fixed: its partial count)
@@ -214,6 +216,7 @@ void free_solver(fem_ctx* c) {
   elem_op_free(&w->eop);
   resident_free(&w->res_csc);
   resident_free(&w->res_lat);
+  brick_free(&w->bricks);
   CellOp& cl = w->cells;
   dev_free(&cl.corg); dev_free(&cl.kc64); dev_free(&cl.kc32); dev_free(&cl.t64); dev_free(&cl.t32);
   dev_free(&cl.cnt); dev_free(&cl.up64); dev_free(&cl.yp64); dev_free(&cl.tm64); dev_free(&cl.s0);
@@ -2298,6 +2301,7 @@ static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv, 
   w->use_cells = false;
   w->use_elem = false;
   w->res_op = nullptr;
+  w->use_bricks = false;
   const bool want = sizeof(X) == 4 ? c->tune.lattice != -1 : c->tune.lattice == 1;
   const bool want_cells = sizeof(X) == 4 ? c->tune.cell_operator != -1 : c->tune.cell_operator == 1;
   if (want || want_cells) {
@@ -2347,6 +2351,12 @@ static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv, 
     if (ok) {
       w->res_op = *op;
       return FEM_OK;
+    }
+    if (sizeof(X) == 4 && w->use_cells && cl.dim == 3) {
+      if ((rc = brick_prepare(c, &w->bricks, (int)l.px - 2, (int)(l.pxy / l.px) - 2, (int)(l.npad / l.pxy) - 2, &ok)))
+        return rc;
+      w->use_bricks = ok;
+      if (ok) return FEM_OK;
     }
   }
   if (w->use_lat || w->use_elem) return FEM_OK;
@@ -2613,17 +2623,28 @@ static int cg_run_resident(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double
   const int64_t most = ((int64_t)maxit + kBatch - 1) / kBatch * kBatch;   // as the batches round it up
   const int32_t* dofp = w->use_lat ? w->lat.dofp : nullptr;
   const double* res = c->d_f;
-  int rc, nho = 0, stall = 0;
+  int rc = FEM_OK, nho = 0, stall = 0;
   bool converged = false;
   double prev_true = bnorm2;
   Scal h{};
   FEM_HIP(c, hipEventRecord(c->ev0, c->stream));
   for (;;) {
     const int lim = (int)std::min<int64_t>(1 << 24, most - h.iters);
+    const int restart = res == c->d_f ? 1 : 0;
     bool launched = false;
-    if ((rc = resident_run<X>(c, w->res_op, res, w->sc, v.p, v.sv, c->d_u, w->s, dofp, hold_factor2, tol2,
-                              res == c->d_f ? 1 : 0, lim, &launched)))
-      return rc;
+    if (w->use_bricks) {
+      if constexpr (sizeof(X) == 4) {
+        const LatOp& l = w->lat;
+        BrickSource b{(int32_t)l.px, (int32_t)l.pxy, w->cells.t32, w->cells.kc32, l.dofp, {}};
+        for (int i = 0; i < 8; ++i) b.f[i] = w->cells.f[i];
+        rc = brick_run(c, w->bricks, b, res, w->sc, v.p, v.sv, c->d_u, w->s, hold_factor2, tol2, restart, lim,
+                       &launched);
+      }
+    } else {
+      rc = resident_run<X>(c, w->res_op, res, w->sc, v.p, v.sv, c->d_u, w->s, dofp, hold_factor2, tol2, restart, lim,
+                           &launched);
+    }
+    if (rc) return rc;
     if (!launched) {
       *gave_up = true;
       return FEM_OK;
@@ -2666,7 +2687,7 @@ static int cg_solve(fem_ctx* c, SolverWork* w, int jacobi, double bnorm2, double
     if constexpr (sizeof(X) == 4) return CgVecs<X>{w->x32, w->r32, w->wv32, w->p32, w->sv32, nv, map};
     else return CgVecs<X>{w->x, w->r, w->wv, w->p, w->sv, nv, map};
   };
-  if (w->res_op) {
+  if (w->res_op || w->use_bricks) {
     bool gave_up = false;
     rc = cg_run_resident<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, iters, handovers, ms, &gave_up);
     if (!gave_up) return rc;

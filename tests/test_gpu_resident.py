@@ -2,7 +2,7 @@
 
 Sizes at the edges of its parts: one block (up to a few hundred rows), one row more than a
 block's 512 threads, several rows per thread, rows whose entries lie in LDS (FP64, 27 entries,
-more than 1,024 rows per block); every source of rows (K's columns, lattice planes, cell form),
+more than 1,024 rows per block), lattices beyond that; every source of rows (K's columns, lattice planes, cell form),
 9, 18 and 27 entries per row.  An explicit launch shape of the separate kernels (cg_elems)
 selects those.  Both solve to a true residual of 1e-12, so their u differ by a few times
 cond · 1e-12: 1e-8, the bar the other solver tests use."""
@@ -77,6 +77,15 @@ def test_lattice_rows(nel, operator):
     for mode in ("mixed", "cg"):
         fa.set_tuning(K, cg_elems=0)
         _check(K, f, mode, operator)
+
+
+@pytest.mark.parametrize("nel", [(90, 84, 80), (61, 140, 66), (200, 60, 50)])
+def test_cell_bricks(nel):
+    """More rows than the entries of which fit on chip: bricks of the cell form (uneven cuts,
+    inhomogeneous prescribed rows on one side)."""
+    print("case resident cell bricks", nel, flush=True)
+    K, f = _poisson(nel, False)
+    _check(K, f, "mixed", "cells")
 
 
 @pytest.mark.parametrize("nel", [(11, 11), (40, 23), (130, 64)])
