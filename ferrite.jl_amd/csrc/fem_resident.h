@@ -12,10 +12,15 @@ namespace fem {
 struct ResSource {
   int src = 0;
   int64_t n = 0;                 // rows: dofs (0) or padded lattice rows (1, 2)
-  int dim = 0;                   // 1, 2: lattice dimension
+  int widest = 0;                // most entries of a column of K
+  int dim = 0;                   // lattice dimension; 0 with `node`: of the coordinates
+  const int32_t* node = nullptr;           // 0: a node of each row and the nodes' coordinates, or null:
+  const double* x[3] = {};                 //    those of the context's mesh
+  int nsys = 0;                            // independent systems, their row ranges sys[2 i], sys[2 i + 1];
+  const int32_t* sys = nullptr;            //    0: all rows are one
   int32_t px = 0, pxy = 0;
   int64_t npad = 0;
-  const int32_t* dofp = nullptr;
+  const int32_t *dofp = nullptr, *map = nullptr;   // map: the padded row of a dof
   const void* val = nullptr;     // 1: planes [s][npad]
   const double* kc = nullptr;    // 2: k_c at the padded row of each cell's first corner
   const void* t = nullptr;       // 2: masked scaling (X precision; 0 on prescribed rows and padding)
@@ -24,18 +29,29 @@ struct ResSource {
 
 struct ResOp;
 
+// What the launch did for one system.
+struct ResState {
+  double rr;                     // square of the true residual of u
+  int iters, handovers;
+  int status;                    // 1: rr <= tol2
+  int lost;                      // 1: a block gave up waiting for another one
+  int prods;                     // products with Â run
+  uint32_t epoch;                // exchange numbers used up to here
+  long long ticks, begin, end;   // 100 MHz clock: in block 0's products (time), the system's first and last
+};
+
 // Ready to run on `s` in FP32 or FP64 (structure once per pattern, values when K or the scaling
 // changed); *ok = false when the rows do not fit (the caller keeps the separate kernels).
 int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok);
 
-// One stretch of the recurrence: (re)seeded from the FP64 residual `res` (p, sv: the last
-// direction and Â times it), iterated until the hand-over or `lim` steps, x̂ folded into u.
-// dofp: the dof of a lattice row, or null.  The scalar record s goes in (rr, rzp, restart) and
-// out; s->pad = 1: gave up waiting for
-// another block (nothing was folded).  *launched = false: the device did not take the launch.
+// The whole solve K u = f from u = 0: the recurrence and its hand-overs (u, the FP64 residual, the
+// reseed) until the true residual meets the tolerance, stalls, or `lim` steps are done.  in:
+// per system the squares of |f| and of the tolerance in device memory, or null (one system):
+// bnorm2, tol2.  Returns when it is done; *out: what it did per system, until the next run.
+// *launched = false: the device did not take the launch.
 template <typename X>
-int resident_run(fem_ctx* c, ResOp* op, const double* res, const double* sc, X* p, X* sv, double* u, Scal* s,
-                 const int32_t* dofp, double hold_factor2, double tol2, int restart, int lim,
+int resident_run(fem_ctx* c, ResOp* op, const ResSource& s, const double* sc, const double* f, double* u,
+                 const double* in, double bnorm2, double tol2, double hold_factor2, int lim, const ResState** out,
                  bool* launched);
 
 void resident_free(ResOp** op);

@@ -1,5 +1,5 @@
 // Resident CG: the Chronopoulos–Gear recurrence of fem_solve.hip (same scalars, same hand-over
-// rule, same reseed) in one cooperative launch per stretch between two hand-overs.
+// rule, same reseed) in one cooperative launch per solve, hand-overs included.
 //
 // What bounds the separate kernels on systems of up to a few hundred thousand rows is not their
 // bytes but two launches per iteration.  Here every block (one per CU) owns a compact part of
@@ -9,7 +9,13 @@
 // w = Âr̂ of its rows and its partials of γ = r̂·r̂ and δ = r̂·w, and reads the others' partials
 // and the w of its coupled rows; with those it also moves the coupled rows' ŝ and r̂ itself
 // (the same operations on the same values as their owner, so they stay equal bit for bit), and
-// the next product needs no second exchange.
+// the next product needs no second exchange.  A hand-over folds x̂ into the FP64 u, publishes the u
+// other blocks read, forms the FP64 residual f − K u from K's own entries and publishes the new r̂:
+// two more exchanges instead of half a dozen launches and a host round trip (301×227 Q1 quads in
+// FP32, 13 hand-overs: whole assembly and solve 5.78 → 5.14 ms; 47×53×61 hexes, 10: 2.68 → 2.29).
+//
+// Several independent systems can share a launch, their rows cut into separate parts: sums and
+// waits stay inside a system's own blocks, which leave when their system is done.
 //
 // The exchange has no barrier and no fence.  Every published value travels in 8-byte words of
 // 32 data bits and the exchange's 32-bit number, written and read with agent-scope accesses
@@ -21,9 +27,9 @@
 // publishing, so every other block gives up too, and the host runs the separate kernels.
 //
 // Measured, µs per iteration, separate kernels → here: 100×100 Q1 quads FP64 11.7 → 3.0 (21
-// blocks); 24×20×17 distorted hexes FP64 17.4 → 3.6 (24); 64³ hexes FP64 33 → 6.1 (250); 512×256
-// Q1² quads FP64 26.5 → 3.95 (180); 301×227 Q1 quads FP32 cell form 13.3 → 4.0 and 47×53×61 hexes
-// FP32 planes 16.2 → 6.6 (both with their hand-overs).  At 100×100 an iteration is about 0.3 µs of
+// blocks); 24×20×17 distorted hexes FP64 17.4 → 3.6 (24); 64³ hexes FP64 33 → 6.4 (250); 512×256
+// Q1² quads FP64 26.5 → 4.0 (180); 301×227 Q1 quads FP32 cell form 13.3 → 3.75 and 47×53×61 hexes
+// FP32 planes 16.2 → 5.9 (both with their hand-overs).  At 100×100 an iteration is about 0.25 µs of
 // products, 0.3 µs of sums inside the block, 1.3 µs until the other blocks' values are there and
 // 0.5 µs of scalars and vector moves.
 #include <algorithm>
@@ -34,13 +40,14 @@
 namespace fem {
 
 constexpr int kResRows = 256;           // least rows per block when there are several
+constexpr int kMaxStallRes = 6;         // hand-overs in a row without progress (kMaxStall of fem_solve.hip)
 
 struct ResOp {
   int state = 0;                        // 1 usable, −1 does not fit
-  int64_t n = 0;                        // rows of the numbering
   // parts: one block each; own rows (those other parts read first, each class ascending),
   // coupled rows (ascending), published slots
-  int nb = 0, Rmax = 0, Rp = 0, nz = 0, nlocmax = 0, nhmax = 0, nslots = 0;
+  int nb = 0, ng = 0, Rmax = 0, Rp = 0, nz = 0, nlocmax = 0, nhmax = 0, nslots = 0;
+  int4* grp = nullptr;                  // [nb] system of each part, its first part, how many, 0
   int32_t* oofs = nullptr;              // [nb + 1] ranges of orow
   int32_t* orow = nullptr;              // own rows of each part
   int32_t* pofs = nullptr;              // [nb + 1] published slots: one per row other parts read
@@ -51,10 +58,13 @@ struct ResOp {
   // values per precision: [nb][nz][Rp]
   float* val32 = nullptr;
   double* val64 = nullptr;
+  double* raw = nullptr;                // [nb][nz][Rp] unscaled FP64 entries (FP32 solver: residuals)
   uint64_t ver[2] = {0, 0}, aux[2] = {0, 0};
   int jac[2] = {-1, -1}, vsrc[2] = {-1, -1};
   // exchange buffers and the number of the last exchange handed out
   uint32_t* wx = nullptr;               // [2][nslots] values (8 or 16 bytes each)
+  uint32_t* wu = nullptr;               // [nslots] FP64 values: u of a hand-over
+  ResState* st = nullptr;               // [ng] pinned host memory, written by the launch
   uint32_t* rec = nullptr;              // [2][kResCopies][2][kResMaxBlocks] values of 16 bytes
   uint32_t epoch = 0;
 };
@@ -62,8 +72,10 @@ struct ResOp {
 void resident_free(ResOp** op) {
   if (!*op) return;
   ResOp* o = *op;
-  dev_free(&o->oofs); dev_free(&o->orow); dev_free(&o->pofs); dev_free(&o->hoff); dev_free(&o->hrow);
-  dev_free(&o->hslot); dev_free(&o->ai); dev_free(&o->val32); dev_free(&o->val64); dev_free(&o->wx); dev_free(&o->rec);
+  dev_free(&o->grp); dev_free(&o->oofs); dev_free(&o->orow); dev_free(&o->pofs); dev_free(&o->hoff); dev_free(&o->hrow);
+  dev_free(&o->hslot); dev_free(&o->ai); dev_free(&o->val32); dev_free(&o->val64); dev_free(&o->raw);
+  dev_free(&o->wx); dev_free(&o->wu);
+  if (o->st) (void)hipHostFree(o->st); dev_free(&o->rec);
   delete o;
   *op = nullptr;
 }
@@ -73,23 +85,19 @@ struct ResRows {
   int src, dim;
   int64_t n, npad;
   int32_t px, pxy;
-  const int32_t *colptr, *rowval, *dofp;
+  const int32_t *colptr, *rowval, *dofp, *map;
   const double *nzval, *sc, *kc;
   const void *val, *t;
   double f[8];
 };
 
-// Column of entry k of a row, −1 when the row has no such entry.  Lattice rows: entry k is the
-// neighbour with code k (3D, (dx + 1) + 3 (dy + 1) + 9 (dz + 1)) or 9 + k (2D).
+// Row of entry k of a row in the order of K's column, −1 when the column has no such entry.
 __device__ __forceinline__ int32_t res_col(const ResRows& a, int32_t row, int k) {
-  if (a.src == 0) {
-    const int32_t p = a.colptr[row] + k;
-    return p < a.colptr[row + 1] ? a.rowval[p] : -1;
-  }
-  if (a.dofp[row] < 0) return -1;
-  const int code = a.dim == 3 ? k : 9 + k;
-  const int32_t q = row + (code % 3 - 1) + a.px * ((code / 3) % 3 - 1) + (a.dim == 3 ? a.pxy * (code / 9 - 1) : 0);
-  return a.dofp[q] >= 0 ? q : -1;
+  const int32_t j = a.src == 0 ? row : a.dofp[row];
+  if (j < 0) return -1;
+  const int32_t p = a.colptr[j] + k;
+  if (p >= a.colptr[j + 1]) return -1;
+  return a.src == 0 ? a.rowval[p] : a.map[a.rowval[p]];
 }
 
 // ---- parts --------------------------------------------------------------------------------
@@ -99,15 +107,12 @@ __device__ __forceinline__ int32_t res_col(const ResRows& a, int32_t row, int k)
 // rows reads 1,000): what the parts publish and read per iteration is what bounds it.
 constexpr int kResBins = 4096;
 
-// Bin of a row along each axis.  Lattice rows: their lattice index.  Others: the position of a
-// node of the row's first cell, scaled by the bounding box.
+// Position of a row: its lattice index, or that of a node of its first cell.
 struct ResPos {
-  int src, dim;
-  int64_t n;
+  int src, dim;                      // dim: of the lattice / of the coordinates
   int32_t px, pxy;
   const int32_t *dofp, *node;        // node: [n]
   const double* x[3];
-  double lo[3], inv[3];              // (x − lo) inv in [0, kResBins)
 };
 __device__ __forceinline__ bool res_pos(const ResPos& a, int32_t row, double (&x)[3]) {
   x[1] = x[2] = 0.0;
@@ -123,26 +128,35 @@ __device__ __forceinline__ bool res_pos(const ResPos& a, int32_t row, double (&x
   for (int d = 0; d < a.dim; ++d) x[d] = a.x[d][nd];
   return true;
 }
-__device__ __forceinline__ int res_bin(const ResPos& a, const double (&x)[3], int d) {
-  return max(0, min(kResBins - 1, (int)((x[d] - a.lo[d]) * a.inv[d])));
+
+// A system of the launch: its rows, and (x − lo) inv in [0, kResBins) along each axis.
+struct ResSystem {
+  int32_t row0, row1;
+  double lo[3], inv[3];
+};
+__device__ __forceinline__ int res_bin(const ResSystem& g, const double (&x)[3], int d) {
+  return max(0, min(kResBins - 1, (int)((x[d] - g.lo[d]) * g.inv[d])));
 }
 
-// One block: bounding box of the rows (out[0..2], out[3..5]), their number (out[9]), and per axis
-// the mean over sampled rows of the largest distance to a row they couple to (out[6..8]): the
-// spacing of the rows.
-__global__ __launch_bounds__(1024) void k_res_geom(ResPos g, ResRows a, int nz, double* __restrict__ out) {
+// One block per system: bounding box of its rows (out[0..2], out[3..5]), their number (out[9]),
+// and per axis the mean over sampled rows of the largest distance to a row they couple to
+// (out[6..8]): the spacing of the rows.
+__global__ __launch_bounds__(1024) void k_res_geom(ResPos g, ResRows a, const ResSystem* __restrict__ sys, int nz,
+                                                   double* __restrict__ out) {
   __shared__ double sh[10][16];
+  __shared__ double hsum[16];
+  const int32_t row0 = sys[blockIdx.x].row0, row1 = sys[blockIdx.x].row1;
   double v[10] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300, 0.0, 0.0, 0.0, 0.0};
-  for (int64_t row = threadIdx.x; row < g.n; row += 1024) {
+  for (int32_t row = row0 + (int32_t)threadIdx.x; row < row1; row += 1024) {
     double x[3];
-    if (!res_pos(g, (int32_t)row, x)) continue;
+    if (!res_pos(g, row, x)) continue;
     for (int d = 0; d < 3; ++d) {
       v[d] = fmin(v[d], x[d]);
       v[3 + d] = fmax(v[3 + d], x[d]);
     }
     v[9] += 1.0;
   }
-  const int32_t s = (int32_t)(((int64_t)threadIdx.x * g.n) / 1024);
+  const int32_t s = row0 + (int32_t)(((int64_t)threadIdx.x * (row1 - row0)) / 1024);
   double xs[3], hs = 0.0;
   if (res_pos(g, s, xs)) {
     double far[3] = {0.0, 0.0, 0.0};
@@ -161,7 +175,6 @@ __global__ __launch_bounds__(1024) void k_res_geom(ResPos g, ResRows a, int nz, 
       v[i] = i < 3 ? fmin(v[i], u) : i < 6 ? fmax(v[i], u) : v[i] + u;
     }
   for (int o = 32; o > 0; o >>= 1) hs += __shfl_down(hs, o, 64);
-  __shared__ double hsum[16];
   if ((threadIdx.x & 63) == 0) {
     for (int i = 0; i < 10; ++i) sh[i][threadIdx.x >> 6] = v[i];
     hsum[threadIdx.x >> 6] = hs;
@@ -175,21 +188,35 @@ __global__ __launch_bounds__(1024) void k_res_geom(ResPos g, ResRows a, int nz, 
       r = i < 3 ? fmin(r, u) : i < 6 ? fmax(r, u) : r + u;
       h += hsum[w];
     }
-    out[i] = i >= 6 && i < 9 ? r / fmax(h, 1.0) : r;
+    out[10 * blockIdx.x + i] = i >= 6 && i < 9 ? r / fmax(h, 1.0) : r;
+  }
+}
+
+// part = the system of each row that has a place, −1 elsewhere.
+__global__ __launch_bounds__(256) void k_res_start(ResPos g, const ResSystem* __restrict__ sys,
+                                                   int32_t* __restrict__ part) {
+  const int32_t row0 = sys[blockIdx.y].row0, row1 = sys[blockIdx.y].row1;
+  for (int32_t row = row0 + (int32_t)(blockIdx.x * 256 + threadIdx.x); row < row1; row += gridDim.x * 256) {
+    double x[3];
+    part[row] = res_pos(g, row, x) ? (int32_t)blockIdx.y : -1;
   }
 }
 
 // One level of the cut along axis d: rows per (slab, bin), the finer slab of each (slab, bin),
-// the rows' finer slabs.  part starts as 0 (level 0).
-__global__ __launch_bounds__(256) void k_res_hist(ResPos g, int d, const int32_t* __restrict__ part,
-                                                  int32_t* __restrict__ hist) {
-  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < g.n; row += (int64_t)gridDim.x * 256) {
+// the rows' finer slabs.  A slab: its system, how many slabs it is cut into, the first of them.
+__global__ __launch_bounds__(256) void k_res_hist(ResPos g, const ResSystem* __restrict__ sys,
+                                                  const int4* __restrict__ slab, int64_t n, int d,
+                                                  const int32_t* __restrict__ part, int32_t* __restrict__ hist) {
+  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < n; row += (int64_t)gridDim.x * 256) {
+    const int32_t p = part[row];
     double x[3];
-    if (res_pos(g, (int32_t)row, x)) atomicAdd(&hist[(int64_t)part[row] * kResBins + res_bin(g, x, d)], 1);
+    if (p >= 0 && res_pos(g, (int32_t)row, x))
+      atomicAdd(&hist[(int64_t)p * kResBins + res_bin(sys[slab[p].x], x, d)], 1);
   }
 }
-__global__ __launch_bounds__(256) void k_res_cut(int s, int32_t* __restrict__ hist) {   // one block per slab
+__global__ __launch_bounds__(256) void k_res_cut(const int4* __restrict__ slab, int32_t* __restrict__ hist) {   // one block per slab
   __shared__ int32_t sum[256];
+  const int s = slab[blockIdx.x].y, first = slab[blockIdx.x].z;
   int32_t* h = hist + (int64_t)blockIdx.x * kResBins;
   constexpr int PER = kResBins / 256;
   int32_t c[PER], all = 0;
@@ -207,19 +234,16 @@ __global__ __launch_bounds__(256) void k_res_cut(int s, int32_t* __restrict__ hi
   for (int i = 0; i < PER; ++i) {   // the slab that holds the bin's middle row
     const int64_t f = total > 0 ? (2 * before + c[i]) * s / (2 * total) : 0;
     before += c[i];
-    h[threadIdx.x * PER + i] = (int32_t)min<int64_t>(f, s - 1);
+    h[threadIdx.x * PER + i] = first + (int32_t)min<int64_t>(f, s - 1);
   }
 }
-__global__ __launch_bounds__(256) void k_res_split(ResPos g, int d, int s, const int32_t* __restrict__ hist,
-                                                   int32_t* __restrict__ part) {
-  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < g.n; row += (int64_t)gridDim.x * 256) {
-    double x[3];
-    if (!res_pos(g, (int32_t)row, x)) {
-      part[row] = -1;
-      continue;
-    }
+__global__ __launch_bounds__(256) void k_res_split(ResPos g, const ResSystem* __restrict__ sys,
+                                                   const int4* __restrict__ slab, int64_t n, int d,
+                                                   const int32_t* __restrict__ hist, int32_t* __restrict__ part) {
+  for (int64_t row = (int64_t)blockIdx.x * 256 + threadIdx.x; row < n; row += (int64_t)gridDim.x * 256) {
     const int32_t p = part[row];
-    part[row] = p * s + hist[(int64_t)p * kResBins + res_bin(g, x, d)];
+    double x[3];
+    if (p >= 0 && res_pos(g, (int32_t)row, x)) part[row] = hist[(int64_t)p * kResBins + res_bin(sys[slab[p].x], x, d)];
   }
 }
 
@@ -282,27 +306,28 @@ __global__ __launch_bounds__(1024) void k_res_sort(int pow2, const int32_t* __re
   if (threadIdx.x == 0) shared[blockIdx.x] = ns;
 }
 
-// A part's bitmap of the rows of other parts that its rows name, in LDS.
-__device__ __forceinline__ void res_mark(const ResRows& a, int nz, const int32_t* __restrict__ part,
+// A part's bitmap of the rows of other parts that its rows name, in LDS: of the rows of its
+// system, which start at row0.
+__device__ __forceinline__ void res_mark(const ResRows& a, int nz, int32_t row0, const int32_t* __restrict__ part,
                                          const int32_t* __restrict__ own, int m, uint32_t* bm, int words) {
   for (int i = threadIdx.x; i < words; i += blockDim.x) bm[i] = 0u;
   __syncthreads();
   for (int i = threadIdx.x; i < m; i += blockDim.x)
     for (int k = 0; k < nz; ++k) {
       const int32_t q = res_col(a, own[i], k);
-      if (q >= 0 && part[q] != (int32_t)blockIdx.x) atomicOr(&bm[q >> 5], 1u << (q & 31));
+      if (q >= 0 && part[q] != (int32_t)blockIdx.x) atomicOr(&bm[(q - row0) >> 5], 1u << ((q - row0) & 31));
     }
   __syncthreads();
 }
 
-__global__ __launch_bounds__(256) void k_res_count(ResRows a, int nz, const int32_t* __restrict__ part,
+__global__ __launch_bounds__(256) void k_res_count(ResRows a, int nz, int words, const ResSystem* __restrict__ sys,
+                                                   const int4* __restrict__ grp, const int32_t* __restrict__ part,
                                                    const int32_t* __restrict__ oofs,
                                                    const int32_t* __restrict__ orow, int32_t* __restrict__ cnt) {
   extern __shared__ uint32_t res_bm[];
   __shared__ int tot;
-  const int words = (int)((a.n + 31) / 32);
   if (threadIdx.x == 0) tot = 0;
-  res_mark(a, nz, part, orow + oofs[blockIdx.x], oofs[blockIdx.x + 1] - oofs[blockIdx.x], res_bm, words);
+  res_mark(a, nz, sys[grp[blockIdx.x].x].row0, part, orow + oofs[blockIdx.x], oofs[blockIdx.x + 1] - oofs[blockIdx.x], res_bm, words);
   int all = 0;
   for (int i = threadIdx.x; i < words; i += blockDim.x) all += __popc(res_bm[i]);
   atomicAdd(&tot, all);
@@ -312,17 +337,18 @@ __global__ __launch_bounds__(256) void k_res_count(ResRows a, int nz, const int3
 
 // The coupled rows of each part with their slots, and the entries' positions in its local
 // numbering: own rows by rank, then the coupled rows.
-__global__ __launch_bounds__(256) void k_res_fill(ResRows a, int nz, int Rp, const int32_t* __restrict__ part,
+__global__ __launch_bounds__(256) void k_res_fill(ResRows a, int nz, int Rp, int words, const ResSystem* __restrict__ sys,
+                                                  const int4* __restrict__ grp, const int32_t* __restrict__ part,
                                                   const int32_t* __restrict__ rank, const int32_t* __restrict__ oofs,
                                                   const int32_t* __restrict__ orow, const int32_t* __restrict__ pofs,
                                                   const int32_t* __restrict__ hoff, int32_t* __restrict__ hrow,
                                                   int32_t* __restrict__ hslot, uint32_t* __restrict__ ai) {
   extern __shared__ uint32_t res_bm[];
-  const int words = (int)((a.n + 31) / 32);
   const int ng = (words + 7) / 8;
+  const int32_t row0 = sys[grp[blockIdx.x].x].row0;
   uint32_t* pre = res_bm + words;    // [ng] rows before each group of 8 words
   const int32_t o0 = oofs[blockIdx.x], m = oofs[blockIdx.x + 1] - o0, h0 = hoff[blockIdx.x];
-  res_mark(a, nz, part, orow + o0, m, res_bm, words);
+  res_mark(a, nz, row0, part, orow + o0, m, res_bm, words);
   for (int g = threadIdx.x; g < ng; g += blockDim.x) {
     uint32_t c = 0;
     for (int i = 8 * g; i < min(words, 8 * g + 8); ++i) c += __popc(res_bm[i]);
@@ -345,6 +371,7 @@ __global__ __launch_bounds__(256) void k_res_fill(ResRows a, int nz, int Rp, con
   }
   __syncthreads();
   auto coupled = [&](int32_t q) {    // place of a marked row
+    q -= row0;
     const int w = q >> 5, g = w >> 3;
     uint32_t l = pre[g];
     for (int i = 8 * g; i < w; ++i) l += __popc(res_bm[i]);
@@ -353,7 +380,7 @@ __global__ __launch_bounds__(256) void k_res_fill(ResRows a, int nz, int Rp, con
   for (int i = threadIdx.x; i < words; i += blockDim.x) {
     uint32_t bits = res_bm[i];
     while (bits) {
-      const int32_t q = i * 32 + __ffs(bits) - 1;
+      const int32_t q = row0 + i * 32 + __ffs(bits) - 1;
       bits &= bits - 1;
       const int32_t h = h0 + (int32_t)coupled(q);
       hrow[h] = q;
@@ -374,111 +401,150 @@ __global__ __launch_bounds__(256) void k_res_fill(ResRows a, int nz, int Rp, con
   }
 }
 
-// Values of the rows' entries in X precision (0 where an entry is missing).
+// Values of the rows' entries in X precision (0 where an entry is missing), and unscaled in raw.
 template <typename X>
 __global__ __launch_bounds__(256) void k_res_vals(ResRows a, int nz, int Rp, int nb, const int32_t* __restrict__ oofs,
-                                                  const int32_t* __restrict__ orow, X* __restrict__ val) {
+                                                  const int32_t* __restrict__ orow, X* __restrict__ val,
+                                                  double* __restrict__ raw) {
   for (int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x; g < (int64_t)nb * Rp; g += (int64_t)gridDim.x * 256) {
     const int b = (int)(g / Rp), i = (int)(g - (int64_t)b * Rp);
     const int32_t o0 = oofs[b];
     const bool in = i < oofs[b + 1] - o0;
-    const int64_t row = in ? orow[o0 + i] : 0;
-    X* out = val + (int64_t)b * nz * Rp + i;
-    if (a.src == 0) {
-      const int32_t p0 = in ? a.colptr[row] : 0, len = in ? a.colptr[row + 1] - p0 : 0;
-      const double sr = in ? a.sc[row] : 0.0;
-      for (int k0 = 0; k0 < nz; k0 += 9) {   // nz is a multiple of 9
-        double v[9], sj[9];
-#pragma unroll
-        for (int u = 0; u < 9; ++u) {
-          const bool real = k0 + u < len;
-          v[u] = real ? a.nzval[p0 + k0 + u] : 0.0;
-          sj[u] = real ? a.sc[a.rowval[p0 + k0 + u]] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < 9; ++u) out[(int64_t)(k0 + u) * Rp] = (X)(v[u] * (sr * sj[u]));
-      }
-      continue;
-    }
-    const bool real = in && a.dofp[row] >= 0;
-    if (a.src == 1) {
-      const X* val0 = static_cast<const X*>(a.val);
-      for (int k = 0; k < nz; ++k) {
-        const int32_t q = real ? res_col(a, (int32_t)row, k) : -1;
-        const int code = a.dim == 3 ? k : 9 + k;
-        X v = X(0);
-        if (q >= 0) v = code >= 13 ? val0[(int64_t)(code - 13) * a.npad + row] : val0[(int64_t)(13 - code) * a.npad + q];
-        out[(int64_t)k * Rp] = v;
-      }
-      continue;
-    }
-    // cell form: s_P s_Q f[class] Σ k over the cells that hold both corners, in FP64 and rounded
-    // once (Â stays symmetric to the last bit); a prescribed row (t = 0) keeps its unit diagonal
+    const int32_t row = in ? orow[o0 + i] : 0, j = a.src == 0 ? row : a.dofp[row];
+    const int64_t out = (int64_t)b * nz * Rp + i;
+    const int32_t p0 = in ? a.colptr[j] : 0, len = in ? a.colptr[j + 1] - p0 : 0;
+    const double sr = in ? a.sc[j] : 0.0;
+    // cell form: the coefficients around the row; a prescribed row (t = 0) keeps its unit diagonal
     const X* tt = static_cast<const X*>(a.t);
-    const bool free_p = real && tt[row] != X(0);
-    const double sp = free_p ? a.sc[a.dofp[row]] : 0.0;
-    double k8[8];
+    const bool free_p = a.src == 2 && in && tt[row] != X(0);
+    double k8[8] = {};
+    if (a.src == 2)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const bool on = real && (a.dim == 3 || e < 4);
-      k8[e] = on ? a.kc[row - (e & 1) - (int64_t)a.px * ((e >> 1) & 1) - (int64_t)a.pxy * (e >> 2)] : 0.0;
-    }
-    for (int k = 0; k < nz; ++k) {
-      const int32_t q = real ? res_col(a, (int32_t)row, k) : -1;
-      const int code = a.dim == 3 ? k : 9 + k;
-      const int dx = code % 3 - 1, dy = (code / 3) % 3 - 1, dz = code / 9 - 1;
-      double ks = 0.0;
+      for (int e = 0; e < 8; ++e)
+        if (in && (a.dim == 3 || e < 4))
+          k8[e] = a.kc[row - (e & 1) - (int64_t)a.px * ((e >> 1) & 1) - (int64_t)a.pxy * (e >> 2)];
+    for (int k0 = 0; k0 < nz; k0 += 9) {   // nz is a multiple of 9; nine entries in flight
+      double v[9], sj[9];
+      int32_t q[9];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const bool both = (dx == 0 || (e & 1) == (dx < 0)) && (dy == 0 || ((e >> 1) & 1) == (dy < 0)) &&
-                          (dz == 0 || (e >> 2) == (dz < 0));
-        ks += both ? k8[e] : 0.0;
+      for (int u = 0; u < 9; ++u) {
+        const bool real = k0 + u < len;
+        v[u] = real ? a.nzval[p0 + k0 + u] : 0.0;
+        q[u] = real ? a.rowval[p0 + k0 + u] : -1;
       }
-      double v = 0.0;
-      if (q >= 0) {
-        if (free_p && tt[q] != X(0)) v = a.f[(dx != 0) + 2 * (dy != 0) + 4 * (dz != 0)] * ks * (sp * a.sc[a.dofp[q]]);
-        if (!free_p && q == row) v = 1.0;
+#pragma unroll
+      for (int u = 0; u < 9; ++u) sj[u] = q[u] >= 0 ? a.sc[q[u]] : 0.0;
+#pragma unroll
+      for (int u = 0; u < 9; ++u) {
+        const int64_t at = out + (int64_t)(k0 + u) * Rp;
+        if (raw) raw[at] = v[u];
+        X x = X(0);
+        if (a.src == 0) {
+          x = (X)(v[u] * (sr * sj[u]));
+        } else if (q[u] >= 0) {
+          const int32_t Q = a.map[q[u]], off = Q - row, shift = 1 + a.px + (a.dim == 3 ? a.pxy : 0);
+          // lattice offsets as digits of off + shift (fem_solve.hip lat_code; the pattern is checked there)
+          const int32_t t = off + shift, rz = a.dim == 3 ? t % a.pxy : t;
+          const int dz = a.dim == 3 ? t / a.pxy - 1 : 0, dy = rz / a.px - 1, dx = rz % a.px - 1;
+          const bool near = t >= 0 && dx >= -1 && dx <= 1 && dy >= -1 && dy <= 1 && dz >= -1 && dz <= 1;
+          if (near && a.src == 1) {
+            const int code = (dx + 1) + 3 * (dy + 1) + 9 * (dz + 1);
+            const X* val0 = static_cast<const X*>(a.val);
+            x = code >= 13 ? val0[(int64_t)(code - 13) * a.npad + row] : val0[(int64_t)(13 - code) * a.npad + Q];
+          } else if (near) {
+            // s_P s_Q f[class] Σ k over the cells that hold both corners, in FP64 and rounded once
+            double ks = 0.0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              const bool both = (dx == 0 || (e & 1) == (dx < 0)) && (dy == 0 || ((e >> 1) & 1) == (dy < 0)) &&
+                                (dz == 0 || (e >> 2) == (dz < 0));
+              ks += both ? k8[e] : 0.0;
+            }
+            if (free_p && tt[Q] != X(0)) x = (X)(a.f[(dx != 0) + 2 * (dy != 0) + 4 * (dz != 0)] * ks * (sr * sj[u]));
+            if (!free_p && Q == row) x = X(1);
+          }
+        }
+        val[at] = x;
       }
-      out[(int64_t)k * Rp] = (X)v;
     }
   }
 }
 
 // ---- the recurrence -----------------------------------------------------------------------
+// Σ a[e] r[position e] of a row whose entries are in registers; pos[m]: the byte offsets of entries
+// 2 m and 2 m + 1.  The LDS reads of a group of entries are under way while the group before is
+// summed: left to itself the compiler, short of registers, waits for each (FP64, 18 entries, three
+// rows a thread: a product 1.55 → 0.60 µs, an iteration at 512×256 Q1² quads 4.8 → 4.0 µs).
+template <typename X, int NZ>
+__device__ __forceinline__ X gather_dot(const X* r, const X (&a)[NZ], const uint32_t (&pos)[(NZ + 1) / 2]) {
+  constexpr int G = sizeof(X) == 4 ? 6 : 4, NG = (NZ + G - 1) / G;   // G even
+  X v[2][G];
+  auto load = [&](int g) {
+#pragma unroll
+    for (int i = 0; i < G; i += 2) {
+      const int e = g * G + i;
+      if (e >= NZ) break;
+      const uint32_t q = pos[e / 2];
+      v[g & 1][i] = at_lds(r, q & 0xffffu);
+      if (e + 1 < NZ) v[g & 1][i + 1] = at_lds(r, q >> 16);
+    }
+  };
+  X acc = X(0);
+  load(0);
+#pragma unroll
+  for (int g = 0; g < NG; ++g) {
+    if (g + 1 < NG) load(g + 1);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < G; ++i)
+      if (g * G + i < NZ) acc += a[g * G + i] * v[g & 1][i];
+  }
+  return acc;
+}
+
 template <typename X>
 struct ResArgs {
-  int Rp, nb, nslots;
-  int nl, rl0;                // rows whose entries LDS holds; elements of r̂, ŝ and w there
-  int nhmax;
+  int Rp, nslots;
+  int nl, rl0, nhmax;            // rows whose entries LDS holds; elements of r̂, and of ŝ and w, there
+  const int4* grp;
   const int32_t *oofs, *orow, *pofs, *hoff, *hrow, *hslot;
   const uint32_t* ai;
   const X* val;
-  const int32_t* dofp;        // dof of a row (lattice rows), or null: the same index
-  const double *res, *sc;
-  X *p, *sv;
+  const double* raw;             // unscaled entries, or null: read from nzval
+  const int32_t* colptr;
+  const double* nzval;
+  const int32_t* dofp;           // dof of a row (lattice rows), or null: the same index
+  const double *f, *sc;
   double* u;
-  Scal* s;
-  uint32_t *wx, *rec;
-  double hold2, tol2;
+  const double* in;              // [ng][2] squares of the initial residual and the tolerance, or null: in0
+  ResState* st;
+  uint32_t *wx, *wu, *rec;
+  double in0[2], hold2;
   uint32_t epoch;
-  int restart, lim, time;
+  int lim, time;
 };
 
 // Rows per thread RT; the entries (NZ per row) of the first RRES stay in registers, those of the
-// block's other rows (a.nl of them) in LDS.  LDS: r̂ of
-// the rows the block reads (own, coupled, and a zero slot for the threads' unused rows); ŝ, w and
-// the slots of the coupled rows; the entries of a.nl rows.
+// block's other rows (a.nl of them) in LDS.  LDS: r̂ of the rows the block reads (own, coupled,
+// and a zero slot for the threads' unused rows), at a hand-over their u in its place; ŝ, w and the
+// slots of the coupled rows; the entries of a.nl rows.
 template <typename X, int NZ, int RRES, int RT>
 __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
   constexpr int NZ2 = (NZ + 1) / 2;
   constexpr int QS = NZ2 | 1;                 // a row's words in LDS (odd: no bank conflicts)
   constexpr int H = sizeof(X) == 4 ? 8 : 4;   // coupled rows a thread polls at once
+  // reads ahead of the sums, but not where the entries fill the registers (FP64, 27 entries: 64³
+  // hexes 6.4 µs per iteration without, 6.8 with)
+  constexpr bool AHEAD = sizeof(X) * NZ < 8 * 27;
   extern __shared__ __align__(16) unsigned char res_lds[];
   __shared__ double red[2][2][kResWaves];    // wave sums, alternating
   __shared__ double tot[2][2][4];            // sums of 64 blocks' partials each
   __shared__ int gaveup;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int b = blockIdx.x;
+  const int4 gr = a.grp[b];
+  const int b0 = gr.y, nb = gr.z;            // the system's blocks
+  const long long begin = wall_clock64();
   const int32_t o0 = a.oofs[b], nown = a.oofs[b + 1] - o0;
   const int32_t p0 = a.pofs[b], npub = a.pofs[b + 1] - p0;
   const int32_t h0 = a.hoff[b], nh = a.hoff[b + 1] - h0;
@@ -489,8 +555,8 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
   uint32_t* lq = reinterpret_cast<uint32_t*>(lv + (size_t)NZ * a.nl);
   int32_t* hl = reinterpret_cast<int32_t*>(lq + (size_t)QS * a.nl);
   const int zero = nown + nh;
-  const double rzp0 = a.s->rzp, rr0 = a.s->rr;
-  const bool keep0 = !a.restart && !a.s->restart && rzp0 > 0.0;
+  double rrt = a.in ? a.in[2 * gr.x] : a.in0[0];   // the true residual's square
+  const double tol2 = a.in ? a.in[2 * gr.x + 1] : a.in0[1];
   if (t == 0) {
     gaveup = 0;
     rl[zero] = X(0);
@@ -510,10 +576,10 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
 #pragma unroll
     for (int j = 0; j < NZ2; ++j) ai[k][j] = in ? ib[(int64_t)j * a.Rp + i] * (uint32_t)sizeof(X) : 0u;   // byte offsets
   }
-  // the seed r̂ = S res, the last direction and Â times it
+  // the first residual is f: r̂ = S f
   auto seed = [&](int32_t q) {
     const int32_t d = a.dofp ? a.dofp[q] : q;
-    return d >= 0 ? (X)(a.sc[d] * a.res[d]) : X(0);
+    return d >= 0 ? (X)(a.sc[d] * a.f[d]) : X(0);
   };
   X p[RT], sv[RT], x[RT], w[RT];
   int il[RT];                                // this thread's rows in rl
@@ -523,20 +589,12 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
     const bool in = i < nown;
     il[k] = in ? i : zero;
     p[k] = sv[k] = x[k] = X(0);
-    if (in) {
-      const int32_t row = a.orow[o0 + i];
-      rl[i] = seed(row);
-      if (keep0) {
-        p[k] = a.p[row];
-        sv[k] = a.sv[row];
-      }
-    }
+    if (in) rl[i] = seed(a.orow[o0 + i]);
   }
   for (int h = t; h < nh; h += kResT) {
-    const int32_t q = a.hrow[h0 + h];
     hl[h] = a.hslot[h0 + h];
-    sl[h] = keep0 ? a.sv[q] : X(0);
-    rl[nown + h] = seed(q);
+    sl[h] = X(0);
+    rl[nown + h] = seed(a.hrow[h0 + h]);
   }
   for (int i = t; i < a.nl; i += kResT) {
     const int row = RRES * kResT + i;
@@ -560,8 +618,8 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
       if (k * kResT < npub) ll_put(ro, (uint32_t)(t + k * kResT), w[k], ep);
   };
   double rzp = 0.0, alpha = 0.0, irz = 0.0, ira = 0.0;   // γ and α of the last step; 1 / γ, 1 / (γ α)
-  // Sums g0, g1 over all blocks; with `halo`, reads the coupled rows' w into wl.  Every thread
-  // returns the same sums; false when a wait was given up.
+  // Sums g0, g1 over the system's blocks; with `halo`, reads the coupled rows' w into wl.  Every
+  // thread returns the same sums; false when a wait was given up.
   auto exchange = [&](double& g0, double& g1, bool halo) {
     const int par = (int)(ep & 1u);
     const double v0 = wave_sum63(g0), v1 = wave_sum63(g1);
@@ -570,7 +628,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
       red[par][1][wave] = v1;
     }
     res_barrier();
-    if (a.nb == 1) {
+    if (nb == 1) {
       irz = 1.0 / rzp;
       ira = 1.0 / (rzp * alpha);
       g0 = g1 = 0.0;
@@ -591,12 +649,12 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
       for (int i = 0; i < kResWaves; ++i) sum += red[par][t & 1][i];
       ll_put(rr, rec + (uint32_t)(t * kResMaxBlocks + b), sum, ep);
     }
-    const uint32_t rin = rec + (uint32_t)((b % kResCopies) * 2 * kResMaxBlocks + t);
+    const uint32_t rin = rec + (uint32_t)((b % kResCopies) * 2 * kResMaxBlocks + b0 + t);
     if (halo) {   // reciprocals of the last step's scalars, while the values travel
       irz = 1.0 / rzp;
       ira = 1.0 / (rzp * alpha);
     }
-    const bool reader = t < a.nb;      // thread t reads block t's record
+    const bool reader = t < nb;        // thread t reads the record of the system's block t
     bool lost = false, need = reader;
     U4 q0 = {}, q1 = {};
     if (halo) {                        // the coupled rows' w, and the records along with them
@@ -653,167 +711,251 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
     return gaveup == 0;
   };
 
-  double rz = 0.0, rz0 = 0.0, gstop = 0.0, beta = 0.0, gam = 0.0, pq = 0.0;
-  long long ticks = 0;
-  int done = 0, restart = 0, prods = 0, it = 0;
-  bool first = true, ok = true;
-  for (;;) {
-    // w = Â r̂ on the block's rows; γ = r̂·r̂ and δ = r̂·w (in a reseed r̂·p instead)
-    const long long c0 = a.time ? wall_clock64() : 0;
+  // w = S (f − K u) on the block's rows after u += S x̂, and the partial sum of its square unscaled:
+  // from the unscaled entries, in FP64, u of the coupled rows by their own slots (whose tag no
+  // other hand-over has; the waits of the iterations in between keep a slot until it was read).
+  // The arguments are read again: kept in scalar registers they would crowd the iteration.
+  bool fresh = true;                         // u is still to be written
+  auto true_residual = [&](double& sum) {
+    const ResArgs<X>& z = *reinterpret_cast<const ResArgs<X>*>(res_kernargs());
+    double* ul = reinterpret_cast<double*>(res_lds);
+    int tt = t;
+    asm volatile("" : "+v"(tt));             // no addresses made ahead of the loop
+    const int32_t* own = z.orow + o0;
+    const __amdgpu_buffer_rsrc_t ru = buf_rsrc(z.wu, 16u * (uint32_t)z.nslots);
+    const __amdgpu_buffer_rsrc_t ro = buf_rsrc(reinterpret_cast<const U4*>(z.wu) + p0, 16u * (uint32_t)npub);
+    res_barrier();                           // r̂ was read
 #pragma unroll
     for (int k = 0; k < RT; ++k) {
-      w[k] = X(0);
-      if (k * kResT < nown) {
-        X acc = X(0);
-        if constexpr (RRES > 0)
-          if (k < RRES) {
-            const int kk = k < RRES ? k : 0;
-#pragma unroll
-            for (int m = 0; m < NZ2; ++m) {
-              asm volatile("" : "+v"(ai[kk][m]));   // keeps packed positions, not LDS addresses, in registers
-              const uint32_t q = ai[kk][m];
-              acc += av[kk][2 * m] * at_lds(rl, q & 0xffffu);
-              if (2 * m + 1 < NZ) acc += av[kk][2 * m + 1 < NZ ? 2 * m + 1 : 0] * at_lds(rl, q >> 16);
-            }
-          }
-        if (k >= RRES) {
-          const int rest = t + (k - RRES) * kResT;
-          if (rest < a.nl) {
-#pragma unroll
-            for (int m = 0; m < NZ2; ++m) {
-              const uint32_t q = lq[rest * QS + m];
-              acc += lv[rest * NZ + 2 * m] * at_lds(rl, q & 0xffffu);
-              if (2 * m + 1 < NZ) acc += lv[rest * NZ + 2 * m + 1] * at_lds(rl, q >> 16);
-            }
-          }
-        }
-        w[k] = acc;      // 0 on unused rows: their entries are 0
+      const int i = tt + k * kResT;
+      if (i < nown) {
+        const int32_t row = own[i], d = z.dofp ? z.dofp[row] : row;
+        const double un = (fresh ? 0.0 : z.u[d]) + z.sc[d] * (double)x[k];
+        z.u[d] = un;
+        ul[i] = un;
+        if (nb > 1) ll_put(ro, (uint32_t)i, un, ep);   // (dropped past the published rows)
       }
+      x[k] = X(0);
+      asm volatile("" ::: "memory");
     }
-    if (a.nb > 1) publish();
-    double g0 = 0.0, g1 = 0.0;
-#pragma unroll
-    for (int k = 0; k < RT; ++k)
-      if (k * kResT < nown) {
-        const X r = rl[il[k]];
-        g0 += (double)r * (double)r;
-        g1 += (double)r * (double)(first ? p[k] : w[k]);
+    fresh = false;
+    for (int h = tt; h < nh; h += kResT) {
+      const uint32_t at = (uint32_t)hl[h];
+      U4 q = {};
+      for (uint32_t spin = 0;; ++spin) {
+        asm volatile("" ::: "memory");
+        q = LL<double>::get(ru, at);
+        if (LL<double>::ok(q, ep)) break;
+        if (spin >= kSpinLimit) { gaveup = 1; break; }
       }
-    if (a.time) ticks += wall_clock64() - c0;
-    ++prods;
-    ok = exchange(g0, g1, true);
-    if (!ok) break;
-    if (first) {
-      // reseed: p made orthogonal to the new residual and extended, α = γ / p·ŝ
-      const bool keep = keep0 && g0 > 0.0;
-      gam = g0 > 0.0 ? g1 / g0 : 0.0;
-      rz = rz0 = g0;
-      const double conv = rr0 > 0.0 ? a.tol2 / rr0 : 0.0;
-      gstop = g0 * (a.hold2 > conv ? a.hold2 : conv);
-      const X be = (X)(keep ? g0 / rzp0 : 0.0), ga = (X)gam;
-      double none = 0.0;
-      pq = 0.0;
+      ul[nown + h] = LL<double>::val(q);
+    }
+    res_barrier();
+    const uint32_t* iz = z.ai + (int64_t)b * NZ2 * z.Rp;
+    const double* raw = z.raw + (int64_t)b * NZ * z.Rp;
+#pragma unroll
+    for (int k = 0; k < RT; ++k) {
+      const int i = tt + k * kResT;
+      w[k] = X(0);
+      if (i < nown) {
+        const int32_t row = own[i], d = z.dofp ? z.dofp[row] : row;
+        double acc = z.f[d];
+        if (z.raw) {
+#pragma unroll 3
+          for (int m = 0; m < NZ2; ++m) {
+            const uint32_t q = iz[(int64_t)m * z.Rp + i];
+            acc -= raw[(int64_t)(2 * m) * z.Rp + i] * ul[q & 0xffffu];
+            if (2 * m + 1 < NZ) acc -= raw[(int64_t)(2 * m + 1) * z.Rp + i] * ul[q >> 16];
+          }
+        } else {
+          const int32_t c0 = z.colptr[d], len = z.colptr[d + 1] - c0;
+#pragma unroll 1
+          for (int m = 0; m < len; ++m)
+            acc -= z.nzval[c0 + m] * ul[(iz[(int64_t)(m >> 1) * z.Rp + i] >> (16 * (m & 1))) & 0xffffu];
+        }
+        sum += acc * acc;
+        w[k] = (X)(z.sc[d] * acc);
+      }
+      asm volatile("" ::: "memory");         // one row's entries in flight
+    }
+    res_barrier();                           // u was read
+  };
+
+  double gstop = 0.0, prev = rrt, rzp0 = 0.0;   // rzp0: γ that the kept p belongs to, 0: p starts anew
+  long long ticks = 0;
+  int prods = 0, it = 0, handovers = 0, stall = 0, status = 0, done = 0, restart = 0;
+  bool first = true, ok = true;
+  for (;;) {
+    for (;;) {                    // a stretch of the recurrence
+      double g0 = 0.0, g1 = 0.0;
+      // w = Â r̂ on the block's rows; γ = r̂·r̂ and δ = r̂·w (in a reseed r̂·p instead)
+      const long long c0 = a.time ? wall_clock64() : 0;
 #pragma unroll
       for (int k = 0; k < RT; ++k) {
-        const X r = rl[il[k]];
-        p[k] = keep ? r + be * (p[k] - ga * r) : r;
-        sv[k] = keep ? w[k] + be * (sv[k] - ga * w[k]) : w[k];
-        pq += (double)p[k] * (double)sv[k];
+        w[k] = X(0);
+        if (k * kResT < nown) {
+          if constexpr (RRES > 0)
+            if (k < RRES) {
+              const int kk = k < RRES ? k : 0;
+              if constexpr (AHEAD) {
+#pragma unroll
+                for (int m = 0; m < NZ2; ++m)
+                  asm volatile("" : "+v"(ai[kk][m]));   // keeps packed positions, not LDS addresses, in registers
+                w[k] = gather_dot<X, NZ>(rl, av[kk], ai[kk]);
+              } else {
+                X acc = X(0);
+#pragma unroll
+                for (int m = 0; m < NZ2; ++m) {
+                  asm volatile("" : "+v"(ai[kk][m]));
+                  const uint32_t q = ai[kk][m];
+                  acc += av[kk][2 * m] * at_lds(rl, q & 0xffffu);
+                  if (2 * m + 1 < NZ) acc += av[kk][2 * m + 1 < NZ ? 2 * m + 1 : 0] * at_lds(rl, q >> 16);
+                }
+                w[k] = acc;
+              }
+            }
+          if (k >= RRES) {
+            const int rest = t + (k - RRES) * kResT;
+            if (rest < a.nl) {
+              X acc = X(0);
+#pragma unroll
+              for (int m = 0; m < NZ2; ++m) {
+                const uint32_t q = lq[rest * QS + m];
+                acc += lv[rest * NZ + 2 * m] * at_lds(rl, q & 0xffffu);
+                if (2 * m + 1 < NZ) acc += lv[rest * NZ + 2 * m + 1] * at_lds(rl, q >> 16);
+              }
+              w[k] = acc;
+            }
+          }
+        }                  // 0 on unused rows: their entries are 0
       }
-      for (int h = t; h < nh; h += kResT) sl[h] = keep ? wl[h] + be * (sl[h] - ga * wl[h]) : wl[h];
-      ok = exchange(pq, none, false);
+      if (a.time) ticks += wall_clock64() - c0;
+      ++prods;
+      if (nb > 1) publish();
+#pragma unroll
+      for (int k = 0; k < RT; ++k)
+        if (k * kResT < nown) {
+          const X r = rl[il[k]];
+          g0 += (double)r * (double)r;
+          g1 += (double)r * (double)(first ? p[k] : w[k]);
+        }
+      ok = exchange(g0, g1, true);
       if (!ok) break;
-      alpha = pq > 0.0 ? rz / pq : 0.0;
-      if (!(pq > 0.0)) {          // p vanished (r̂ already zero): nothing to step
-        done = restart = 1;
-        break;
+      if (first) {
+        // reseed: p made orthogonal to the new residual and extended, α = γ / p·ŝ
+        const bool keep = rzp0 > 0.0 && g0 > 0.0;
+        const double gam = g0 > 0.0 ? g1 / g0 : 0.0;
+        const double conv = rrt > 0.0 ? tol2 / rrt : 0.0;
+        gstop = uniform(g0 * (a.hold2 > conv ? a.hold2 : conv));
+        const X be = (X)(keep ? g0 / rzp0 : 0.0), ga = (X)gam;
+        double pq = 0.0, none = 0.0;
+#pragma unroll
+        for (int k = 0; k < RT; ++k) {
+          const X r = rl[il[k]];
+          p[k] = keep ? r + be * (p[k] - ga * r) : r;
+          sv[k] = keep ? w[k] + be * (sv[k] - ga * w[k]) : w[k];
+          pq += (double)p[k] * (double)sv[k];
+        }
+        for (int h = t; h < nh; h += kResT) sl[h] = keep ? wl[h] + be * (sl[h] - ga * wl[h]) : wl[h];
+        ok = exchange(pq, none, false);
+        if (!ok) break;
+        alpha = pq > 0.0 ? g0 / pq : 0.0;
+        if (!(pq > 0.0)) {          // p vanished (r̂ already zero): nothing to step
+          done = restart = 1;
+          break;
+        }
+        rzp = g0;                   // the first step moves x̂ and r̂ along the reseed's p, ŝ
       }
-      rzp = rz;                   // the first step moves x̂ and r̂ along the reseed's p, ŝ
-    } else {
-      const double be = g0 * irz;
-      const double den = g1 - g0 * g0 * ira;
-      const bool stop = g0 <= gstop;
-      const bool brk = !(rzp > 0.0) || !(alpha != 0.0) || !(den > 0.0);
-      rz = g0;
-      if (stop || brk) {          // hand over: x̂, p and ŝ of the last step
-        done = 1;
-        restart = stop ? 0 : 1;
-        break;
+      double be = 0.0;
+      if (!first) {
+        be = g0 * irz;
+        const double den = g1 - g0 * g0 * ira;
+        const bool stop = g0 <= gstop;
+        const bool brk = !(rzp > 0.0) || !(alpha != 0.0) || !(den > 0.0);
+        if (stop || brk || it >= a.lim) {   // hand over: x̂, p and ŝ of the last step
+          done = uniform(stop || brk ? 1 : 0);
+          restart = uniform(!stop && brk ? 1 : 0);
+          break;
+        }
+        alpha = g0 / den;
+        rzp = g0;
       }
-      if (it >= a.lim) break;
-      alpha = g0 / den;
-      beta = be;
-      rzp = g0;
+      ++it;
+      const X al = (X)alpha, bx = (X)be;
+#pragma unroll
+      for (int k = 0; k < RT; ++k)
+        if (k * kResT < nown) {
+          const X r = rl[il[k]];
+          if (!first) {
+            p[k] = r + bx * p[k];
+            sv[k] = w[k] + bx * sv[k];
+          }
+          x[k] += al * p[k];
+          rl[il[k]] = r - al * sv[k];
+        }
+      for (int base = t; base < nh; base += 4 * kResT) {   // four rows' LDS reads in flight
+        X sn[4], rn[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int h = base + k * kResT;
+          if (h < nh) {
+            sn[k] = first ? sl[h] : wl[h] + bx * sl[h];
+            rn[k] = rl[nown + h];
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const int h = base + k * kResT;
+          if (h < nh) {
+            sl[h] = sn[k];
+            rl[nown + h] = rn[k] - al * sn[k];
+          }
+        }
+      }
+      first = false;
+      res_barrier();
     }
-    ++it;
-    const X al = (X)alpha, be = (X)beta;
+    if (!ok) break;
+    double g0 = 0.0, none = 0.0;
+    true_residual(g0);
+    if (nb > 1) publish();
+    ok = exchange(g0, none, true);
+    if (!ok) break;
+    // the true residual: finished, or the next stretch starts from it
+    rrt = uniform(g0);
+    handovers += done;
+    status = uniform(rrt <= tol2 ? 1 : 0);
+    stall = uniform(rrt <= 0.81 * prev ? 0 : stall + 1);   // (a NaN stalls)
+    prev = uniform(fmin(prev, rrt));
+    if (status || it >= a.lim || stall >= kMaxStallRes) break;
 #pragma unroll
-    for (int k = 0; k < RT; ++k)
-      if (k * kResT < nown) {
-        const X r = rl[il[k]];
-        if (!first) {
-          p[k] = r + be * p[k];
-          sv[k] = w[k] + be * sv[k];
-        }
-        x[k] += al * p[k];
-        rl[il[k]] = r - al * sv[k];
-      }
-    for (int base = t; base < nh; base += 4 * kResT) {   // four rows' LDS reads in flight
-      X sn[4], rn[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int h = base + k * kResT;
-        if (h < nh) {
-          sn[k] = first ? sl[h] : wl[h] + be * sl[h];
-          rn[k] = rl[nown + h];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int h = base + k * kResT;
-        if (h < nh) {
-          sl[h] = sn[k];
-          rl[nown + h] = rn[k] - al * sn[k];
-        }
-      }
+    for (int k = 0; k < RT; ++k) {
+      const int i = t + k * kResT;
+      if (i < nown) rl[i] = w[k];
     }
-    first = false;
+    for (int h = t; h < nh; h += kResT) rl[nown + h] = wl[h];
+    if (t == 0) rl[zero] = X(0);
+    rzp0 = uniform(restart || !(rzp > 0.0) ? 0.0 : rzp);
+    first = true;
+    done = restart = 0;
     res_barrier();
   }
-  // the arguments read again: kept in scalar registers across the loop they would crowd it
   const ResArgs<X>& z = *reinterpret_cast<const ResArgs<X>*>(res_kernargs());
+  ResState* o = z.st + gr.x;
   if (!ok) {
-    if (t == 0) z.s->pad = 1;
+    if (t == 0) o->lost = 1;
     return;
   }
-#pragma unroll
-  for (int k = 0; k < RT; ++k) {
-    const int i = t + k * kResT;
-    if (i < nown) {
-      const int32_t row = z.orow[o0 + i];
-      z.p[row] = p[k];
-      z.sv[row] = sv[k];
-      const int32_t d = z.dofp ? z.dofp[row] : row;
-      if (d >= 0) z.u[d] += z.sc[d] * (double)x[k];
-    }
-  }
-  if (b == 0 && t == 0) {
-    Scal* o = z.s;                // all but pad, which a block that gave up sets
-    o->rz = rz;
-    o->rz0 = rz0;
-    o->rzp = rzp;
-    o->gstop = gstop;
-    o->alpha = alpha;
-    o->beta = beta;
-    o->gam = gam;
-    o->pq = pq;
-    o->done = done;
-    o->restart = restart;
-    o->fresh = 0;
-    o->pend = 0.0;
-    o->iters += it;
-    o->prods += prods;
-    o->prod_ticks += ticks;
+  if (b == b0 && t == 0) {
+    o->rr = rrt;
+    o->iters = it;
+    o->handovers = handovers;
+    o->status = status;
+    o->prods = prods;
+    o->ticks = ticks;
+    o->begin = begin;
+    o->end = wall_clock64();
+    o->epoch = ep;
   }
 }
 
@@ -844,11 +986,13 @@ static const void* res_kernel(int nz, int R) {
   return nullptr;
 }
 
-// LDS of a block with nl rows' entries in it: r̂ (and a zero slot), ŝ, w and the slots of the
-// coupled rows, the entries
+// Elements of r̂ in LDS: its rows and a zero slot, or their u in FP64.
+static int res_lds_r(const ResOp* o, size_t xb) { return xb == 4 ? 2 * o->nlocmax + 2 : o->nlocmax + 1; }
+
+// LDS of a block with nl rows' entries in it: r̂, ŝ, w and the slots of the coupled rows, the entries
 static size_t res_lds_bytes(const ResOp* o, size_t xb, int nl) {
   const size_t nz2 = (size_t)((o->nz + 1) / 2 | 1);
-  return ((size_t)o->nlocmax + 1 + 2 * (size_t)o->nhmax + (size_t)o->nz * nl) * xb + 4 * (nz2 * nl + (size_t)o->nhmax);
+  return ((size_t)res_lds_r(o, xb) + 2 * (size_t)o->nhmax + (size_t)o->nz * nl) * xb + 4 * (nz2 * nl + (size_t)o->nhmax);
 }
 
 // Register rows of the instantiated kernels (kResT threads).
@@ -861,7 +1005,7 @@ static int res_register_rows(int nz, bool fp32) {
 // kResT rows of the largest part begun (more where their entries are in LDS), its coupled rows,
 // and every part's record read by all; parts too large for FP64 values only where nothing else
 // is left.
-static void res_triple(const double* ext, int dim, double per, int nz, int most, int* out) {
+static double res_triple(const double* ext, int dim, double per, int nz, int most, int* out) {
   double best = 1e300;
   const double regs = kResT * (nz == 9 ? 4 : nz == 18 ? 3 : 2), cap = nz == 27 ? regs + 360.0 : regs;
   for (int x = 1; x <= most; ++x)
@@ -886,6 +1030,52 @@ static void res_triple(const double* ext, int dim, double per, int nz, int most,
         }
       }
     }
+  return best;
+}
+
+// Blocks per system, at most `total` of them: each the fewest that hold its rows, the others one by
+// one to the system that is expected to take longest (its extent in rows, times an iteration's
+// cost) as long as it gains.  cut: [ng][3].  false: they do not fit.
+struct ResExtent {
+  double ext[3], per, count;
+  int dim;
+};
+static bool res_share(const std::vector<ResExtent>& e, int nz, int total, int most_rows, std::vector<int>* cut) {
+  const int ng = (int)e.size();
+  std::vector<int> m(ng), cap(ng);
+  std::vector<double> cost(ng), its(ng);
+  cut->assign(3 * ng, 1);
+  int used = 0;
+  for (int i = 0; i < ng; ++i) {
+    cap[i] = (int)std::max<double>(1.0, std::min<double>(total, std::ceil(e[i].count / kResRows)));
+    m[i] = (int)std::max<double>(1.0, std::ceil(e[i].count / (ng > 1 ? 0.85 * most_rows : most_rows)));
+    if (m[i] > cap[i]) return false;
+    if (ng == 1) m[i] = cap[i];
+    its[i] = e[i].ext[0] + e[i].ext[1] + e[i].ext[2];
+    used += m[i];
+  }
+  if (used > total) return false;
+  for (int i = 0; i < ng; ++i) cost[i] = res_triple(e[i].ext, e[i].dim, e[i].per, nz, m[i], &(*cut)[3 * i]);
+  std::vector<bool> last(ng, false);
+  for (;;) {
+    int at = -1;
+    for (int i = 0; i < ng; ++i)
+      if (!last[i] && (at < 0 || its[i] * cost[i] > its[at] * cost[at])) at = i;
+    if (at < 0) return true;
+    bool better = false;
+    for (int k = m[at] + 1; k <= std::min(cap[at], m[at] + total - used) && !better; ++k) {
+      int c3[3] = {1, 1, 1};
+      const double v = res_triple(e[at].ext, e[at].dim, e[at].per, nz, k, c3);
+      if (v < cost[at]) {
+        used += k - m[at];
+        m[at] = k;
+        cost[at] = v;
+        for (int d = 0; d < 3; ++d) (*cut)[3 * at + d] = c3[d];
+        better = true;
+      }
+    }
+    if (!better) last[at] = true;
+  }
 }
 
 static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& rows, int nz, int most_rows) {
@@ -894,31 +1084,41 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   (void)hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device);
   (void)hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device);
   const int64_t n = rows.n;
+  const int ng = s.nsys > 0 ? s.nsys : 1;
   o->state = -1;
-  o->n = n;
   o->nz = nz;
-  const int words = (int)((n + 31) / 32), ng = (words + 7) / 8;
-  const int lds = 4 * (words + ng);
+  o->ng = ng;
+  std::vector<ResSystem> sys(ng);
+  int64_t longest = 0;
+  for (int i = 0; i < ng; ++i) {
+    sys[i] = ResSystem{s.nsys > 0 ? s.sys[2 * i] : 0, s.nsys > 0 ? s.sys[2 * i + 1] : (int32_t)n, {}, {}};
+    longest = std::max<int64_t>(longest, sys[i].row1 - sys[i].row0);
+  }
+  const int words = (int)((longest + 31) / 32);
+  const int lds = 4 * (words + (words + 7) / 8);
   if (lds > maxlds - 1024) return FEM_OK;   // a bitmap of the rows (more than a million): far too many anyway
 
   struct Scratch {                          // freed on every way out
     int32_t *node = nullptr, *part = nullptr, *hist = nullptr, *size = nullptr, *rank = nullptr, *cnt = nullptr;
+    int4* slab = nullptr;
+    ResSystem* sys = nullptr;
     uint8_t* flag = nullptr;
     double* geom = nullptr;
     ~Scratch() {
       dev_free(&node); dev_free(&part); dev_free(&hist); dev_free(&size); dev_free(&rank); dev_free(&cnt);
-      dev_free(&flag); dev_free(&geom);
+      dev_free(&slab); dev_free(&sys); dev_free(&flag); dev_free(&geom);
     }
   } w;
   int rc;
   ResPos g{};
   g.src = s.src;
-  g.n = n;
   g.px = s.px;
   g.pxy = s.pxy;
   g.dofp = s.dofp;
-  g.dim = s.src ? s.dim : c->sdim;
-  if (s.src == 0) {   // a node of each dof's first cell (its own node for a Q1 field)
+  g.dim = s.dim;
+  g.node = s.node;
+  for (int d = 0; d < 3; ++d) g.x[d] = s.x[d];
+  if (s.src == 0 && !s.node) {   // a node of each dof's first cell (its own node for a Q1 field)
     const int64_t nc = c->ncells, nd = c->ndpc, npc = c->npc;
     if (nd <= 0 || npc <= 0 || (int64_t)c->h_cell_dofs.size() != nc * nd || (int64_t)c->h_cell_nodes.size() != nc * npc)
       return FEM_OK;
@@ -936,48 +1136,78 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
     if ((rc = dev_alloc(c, &w.node, n))) return rc;
     FEM_HIP(c, hipMemcpy(w.node, node.data(), 4 * n, hipMemcpyHostToDevice));
     g.node = w.node;
+    g.dim = c->sdim;
     for (int d = 0; d < 3; ++d) g.x[d] = c->d_x[d];
   }
-  double geom[10];
-  if ((rc = dev_alloc(c, &w.geom, 10))) return rc;
-  k_res_geom<<<1, 1024, 0, c->stream>>>(g, rows, nz, w.geom);
+  std::vector<double> geom(10 * ng);
+  if ((rc = dev_alloc(c, &w.geom, 10 * ng)) || (rc = dev_alloc(c, &w.sys, ng))) return rc;
+  FEM_HIP(c, hipMemcpyAsync(w.sys, sys.data(), sizeof(ResSystem) * ng, hipMemcpyHostToDevice, c->stream));
+  k_res_geom<<<ng, 1024, 0, c->stream>>>(g, rows, w.sys, nz, w.geom);
   FEM_HIP(c, hipGetLastError());
-  FEM_HIP(c, hipMemcpyAsync(geom, w.geom, sizeof geom, hipMemcpyDeviceToHost, c->stream));
+  FEM_HIP(c, hipMemcpyAsync(geom.data(), w.geom, sizeof(double) * 10 * ng, hipMemcpyDeviceToHost, c->stream));
   FEM_HIP(c, hipStreamSynchronize(c->stream));
-  const double count = geom[9];
-  double ext[3] = {1.0, 1.0, 1.0}, cells = 1.0;
-  for (int d = 0; d < 3; ++d) {
-    const double len = geom[3 + d] - geom[d];
-    const bool flat = d >= g.dim || !(len > 0.0);
-    g.lo[d] = geom[d];
-    g.inv[d] = flat ? 0.0 : (kResBins - 0.5) / len;
-    if (!flat && geom[6 + d] > 0.0) ext[d] = std::max(1.0, std::floor(len / geom[6 + d] + 1.5));
-    cells *= ext[d];
+  std::vector<ResExtent> ext(ng);
+  for (int i = 0; i < ng; ++i) {
+    const double* e = &geom[10 * i];
+    double cells = 1.0;
+    for (int d = 0; d < 3; ++d) {
+      const double len = e[3 + d] - e[d];
+      const bool flat = d >= g.dim || !(len > 0.0);
+      sys[i].lo[d] = e[d];
+      sys[i].inv[d] = flat ? 0.0 : (kResBins - 0.5) / len;
+      ext[i].ext[d] = !flat && e[6 + d] > 0.0 ? std::max(1.0, std::floor(len / e[6 + d] + 1.5)) : 1.0;
+      cells *= ext[i].ext[d];
+    }
+    ext[i].count = e[9];
+    ext[i].per = e[9] / cells;
+    ext[i].dim = g.dim;
   }
-  const int most = (int)std::max<double>(
-      1.0, std::min<double>(std::min(ncu, kResMaxBlocks), std::ceil(count / kResRows)));
-  if ((most > 1 && !coop) || count > (double)most * most_rows) return FEM_OK;
-  int cut[3] = {1, 1, 1};
-  res_triple(ext, g.dim, count / cells, nz, most, cut);
-  const int nb = cut[0] * cut[1] * cut[2];
+  std::vector<int> cut;
+  if (!res_share(ext, nz, std::min(ncu, kResMaxBlocks), most_rows, &cut)) return FEM_OK;
+  int nb = 0;
+  std::vector<int4> grp;
+  for (int i = 0; i < ng; ++i) {
+    const int m = cut[3 * i] * cut[3 * i + 1] * cut[3 * i + 2];
+    for (int k = 0; k < m; ++k) grp.push_back(make_int4(i, nb, m, 0));
+    if (m > 1 && !coop) return FEM_OK;
+    nb += m;
+  }
   o->nb = nb;
   const int grid = (int)std::min<int64_t>(2048, (n + 255) / 256);
+  const int gridy = (int)std::max<int64_t>(1, std::min<int64_t>(2048 / ng, (longest + 255) / 256));
   if ((rc = dev_alloc(c, &w.part, n)) || (rc = dev_alloc(c, &w.hist, (size_t)kResBins * nb)) ||
       (rc = dev_alloc(c, &w.flag, n)) || (rc = dev_alloc(c, &w.size, 2 * nb)) || (rc = dev_alloc(c, &w.rank, n)) ||
-      (rc = dev_alloc(c, &w.cnt, nb)) || (rc = dev_alloc(c, &o->oofs, nb + 1)) ||
-      (rc = dev_alloc(c, &o->pofs, nb + 1)) || (rc = dev_alloc(c, &o->hoff, nb + 1)))
+      (rc = dev_alloc(c, &w.cnt, nb)) || (rc = dev_alloc(c, &w.slab, nb)) || (rc = dev_alloc(c, &o->grp, nb)) ||
+      (rc = dev_alloc(c, &o->oofs, nb + 1)) || (rc = dev_alloc(c, &o->pofs, nb + 1)) ||
+      (rc = dev_alloc(c, &o->hoff, nb + 1)))
     return rc;
-  FEM_HIP(c, hipMemsetAsync(w.part, 0, 4 * n, c->stream));
+  FEM_HIP(c, hipMemcpyAsync(w.sys, sys.data(), sizeof(ResSystem) * ng, hipMemcpyHostToDevice, c->stream));
+  FEM_HIP(c, hipMemcpyAsync(o->grp, grp.data(), sizeof(int4) * nb, hipMemcpyHostToDevice, c->stream));
+  FEM_HIP(c, hipMemsetAsync(w.part, 0xff, 4 * n, c->stream));
   FEM_HIP(c, hipMemsetAsync(w.flag, 0, n, c->stream));
   FEM_HIP(c, hipMemsetAsync(w.size, 0, 8 * nb, c->stream));
-  int slabs = 1;
+  k_res_start<<<dim3(gridy, ng), 256, 0, c->stream>>>(g, w.sys, w.part);
+  std::vector<int> per(ng, 1);              // slabs of each system so far
   for (int d = 0; d < 3; ++d) {
-    if (cut[d] == 1 && !(d == 2)) continue;   // the last level also marks the rows without a place
-    FEM_HIP(c, hipMemsetAsync(w.hist, 0, (size_t)4 * kResBins * slabs, c->stream));
-    k_res_hist<<<grid, 256, 0, c->stream>>>(g, d, w.part, w.hist);
-    k_res_cut<<<slabs, 256, 0, c->stream>>>(cut[d], w.hist);
-    k_res_split<<<grid, 256, 0, c->stream>>>(g, d, cut[d], w.hist, w.part);
-    slabs *= cut[d];
+    std::vector<int4> slab;
+    int next = 0;
+    bool any = false;
+    for (int i = 0; i < ng; ++i) {
+      any = any || cut[3 * i + d] > 1;
+      for (int k = 0; k < per[i]; ++k) {
+        slab.push_back(make_int4(i, cut[3 * i + d], next, 0));
+        next += cut[3 * i + d];
+      }
+    }
+    if (!any) continue;
+    for (int i = 0; i < ng; ++i) per[i] *= cut[3 * i + d];
+    const int ns = (int)slab.size();
+    FEM_HIP(c, hipMemcpyAsync(w.slab, slab.data(), sizeof(int4) * ns, hipMemcpyHostToDevice, c->stream));
+    FEM_HIP(c, hipMemsetAsync(w.hist, 0, (size_t)4 * kResBins * ns, c->stream));
+    k_res_hist<<<grid, 256, 0, c->stream>>>(g, w.sys, w.slab, n, d, w.part, w.hist);
+    k_res_cut<<<ns, 256, 0, c->stream>>>(w.slab, w.hist);
+    k_res_split<<<grid, 256, 0, c->stream>>>(g, w.sys, w.slab, n, d, w.hist, w.part);
+    FEM_HIP(c, hipStreamSynchronize(c->stream));   // slab goes
   }
   k_res_shared<<<grid, 256, 0, c->stream>>>(rows, nz, w.part, w.flag, w.size);
   FEM_HIP(c, hipGetLastError());
@@ -1005,7 +1235,7 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   o->nslots = pub[nb];
   (void)hipFuncSetAttribute((const void*)k_res_count, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * words);
   (void)hipFuncSetAttribute((const void*)k_res_fill, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-  k_res_count<<<nb, 256, 4 * words, c->stream>>>(rows, nz, w.part, o->oofs, o->orow, w.cnt);
+  k_res_count<<<nb, 256, 4 * words, c->stream>>>(rows, nz, words, w.sys, o->grp, w.part, o->oofs, o->orow, w.cnt);
   FEM_HIP(c, hipGetLastError());
   FEM_HIP(c, hipMemcpyAsync(h.data(), w.cnt, 4 * nb, hipMemcpyDeviceToHost, c->stream));
   FEM_HIP(c, hipStreamSynchronize(c->stream));
@@ -1020,14 +1250,16 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   const int nz2 = (nz + 1) / 2;
   if ((rc = dev_alloc(c, &o->hrow, hof[nb])) || (rc = dev_alloc(c, &o->hslot, hof[nb])) ||
       (rc = dev_alloc(c, &o->ai, (size_t)nb * nz2 * o->Rp)) || (rc = dev_alloc(c, &o->wx, (size_t)8 * o->nslots)) ||
-      (rc = dev_alloc(c, &o->rec, kRecWords)))
+      (rc = dev_alloc(c, &o->wu, (size_t)4 * o->nslots)) || (rc = dev_alloc(c, &o->rec, kRecWords)))
     return rc;
   FEM_HIP(c, hipMemcpyAsync(o->pofs, pub.data(), 4 * (nb + 1), hipMemcpyHostToDevice, c->stream));
   FEM_HIP(c, hipMemcpyAsync(o->hoff, hof.data(), 4 * (nb + 1), hipMemcpyHostToDevice, c->stream));
   FEM_HIP(c, hipMemsetAsync(o->wx, 0, (size_t)32 * o->nslots, c->stream));
+  FEM_HIP(c, hipMemsetAsync(o->wu, 0, (size_t)16 * o->nslots, c->stream));
   FEM_HIP(c, hipMemsetAsync(o->rec, 0, 4 * kRecWords, c->stream));
-  k_res_fill<<<nb, 256, lds, c->stream>>>(rows, nz, o->Rp, w.part, w.rank, o->oofs, o->orow, o->pofs, o->hoff, o->hrow,
-                                          o->hslot, o->ai);
+  FEM_HIP(c, hipHostMalloc((void**)&o->st, sizeof(ResState) * ng, hipHostMallocDefault));
+  k_res_fill<<<nb, 256, lds, c->stream>>>(rows, nz, o->Rp, words, w.sys, o->grp, w.part, w.rank, o->oofs, o->orow,
+                                          o->pofs, o->hoff, o->hrow, o->hslot, o->ai);
   FEM_HIP(c, hipGetLastError());
   FEM_HIP(c, hipStreamSynchronize(c->stream));   // host vectors and scratch go
   o->epoch = 0;
@@ -1049,12 +1281,12 @@ int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* s
   if (!*op) *op = new ResOp();
   ResOp* o = *op;
   if (o->state == -1) return FEM_OK;
-  ResRows rows{s.src, s.dim, s.n, s.npad, s.px, s.pxy, c->d_colptr, c->d_rowval, s.dofp, c->d_nzval, sc, s.kc, s.val,
+  ResRows rows{s.src, s.dim, s.n, s.npad, s.px, s.pxy, c->d_colptr, c->d_rowval, s.dofp, s.map, c->d_nzval, sc, s.kc, s.val,
                s.t, {}};
   for (int i = 0; i < 8; ++i) rows.f[i] = s.f[i];
   int rc;
   if (o->state == 0) {
-    const int widest = s.src == 0 ? c->max_row_nnz : s.dim == 3 ? 27 : 9;
+    const int widest = s.widest;
     const int nz = widest <= 9 ? 9 : widest <= 18 ? 18 : 27, most = res_most_rows(nz, fp32);
     // clearly too large in this precision (lattice rows include some padding): nothing is built
     if (widest > 27 || s.n < 1 || s.n > (int64_t)kResMaxBlocks * most * 5 / 4) return FEM_OK;
@@ -1069,13 +1301,15 @@ int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* s
     return FEM_OK;
   const int pi = fp32 ? 0 : 1;
   const size_t len = (size_t)o->nb * o->nz * o->Rp;
-  if (fp32 && !o->val32 && (rc = dev_alloc(c, &o->val32, len))) return rc;
+  if (fp32 && !o->val32 && ((rc = dev_alloc(c, &o->val32, len)) || (rc = dev_alloc(c, &o->raw, len)))) return rc;
   if (!fp32 && !o->val64 && (rc = dev_alloc(c, &o->val64, len))) return rc;
   if (o->ver[pi] != c->nzval_version + 1 || o->aux[pi] != c->aux_version + 1 || o->jac[pi] != jacobi ||
       o->vsrc[pi] != s.src) {
     const int g = (int)std::min<int64_t>(8192, ((int64_t)o->nb * o->Rp + 255) / 256);
-    if (fp32) k_res_vals<float><<<g, 256, 0, c->stream>>>(rows, o->nz, o->Rp, o->nb, o->oofs, o->orow, o->val32);
-    else k_res_vals<double><<<g, 256, 0, c->stream>>>(rows, o->nz, o->Rp, o->nb, o->oofs, o->orow, o->val64);
+    if (fp32) k_res_vals<float><<<g, 256, 0, c->stream>>>(rows, o->nz, o->Rp, o->nb, o->oofs, o->orow, o->val32,
+                                                        o->raw);
+    else k_res_vals<double><<<g, 256, 0, c->stream>>>(rows, o->nz, o->Rp, o->nb, o->oofs, o->orow, o->val64,
+                                                    nullptr);
     FEM_HIP(c, hipGetLastError());
     o->ver[pi] = c->nzval_version + 1;
     o->aux[pi] = c->aux_version + 1;
@@ -1087,40 +1321,78 @@ int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* s
 }
 
 template <typename X>
-int resident_run(fem_ctx* c, ResOp* o, const double* res, const double* sc, X* p, X* sv, double* u, Scal* s,
-                 const int32_t* dofp, double hold_factor2, double tol2, int restart, int lim, bool* launched) {
+int resident_run(fem_ctx* c, ResOp* o, const ResSource& s, const double* sc, const double* f, double* u,
+                 const double* in, double bnorm2, double tol2, double hold_factor2, int lim, const ResState** out,
+                 bool* launched) {
   *launched = false;
-  // exchange numbers: one per product and one more per reseed; started over long before 2³²
-  const uint32_t need = (uint32_t)lim + 8u;
-  if (o->epoch > 0xf0000000u - need) {
+  // exchange numbers: one per product and two more per hand-over, of which seven in a row may
+  // do without a product; started over before lim of those could reach 2³²
+  lim = std::min(lim, 1 << 25);
+  if (o->epoch > 0xffffffffu - 32u * (uint32_t)lim - 64u) {
     FEM_HIP(c, hipMemsetAsync(o->wx, 0, (size_t)32 * o->nslots, c->stream));
+    FEM_HIP(c, hipMemsetAsync(o->wu, 0, (size_t)16 * o->nslots, c->stream));
     FEM_HIP(c, hipMemsetAsync(o->rec, 0, 4 * kRecWords, c->stream));
     o->epoch = 0;
   }
   int maxlds = 0;
   FEM_HIP(c, hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
-  const int nl = res_lds_rows(o, sizeof(X) == 4, maxlds);
-  ResArgs<X> a{o->Rp, o->nb, o->nslots, nl, o->nlocmax + 1, o->nhmax, o->oofs, o->orow, o->pofs, o->hoff, o->hrow,
-               o->hslot, o->ai,
-               sizeof(X) == 4 ? reinterpret_cast<const X*>(o->val32) : reinterpret_cast<const X*>(o->val64),
-               dofp, res, sc, p, sv, u, s, o->wx, o->rec, hold_factor2, tol2, o->epoch + 1u, restart, lim,
-               c->tune.time_kernels};
-  o->epoch += need;
+  constexpr bool fp32 = sizeof(X) == 4;
+  const int nl = res_lds_rows(o, fp32, maxlds);
+  ResArgs<X> a{};
+  a.Rp = o->Rp;
+  a.nslots = o->nslots;
+  a.nl = nl;
+  a.rl0 = res_lds_r(o, sizeof(X));
+  a.nhmax = o->nhmax;
+  a.grp = o->grp;
+  a.oofs = o->oofs;
+  a.orow = o->orow;
+  a.pofs = o->pofs;
+  a.hoff = o->hoff;
+  a.hrow = o->hrow;
+  a.hslot = o->hslot;
+  a.ai = o->ai;
+  a.val = fp32 ? reinterpret_cast<const X*>(o->val32) : reinterpret_cast<const X*>(o->val64);
+  a.raw = fp32 ? o->raw : nullptr;
+  a.colptr = c->d_colptr;
+  a.nzval = c->d_nzval;
+  a.dofp = s.dofp;
+  a.f = f;
+  a.sc = sc;
+  a.u = u;
+  a.in = in;
+  a.st = o->st;
+  a.wx = o->wx;
+  a.wu = o->wu;
+  a.rec = o->rec;
+  a.in0[0] = bnorm2;
+  a.in0[1] = tol2;
+  a.hold2 = hold_factor2;
+  a.epoch = o->epoch + 1u;
+  a.lim = lim;
+  a.time = c->tune.time_kernels;
+  std::fill(o->st, o->st + o->ng, ResState{});
   const void* k = res_kernel<X>(o->nz, o->Rmax);
   const size_t lds = res_lds_bytes(o, sizeof(X), nl);
   FEM_HIP(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   void* args[] = {&a};
-  const hipError_t e = o->nb == 1 ? hipLaunchKernel(k, dim3(1), dim3(kResT), args, lds, c->stream)
-                                  : hipLaunchCooperativeKernel(k, dim3(o->nb), dim3(kResT), args, (unsigned)lds,
-                                                               c->stream);
-  *launched = e == hipSuccess;
-  if (e != hipSuccess) (void)hipGetLastError();   // not as many blocks at once as the device should hold
+  const hipError_t e = o->nb == o->ng ? hipLaunchKernel(k, dim3(o->nb), dim3(kResT), args, lds, c->stream)
+                                      : hipLaunchCooperativeKernel(k, dim3(o->nb), dim3(kResT), args, (unsigned)lds,
+                                                                   c->stream);
+  if (e != hipSuccess) {   // not as many blocks at once as the device should hold
+    (void)hipGetLastError();
+    return FEM_OK;
+  }
+  *launched = true;
+  FEM_HIP(c, hipStreamSynchronize(c->stream));
+  for (int i = 0; i < o->ng; ++i) o->epoch = std::max(o->epoch, o->st[i].epoch);
+  *out = o->st;
   return FEM_OK;
 }
 
-template int resident_run<float>(fem_ctx*, ResOp*, const double*, const double*, float*, float*, double*, Scal*,
-                                 const int32_t*, double, double, int, int, bool*);
-template int resident_run<double>(fem_ctx*, ResOp*, const double*, const double*, double*, double*, double*, Scal*,
-                                  const int32_t*, double, double, int, int, bool*);
+template int resident_run<float>(fem_ctx*, ResOp*, const ResSource&, const double*, const double*, double*,
+                                 const double*, double, double, double, int, const ResState**, bool*);
+template int resident_run<double>(fem_ctx*, ResOp*, const ResSource&, const double*, const double*, double*,
+                                  const double*, double, double, double, int, const ResState**, bool*);
 
 }  // namespace fem

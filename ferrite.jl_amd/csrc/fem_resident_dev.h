@@ -70,6 +70,13 @@ __device__ __forceinline__ double wave_sum63(double v) {
   return v;
 }
 
+// A value all lanes hold, in scalar registers.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double uniform(double v) {
+  const long long b = __double_as_longlong(v);
+  return __longlong_as_double(((long long)uniform((int)(b >> 32)) << 32) | (unsigned int)uniform((int)b));
+}
+
 // Element of an LDS array at a byte offset.
 template <typename X>
 __device__ __forceinline__ X at_lds(const X* base, uint32_t boff) {

@@ -170,6 +170,7 @@ struct SolverWork {
   int elem_grid = 0;
   ResOp *res_csc = nullptr, *res_lat = nullptr;   // resident CG on K's rows, on the lattice's rows
   ResOp* res_op = nullptr;     // the one the current solve runs on, or null
+  ResSource res_src;           // and where its rows come from
   BrickOp* bricks = nullptr;   // resident CG on the 3D cell form
   bool use_bricks = false;     // the current solve runs on it
   bool res_off = false;        // a resident launch was not taken or gave up: not tried again
@@ -2334,12 +2335,14 @@ static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv, 
     ResSource s;
     s.src = w->use_cells ? 2 : w->use_lat ? 1 : 0;
     s.n = *nv;
+    s.widest = c->max_row_nnz;
     if (w->use_lat) {
       s.dim = l.ns == 14 ? 3 : 2;
       s.px = (int32_t)l.px;
       s.pxy = (int32_t)l.pxy;
       s.npad = l.npad;
       s.dofp = l.dofp;
+      s.map = l.map;
       s.val = sizeof(X) == 4 ? (const void*)l.val32 : (const void*)l.val64;
       s.kc = cl.kc64;
       s.t = sizeof(X) == 4 ? (const void*)cl.t32 : (const void*)cl.t64;
@@ -2350,6 +2353,7 @@ static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv, 
     if ((rc = resident_prepare(c, op, s, w->sc, jacobi, sizeof(X) == 4, &ok))) return rc;
     if (ok) {
       w->res_op = *op;
+      w->res_src = s;
       return FEM_OK;
     }
     if (sizeof(X) == 4 && w->use_cells && cl.dim == 3) {
@@ -2547,9 +2551,15 @@ static int batch_index(const Scal& h, int it) {
   return m >= 5.0 * kBatchMin ? 2 : m >= 2.5 * kBatchMin ? 1 : 0;
 }
 
+struct CgResult {
+  int iters = 0, handovers = 0;
+  double ms = 0.0;
+  double rr = 0.0;         // square of the true residual of the returned u
+};
+
 template <typename X>
 static int cg_run(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double bnorm2, double tol2, double hold_factor2,
-                  int maxit, GraphCache* gcs, int* iters, int* handovers, double* ms) {
+                  int maxit, GraphCache* gcs, CgResult* out) {
   zero_vec<double>(c, c->d_u, c->n);
   // all five: the lattice numbering's padding entries must start (and so stay) zero
   for (X* a : {v.x, v.r, v.w, v.p, v.sv}) zero_vec<X>(c, a, v.n);
@@ -2603,25 +2613,53 @@ static int cg_run(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double bnorm2, 
   }
   FEM_HIP(c, hipEventRecord(c->ev1, c->stream));
   FEM_HIP(c, hipGetLastError());
-  *ms += event_ms(c);
+  out->ms += event_ms(c);
   Scal h{};
   if ((rc = read_scal(c, w, &h))) return rc;
-  *iters = h.iters;
-  *handovers = nho;
+  out->iters = h.iters;
+  out->handovers = nho;
+  out->rr = h.rr;
   return converged ? FEM_OK : FEM_ERR_NOCONV;
 }
 
-// The same with the resident CG: one launch per stretch (reseed, iterations, fold into u), then
-// the FP64 residual, and one read of the record by the host.  *gave_up: the device did not take a
-// launch, or one stopped waiting for its blocks (nothing of it was folded); the caller starts over
-// with the separate kernels.
+// The same with the resident CG on the rows' entries: one launch.  *gave_up: the device did not
+// take it, or it stopped waiting for its blocks; the caller starts over with the separate kernels.
 template <typename X>
-static int cg_run_resident(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double bnorm2, double tol2,
-                           double hold_factor2, int maxit, int* iters, int* handovers, double* ms, bool* gave_up) {
+static int cg_run_rows(fem_ctx* c, SolverWork* w, double bnorm2, double tol2, double hold_factor2, int maxit,
+                       CgResult* out, bool* gave_up) {
+  const int64_t most = ((int64_t)maxit + kBatch - 1) / kBatch * kBatch;   // as the batches round it up
+  const ResState* st = nullptr;
+  bool launched = false;
+  FEM_HIP(c, hipEventRecord(c->ev0, c->stream));
+  int rc = resident_run<X>(c, w->res_op, w->res_src, w->sc, c->d_f, c->d_u, nullptr, bnorm2, tol2, hold_factor2,
+                           (int)std::min<int64_t>(1 << 24, most), &st, &launched);
+  if (rc) return rc;
+  if (!launched || st->lost) {
+    *gave_up = true;
+    return FEM_OK;
+  }
+  FEM_HIP(c, hipEventRecord(c->ev1, c->stream));
+  out->ms += event_ms(c);
+  if (c->tune.time_kernels) {   // 100 MHz clock
+    c->timings.spmv_ms += 1e-5 * (double)st->ticks;
+    c->timings.spmv_launches += st->prods;
+  }
+  out->iters = st->iters;
+  out->handovers = st->handovers;
+  out->rr = st->rr;
+  return st->status ? FEM_OK : FEM_ERR_NOCONV;
+}
+
+// The same on bricks of the cell form: one launch per stretch (reseed, iterations, fold into u),
+// then the FP64 residual, and one read of the record by the host.
+static int cg_run_bricks(fem_ctx* c, SolverWork* w, const CgVecs<float>& v, double bnorm2, double tol2,
+                         double hold_factor2, int maxit, CgResult* out, bool* gave_up) {
   zero_vec<double>(c, c->d_u, c->n);
   k_cg_init_scal<<<1, 1, 0, c->stream>>>(w->s, bnorm2);
-  const int64_t most = ((int64_t)maxit + kBatch - 1) / kBatch * kBatch;   // as the batches round it up
-  const int32_t* dofp = w->use_lat ? w->lat.dofp : nullptr;
+  const int64_t most = ((int64_t)maxit + kBatch - 1) / kBatch * kBatch;
+  const LatOp& l = w->lat;
+  BrickSource b{(int32_t)l.px, (int32_t)l.pxy, w->cells.t32, w->cells.kc32, l.dofp, {}};
+  for (int i = 0; i < 8; ++i) b.f[i] = w->cells.f[i];
   const double* res = c->d_f;
   int rc = FEM_OK, nho = 0, stall = 0;
   bool converged = false;
@@ -2632,18 +2670,7 @@ static int cg_run_resident(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double
     const int lim = (int)std::min<int64_t>(1 << 24, most - h.iters);
     const int restart = res == c->d_f ? 1 : 0;
     bool launched = false;
-    if (w->use_bricks) {
-      if constexpr (sizeof(X) == 4) {
-        const LatOp& l = w->lat;
-        BrickSource b{(int32_t)l.px, (int32_t)l.pxy, w->cells.t32, w->cells.kc32, l.dofp, {}};
-        for (int i = 0; i < 8; ++i) b.f[i] = w->cells.f[i];
-        rc = brick_run(c, w->bricks, b, res, w->sc, v.p, v.sv, c->d_u, w->s, hold_factor2, tol2, restart, lim,
-                       &launched);
-      }
-    } else {
-      rc = resident_run<X>(c, w->res_op, res, w->sc, v.p, v.sv, c->d_u, w->s, dofp, hold_factor2, tol2, restart, lim,
-                           &launched);
-    }
+    rc = brick_run(c, w->bricks, b, res, w->sc, v.p, v.sv, c->d_u, w->s, hold_factor2, tol2, restart, lim, &launched);
     if (rc) return rc;
     if (!launched) {
       *gave_up = true;
@@ -2659,26 +2686,27 @@ static int cg_run_resident(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double
     if (h.done) ++nho;
     if (h.rr <= tol2) { converged = true; break; }
     if (h.iters >= most) break;
-    stall = h.rr > 0.81 * prev_true ? stall + 1 : 0;
+    stall = h.rr <= 0.81 * prev_true ? 0 : stall + 1;   // (a NaN stalls)
     if (stall >= kMaxStall) break;
     prev_true = std::min(prev_true, h.rr);
     res = w->res;
   }
   FEM_HIP(c, hipEventRecord(c->ev1, c->stream));
-  *ms += event_ms(c);
+  out->ms += event_ms(c);
   if (c->tune.time_kernels) {   // 100 MHz clock
     c->timings.spmv_ms += 1e-5 * (double)h.prod_ticks;
     c->timings.spmv_launches += h.prods;
   }
-  *iters = h.iters;
-  *handovers = nho;
+  out->iters = h.iters;
+  out->handovers = nho;
+  out->rr = h.rr;
   return converged ? FEM_OK : FEM_ERR_NOCONV;
 }
 
 // The solve in X precision on whichever form prepare_operator chose.
 template <typename X>
 static int cg_solve(fem_ctx* c, SolverWork* w, int jacobi, double bnorm2, double tol2, double hold_factor2, int maxit,
-                    int* iters, int* handovers, double* ms) {
+                    CgResult* out) {
   int64_t nv = 0;
   int rc = prepare_operator<X>(c, w, jacobi, &nv, true);
   if (rc) return rc;
@@ -2689,13 +2717,14 @@ static int cg_solve(fem_ctx* c, SolverWork* w, int jacobi, double bnorm2, double
   };
   if (w->res_op || w->use_bricks) {
     bool gave_up = false;
-    rc = cg_run_resident<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, iters, handovers, ms, &gave_up);
+    if (w->res_op) rc = cg_run_rows<X>(c, w, bnorm2, tol2, hold_factor2, maxit, out, &gave_up);
+    if constexpr (sizeof(X) == 4)
+      if (w->use_bricks) rc = cg_run_bricks(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, out, &gave_up);
     if (!gave_up) return rc;
     w->res_off = true;
     if ((rc = prepare_operator<X>(c, w, jacobi, &nv))) return rc;
   }
-  return cg_run<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, sizeof(X) == 4 ? w->g32 : w->g64, iters, handovers,
-                   ms);
+  return cg_run<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, sizeof(X) == 4 ? w->g32 : w->g64, out);
 }
 
 }  // namespace fem
@@ -2714,7 +2743,6 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
   const int64_t n = c->n;
   const int maxit = cfg->maxit > 0 ? cfg->maxit : 100000;
   fem_solve_info out{};
-  double cg_ms = 0.0;
   c->timings.spmv_ms = 0.0;
   c->timings.spmv_launches = 0;
 
@@ -2731,17 +2759,17 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
     return FEM_OK;
   }
   const double tol2 = cfg->rtol * cfg->rtol * bnorm2;
-  int iters = 0, handovers = 0;
+  CgResult cg;
   if (!mixed) {
-    rc = cg_solve<double>(c, w, cfg->precond, bnorm2, tol2, 0.0, maxit, &iters, &handovers, &cg_ms);
+    rc = cg_solve<double>(c, w, cfg->precond, bnorm2, tol2, 0.0, maxit, &cg);
   } else {
     // the FP32 recurrence hands over whenever its residual has fallen by δ (inner_rtol)
     const double delta = cfg->inner_rtol > 0 ? cfg->inner_rtol : 0.1;
-    rc = cg_solve<float>(c, w, cfg->precond, bnorm2, tol2, delta * delta, maxit, &iters, &handovers, &cg_ms);
+    rc = cg_solve<float>(c, w, cfg->precond, bnorm2, tol2, delta * delta, maxit, &cg);
   }
   if (rc && rc != FEM_ERR_NOCONV) return rc;
-  out.iterations = iters;
-  out.outer_iterations = handovers;
+  out.iterations = cg.iters;
+  out.outer_iterations = cg.handovers;
   out.operator_format = w->use_elem ? 4 : w->use_cells ? 3 : !w->use_lat ? 0
                         : (mixed ? w->lat.unit32 : w->lat.unit64) ? 2 : 1;
   if (w->use_cells && w->cells.dim == 3) {   // the z-marching template that ran
@@ -2752,9 +2780,8 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
       out.operator_shape = (c->tune.sell_map != 1 && grid % 8 == 0 ? 10000 : 0) + 1000 * cl.zn[pi] +
                            100 * cl.kn[pi] + 10 * cell_stages(mixed ? 4 : 8, cl.rpt[pi]) + cl.rpt[pi];
   }
-  if ((rc = read_scal(c, w, &h))) return rc;   // s->rr: the true residual of the returned u
-  out.relres = std::sqrt(h.rr / bnorm2);
-  c->timings.solve_ms = cg_ms;
+  out.relres = std::sqrt(cg.rr / bnorm2);
+  c->timings.solve_ms = cg.ms;
   if (info) *info = out;
   if (out.relres > cfg->rtol * 1.0000001) {
     char buf[160];

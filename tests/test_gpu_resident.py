@@ -1,4 +1,4 @@
-"""The resident CG (one launch per stretch between hand-overs) against the separate kernels.
+"""The resident CG (one launch, or one per stretch between hand-overs) against the separate kernels.
 
 Sizes at the edges of its parts: one block (up to a few hundred rows), one row more than a
 block's 512 threads, several rows per thread, rows whose entries lie in LDS (FP64, 27 entries,
@@ -105,3 +105,30 @@ def test_vector_field(nel):
     for mode in ("cg", "mixed"):
         fa.set_tuning(K, cg_elems=0)
         _check(K, f, mode, "sell")
+
+
+@pytest.mark.parametrize("nel", [(40, 31), (14, 13, 12)])
+@pytest.mark.parametrize("mode", ["cg", "mixed"])
+def test_ends_without_convergence(nel, mode):
+    """The step limit, and a tolerance below what FP64 reaches (the true residual stalls): the
+    launch ends, and u is what it had reached."""
+    print("case resident without convergence", nel, mode, flush=True)
+    K, f = _poisson(nel, True)
+    with pytest.raises(Exception, match="did not converge.* after 16 iterations"):
+        fa.solve(K, f, mode=mode, rtol=1e-12, maxit=10)
+    with pytest.raises(Exception, match="did not converge"):
+        fa.solve(K, f, mode=mode, rtol=1e-19, maxit=20000)
+    _check(K, f, mode, "sell" if mode == "cg" else "lattice")
+
+
+@pytest.mark.parametrize("nel", [(40, 31), (14, 13, 12)])
+@pytest.mark.parametrize("delta", [0.5, 1e-3])
+def test_hand_overs(nel, delta):
+    """Many hand-overs (δ = 0.5) and few."""
+    print("case resident hand-overs", nel, delta, flush=True)
+    K, f = _poisson(nel, False)
+    A, b = K.to_scipy(), f.to_numpy()
+    one = fa.solve(K, f, mode="mixed", rtol=1e-12, inner_rtol=delta)
+    assert one.outer_iterations >= (10 if delta == 0.5 else 3)
+    assert np.linalg.norm(b - A @ one.u) <= 2e-12 * np.linalg.norm(b)
+    assert abs(np.linalg.norm(b - A @ one.u) / np.linalg.norm(b) - one.relres) <= 1e-13
