@@ -40,6 +40,11 @@ struct ResState {
   long long ticks, begin, end;   // 100 MHz clock: in block 0's products (time), the system's first and last
 };
 
+// Fewest blocks that hold a system of several in a launch (0: its rows have too many entries), and
+// the blocks of a launch.
+int resident_blocks(int64_t rows, int widest, bool fp32);
+int resident_most_blocks(const fem_ctx* c);
+
 // Ready to run on `s` in FP32 or FP64 (structure once per pattern, values when K or the scaling
 // changed); *ok = false when the rows do not fit (the caller keeps the separate kernels).
 int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok);

@@ -965,6 +965,21 @@ static int res_most_rows(int nz, bool fp32) {
   return fp32 ? (nz == 9 ? 4096 : nz == 18 ? 2560 : 2048) : (nz == 9 ? 2048 : nz == 18 ? 1536 : 1400);
 }
 
+static int res_entries(int widest) { return widest <= 9 ? 9 : widest <= 18 ? 18 : 27; }
+
+// (several systems: their parts are less even, and a part's largest must fit)
+static double res_fill_rows(int nz, bool fp32) { return 0.85 * res_most_rows(nz, fp32); }
+
+int resident_blocks(int64_t rows, int widest, bool fp32) {
+  return widest > 27 ? 0 : (int)std::max<double>(1.0, std::ceil((double)rows / res_fill_rows(res_entries(widest), fp32)));
+}
+
+int resident_most_blocks(const fem_ctx* c) {
+  int ncu = 0;
+  (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device);
+  return std::min(ncu, kResMaxBlocks);
+}
+
 // The instantiated kernel for nz entries per row and R rows per block (null: too many).
 // Resident rows are what the 256 VGPRs of a thread hold beside the vectors (512 threads, two
 // waves per SIMD); the entries of further rows are in LDS.
@@ -1005,8 +1020,13 @@ static int res_register_rows(int nz, bool fp32) {
 // kResT rows of the largest part begun (more where their entries are in LDS), its coupled rows,
 // and every part's record read by all; parts too large for FP64 values only where nothing else
 // is left.
-static double res_triple(const double* ext, int dim, double per, int nz, int most, int* out) {
-  double best = 1e300;
+struct ResCut {
+  double cost = 1e300;
+  int n[3] = {1, 1, 1};
+};
+// cuts[m]: the best with at most m parts.
+static std::vector<ResCut> res_cuts(const double* ext, int dim, double per, int nz, int most) {
+  std::vector<ResCut> cuts(most + 1);
   const double regs = kResT * (nz == 9 ? 4 : nz == 18 ? 3 : 2), cap = nz == 27 ? regs + 360.0 : regs;
   for (int x = 1; x <= most; ++x)
     for (int y = 1; x * y <= most; ++y) {
@@ -1022,15 +1042,13 @@ static double res_triple(const double* ext, int dim, double per, int nz, int mos
         const double cost = rounds * (250.0 + 30.0 * nz) + (per * own > regs ? 1500.0 : 0.0) +
                             0.5 * per * (all - own) + 0.1 * per * own + 8.0 * x * y * z +
                             1e4 * std::max(0.0, per * own - cap);
-        if (cost < best) {
-          best = cost;
-          out[0] = x;
-          out[1] = y;
-          out[2] = z;
-        }
+        ResCut& c = cuts[x * y * z];
+        if (cost < c.cost) c = ResCut{cost, {x, y, z}};
       }
     }
-  return best;
+  for (int m = 1; m <= most; ++m)
+    if (cuts[m - 1].cost <= cuts[m].cost) cuts[m] = cuts[m - 1];
+  return cuts;
 }
 
 // Blocks per system, at most `total` of them: each the fewest that hold its rows, the others one by
@@ -1043,44 +1061,43 @@ struct ResExtent {
 static bool res_share(const std::vector<ResExtent>& e, int nz, int total, int most_rows, std::vector<int>* cut) {
   const int ng = (int)e.size();
   std::vector<int> m(ng), cap(ng);
-  std::vector<double> cost(ng), its(ng);
-  cut->assign(3 * ng, 1);
+  std::vector<double> its(ng);
+  std::vector<std::vector<ResCut>> cuts(ng);
   int used = 0;
   for (int i = 0; i < ng; ++i) {
     cap[i] = (int)std::max<double>(1.0, std::min<double>(total, std::ceil(e[i].count / kResRows)));
-    m[i] = (int)std::max<double>(1.0, std::ceil(e[i].count / (ng > 1 ? 0.85 * most_rows : most_rows)));
+    m[i] = (int)std::max<double>(1.0, std::ceil(e[i].count / (ng > 1 ? res_fill_rows(nz, true) : most_rows)));
     if (m[i] > cap[i]) return false;
     if (ng == 1) m[i] = cap[i];
     its[i] = e[i].ext[0] + e[i].ext[1] + e[i].ext[2];
     used += m[i];
+    cuts[i] = res_cuts(e[i].ext, e[i].dim, e[i].per, nz, cap[i]);
   }
   if (used > total) return false;
-  for (int i = 0; i < ng; ++i) cost[i] = res_triple(e[i].ext, e[i].dim, e[i].per, nz, m[i], &(*cut)[3 * i]);
   std::vector<bool> last(ng, false);
   for (;;) {
     int at = -1;
     for (int i = 0; i < ng; ++i)
-      if (!last[i] && (at < 0 || its[i] * cost[i] > its[at] * cost[at])) at = i;
-    if (at < 0) return true;
-    bool better = false;
-    for (int k = m[at] + 1; k <= std::min(cap[at], m[at] + total - used) && !better; ++k) {
-      int c3[3] = {1, 1, 1};
-      const double v = res_triple(e[at].ext, e[at].dim, e[at].per, nz, k, c3);
-      if (v < cost[at]) {
-        used += k - m[at];
-        m[at] = k;
-        cost[at] = v;
-        for (int d = 0; d < 3; ++d) (*cut)[3 * at + d] = c3[d];
-        better = true;
-      }
+      if (!last[i] && (at < 0 || its[i] * cuts[i][m[i]].cost > its[at] * cuts[at][m[at]].cost)) at = i;
+    if (at < 0) break;
+    const int most = std::min(cap[at], m[at] + total - used);
+    int k = m[at] + 1;
+    while (k <= most && !(cuts[at][k].cost < cuts[at][m[at]].cost)) ++k;
+    if (k <= most) {
+      used += k - m[at];
+      m[at] = k;
+    } else {
+      last[at] = true;
     }
-    if (!better) last[at] = true;
   }
+  cut->clear();
+  for (int i = 0; i < ng; ++i)
+    for (int d = 0; d < 3; ++d) cut->push_back(cuts[i][m[i]].n[d]);
+  return true;
 }
 
 static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& rows, int nz, int most_rows) {
-  int ncu = 0, maxlds = 0, coop = 0;
-  (void)hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, c->device);
+  int maxlds = 0, coop = 0;
   (void)hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device);
   (void)hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, c->device);
   const int64_t n = rows.n;
@@ -1163,7 +1180,7 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
     ext[i].dim = g.dim;
   }
   std::vector<int> cut;
-  if (!res_share(ext, nz, std::min(ncu, kResMaxBlocks), most_rows, &cut)) return FEM_OK;
+  if (!res_share(ext, nz, resident_most_blocks(c), most_rows, &cut)) return FEM_OK;
   int nb = 0;
   std::vector<int4> grp;
   for (int i = 0; i < ng; ++i) {
@@ -1287,9 +1304,11 @@ int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* s
   int rc;
   if (o->state == 0) {
     const int widest = s.widest;
-    const int nz = widest <= 9 ? 9 : widest <= 18 ? 18 : 27, most = res_most_rows(nz, fp32);
+    const int nz = res_entries(widest), most = res_most_rows(nz, fp32);
+    int64_t all = s.nsys > 0 ? 0 : s.n;
+    for (int i = 0; i < s.nsys; ++i) all += s.sys[2 * i + 1] - s.sys[2 * i];
     // clearly too large in this precision (lattice rows include some padding): nothing is built
-    if (widest > 27 || s.n < 1 || s.n > (int64_t)kResMaxBlocks * most * 5 / 4) return FEM_OK;
+    if (widest > 27 || all < 1 || all > (int64_t)kResMaxBlocks * most * 5 / 4) return FEM_OK;
     o->state = -1;
     if ((rc = res_build(c, o, s, rows, nz, res_most_rows(nz, true)))) return rc;
     if (o->state == -1) return FEM_OK;

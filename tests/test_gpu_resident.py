@@ -14,6 +14,7 @@ from conftest import gpu_available
 pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not gpu_available(), reason="needs a GPU")]
 
 import ferrite_amd as fa  # noqa: E402
+from ferrite_amd.batch import BatchedPoisson, poisson_problem  # noqa: E402
 
 
 def _move(g, nel, seed):
@@ -132,3 +133,37 @@ def test_hand_overs(nel, delta):
     assert one.outer_iterations >= (10 if delta == 0.5 else 3)
     assert np.linalg.norm(b - A @ one.u) <= 2e-12 * np.linalg.norm(b)
     assert abs(np.linalg.norm(b - A @ one.u) / np.linalg.norm(b) - one.relres) <= 1e-13
+
+
+@pytest.mark.parametrize("grids", [
+    [("Quadrilateral", (2, 2))], [("Hexahedron", (2, 1, 1))],
+    [("Quadrilateral", (2, 2)), ("Quadrilateral", (71, 69)), ("Quadrilateral", (3, 300)), ("Quadrilateral", (16, 15))],
+    [("Hexahedron", (9, 8, 7)), ("Quadrilateral", (40, 41)), ("Hexahedron", (30, 31, 32)), ("Hexahedron", (2, 2, 90)),
+     ("Quadrilateral", (180, 170)), ("Hexahedron", (7, 7, 7)), ("Hexahedron", (2, 1, 1))]])
+def test_batch(grids):
+    """Systems sharing a launch: of one block and of many, 2D and 3D, one with f = 0 (all of
+    its nodes prescribed).  First a
+    tolerance out of reach (they stall, the separate kernels take over and end at the step
+    limit), then one within reach, twice."""
+    print("case resident batch", grids, flush=True)
+    import scipy.sparse as sp
+    b = BatchedPoisson(0)
+    for i, (ct, nel) in enumerate(grids):
+        k = np.exp(np.random.default_rng(i).normal(0.0, 0.5, int(np.prod(nel))))
+        g, dh, colors, ch, k = poisson_problem(ct, nel, k)
+        b.add(g, dh, colors, ch, k)
+    b.finalize()
+    if len(grids) > 1:      # (one unknown is solved exactly)
+        with pytest.raises(fa.FemError, match="missed rtol"):
+            b.run("mixed", rtol=1e-18, maxit=2000)
+    us = []
+    for _ in range(2):
+        res = b.run("mixed", rtol=1e-11)
+        assert res.converged == len(grids) and np.all(res.completion_ms > 0)
+        us.append([b.download(i) for i in range(len(grids))])
+    for i, p in enumerate(b.problems):
+        nz, f, u = us[0][i]
+        A = sp.csc_matrix((nz, p["rowval"] - 1, p["colptr"] - 1), shape=(p["ndofs"], p["ndofs"]))
+        assert np.linalg.norm(f - A @ u) <= 1e-11 * np.linalg.norm(f) * 1.0001
+        assert np.array_equal(u, us[1][i][2])
+    b.close()
