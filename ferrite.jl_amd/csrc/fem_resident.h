@@ -75,4 +75,13 @@ int brick_run(fem_ctx* c, BrickOp* op, const BrickSource& s, const double* res, 
               double* u, Scal* scal, double hold_factor2, double tol2, int restart, int lim, bool* launched);
 void brick_free(BrickOp** op);
 
+// The same on the stored Q2 hex³ element matrices (fem_resident_elems.hip), in FP32 or FP64; the
+// matrices of the current K are read by elems_prepare.
+struct ElemsOp;
+int elems_prepare(fem_ctx* c, ElemsOp** op, const double* sc, bool fp32, bool* ok);
+template <typename X>
+int elems_run(fem_ctx* c, ElemsOp* op, const double* res, const double* sc, X* p, X* sv, double* u, Scal* scal,
+              double hold_factor2, double tol2, int restart, int lim, bool* launched);
+void elems_free(ElemsOp** op);
+
 }  // namespace fem

@@ -173,6 +173,8 @@ struct SolverWork {
   ResSource res_src;           // and where its rows come from
   BrickOp* bricks = nullptr;   // resident CG on the 3D cell form
   bool use_bricks = false;     // the current solve runs on it
+  ElemsOp* elems = nullptr;    // resident CG on Q2 element matrices
+  bool use_elems = false;      // the current solve runs on it
   bool res_off = false;        // a resident launch was not taken or gave up: not tried again
   int64_t cap32 = 0, cap64 = 0;   // length of the recurrence vectors
   int sell_grid = 0;           // blocks of the SELL SpMV (fixed: its partial count)
@@ -218,6 +220,7 @@ void free_solver(fem_ctx* c) {
   resident_free(&w->res_csc);
   resident_free(&w->res_lat);
   brick_free(&w->bricks);
+  elems_free(&w->elems);
   CellOp& cl = w->cells;
   dev_free(&cl.corg); dev_free(&cl.kc64); dev_free(&cl.kc32); dev_free(&cl.t64); dev_free(&cl.t32);
   dev_free(&cl.cnt); dev_free(&cl.up64); dev_free(&cl.yp64); dev_free(&cl.tm64); dev_free(&cl.s0);
@@ -2303,6 +2306,7 @@ static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv, 
   w->use_elem = false;
   w->res_op = nullptr;
   w->use_bricks = false;
+  w->use_elems = false;
   const bool want = sizeof(X) == 4 ? c->tune.lattice != -1 : c->tune.lattice == 1;
   const bool want_cells = sizeof(X) == 4 ? c->tune.cell_operator != -1 : c->tune.cell_operator == 1;
   if (want || want_cells) {
@@ -2324,8 +2328,14 @@ static int prepare_operator(fem_ctx* c, SolverWork* w, int jacobi, int64_t* nv, 
   // than the copy (128³ Q1 hex: 116 vs 74 µs) and run only with tuning elem_operator = 1
   const bool want_elem = c->tune.elem_operator == 1 || (c->tune.elem_operator == 0 && c->ea_kind == 3);
   if (!w->use_lat && want_elem && elem_op_valid(c)) {
-    if ((rc = elem_op_prepare(c, &w->eop, w->sc, sizeof(X) == 4, &w->elem_grid))) return rc;
     w->use_elem = true;
+    if (resident && c->ea_kind == 3 && resident_allowed(c, w)) {
+      *nv = c->n;
+      if ((rc = ensure_vecs<X>(c, w, c->n))) return rc;
+      if ((rc = elems_prepare(c, &w->elems, w->sc, sizeof(X) == 4, &w->use_elems))) return rc;
+      if (w->use_elems) return FEM_OK;
+    }
+    if ((rc = elem_op_prepare(c, &w->eop, w->sc, sizeof(X) == 4, &w->elem_grid))) return rc;
   }
   *nv = w->use_lat ? w->lat.npad : c->n;
   if ((rc = ensure_vecs<X>(c, w, *nv))) return rc;
@@ -2650,10 +2660,11 @@ static int cg_run_rows(fem_ctx* c, SolverWork* w, double bnorm2, double tol2, do
   return st->status ? FEM_OK : FEM_ERR_NOCONV;
 }
 
-// The same on bricks of the cell form: one launch per stretch (reseed, iterations, fold into u),
-// then the FP64 residual, and one read of the record by the host.
-static int cg_run_bricks(fem_ctx* c, SolverWork* w, const CgVecs<float>& v, double bnorm2, double tol2,
-                         double hold_factor2, int maxit, CgResult* out, bool* gave_up) {
+// The same on bricks of the cell form or on the Q2 element matrices: one launch per stretch
+// (reseed, iterations, fold into u), then the FP64 residual, and one read of the record by the host.
+template <typename X>
+static int cg_run_stretches(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double bnorm2, double tol2,
+                            double hold_factor2, int maxit, CgResult* out, bool* gave_up) {
   zero_vec<double>(c, c->d_u, c->n);
   k_cg_init_scal<<<1, 1, 0, c->stream>>>(w->s, bnorm2);
   const int64_t most = ((int64_t)maxit + kBatch - 1) / kBatch * kBatch;
@@ -2670,7 +2681,10 @@ static int cg_run_bricks(fem_ctx* c, SolverWork* w, const CgVecs<float>& v, doub
     const int lim = (int)std::min<int64_t>(1 << 24, most - h.iters);
     const int restart = res == c->d_f ? 1 : 0;
     bool launched = false;
-    rc = brick_run(c, w->bricks, b, res, w->sc, v.p, v.sv, c->d_u, w->s, hold_factor2, tol2, restart, lim, &launched);
+    if (w->use_elems)
+      rc = elems_run<X>(c, w->elems, res, w->sc, v.p, v.sv, c->d_u, w->s, hold_factor2, tol2, restart, lim, &launched);
+    else if constexpr (sizeof(X) == 4)
+      rc = brick_run(c, w->bricks, b, res, w->sc, v.p, v.sv, c->d_u, w->s, hold_factor2, tol2, restart, lim, &launched);
     if (rc) return rc;
     if (!launched) {
       *gave_up = true;
@@ -2715,11 +2729,10 @@ static int cg_solve(fem_ctx* c, SolverWork* w, int jacobi, double bnorm2, double
     if constexpr (sizeof(X) == 4) return CgVecs<X>{w->x32, w->r32, w->wv32, w->p32, w->sv32, nv, map};
     else return CgVecs<X>{w->x, w->r, w->wv, w->p, w->sv, nv, map};
   };
-  if (w->res_op || w->use_bricks) {
+  if (w->res_op || w->use_bricks || w->use_elems) {
     bool gave_up = false;
     if (w->res_op) rc = cg_run_rows<X>(c, w, bnorm2, tol2, hold_factor2, maxit, out, &gave_up);
-    if constexpr (sizeof(X) == 4)
-      if (w->use_bricks) rc = cg_run_bricks(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, out, &gave_up);
+    else rc = cg_run_stretches<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, out, &gave_up);
     if (!gave_up) return rc;
     w->res_off = true;
     if ((rc = prepare_operator<X>(c, w, jacobi, &nv))) return rc;
