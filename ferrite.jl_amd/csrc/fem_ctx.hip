@@ -188,7 +188,7 @@ void fem_ctx_destroy(fem_ctx* c) {
   dev_free(&c->d_acb); dev_free(&c->d_slp); dev_free(&c->d_sld); dev_free(&c->d_slv);
   dev_free(&c->d_scalar); dev_free(&c->d_partials); dev_free(&c->d_err);
   dev_free(&c->d_tab); dev_free(&c->d_tabf); dev_free(&c->d_qc); dev_free(&c->d_qcf);
-  dev_free(&c->d_aff); dev_free(&c->d_afff);
+  dev_free(&c->d_aff); dev_free(&c->d_afff); dev_free(&c->d_facet);
   if (c->ev0) (void)hipEventDestroy(c->ev0);
   if (c->ev1) (void)hipEventDestroy(c->ev1);
   if (c->evm) (void)hipEventDestroy(c->evm);

@@ -206,6 +206,11 @@ struct fem_ctx {
   double* d_ep64 = nullptr;            // Q1 quad^2 planes (36 per cell), FP64 / FP32
   float* d_ep32 = nullptr;
   int64_t ep_cells = 0;
+  // facet traction: device buffer of the largest call so far, and per dof its place in a call's
+  // list (−1 between calls)
+  double* d_facet = nullptr;
+  int64_t facet_words = 0;
+  std::vector<int32_t> facet_at;
 };
 
 namespace fem {
