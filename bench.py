@@ -149,17 +149,23 @@ def main():
         torch.cuda.synchronize()
         dt = (time.perf_counter() - t1) / args.steps
         u = fa.device.DeviceVector(K, 2).to_numpy()
-        # one more step with the CG kernels launched directly and every SpMV bracketed by HIP
-        # events on the context stream: the SpMV's launch duration inside the solve (same
-        # kernels and operands as the timed graphs), used for the roofline below
+        # one more step with timed products: where the timed steps ran the resident CG (the mixed
+        # solver at this size), its products by the clock in the kernel
         fa.set_tuning(K, time_kernels=1)
-        _, _, ts = step(mode)
-        fa.set_tuning(K, time_kernels=0)
+        r1, _, ts = step(mode)
+        product = dict(ms=ts["spmv_ms"], n=ts["spmv_launches"], solve_ms=ts["solve_ms"], its=r1.iterations)
+        # and one with the separate CG kernels (an explicit launch shape selects them; 8 is their
+        # default here), launched directly and every SpMV bracketed by HIP events on the context
+        # stream: the SpMV's launch duration inside the solve, used for the roofline below
+        fa.set_tuning(K, cg_elems=8)
+        r2, _, ts = step(mode)
+        separate = dict(solve_ms=ts["solve_ms"], its=r2.iterations)
+        fa.set_tuning(K, time_kernels=0, cg_elems=0)
         spmv_ms, spmv_n = ts["spmv_ms"], ts["spmv_launches"]
         results[name] = dict(ms=dt * 1e3, cells_per_s=g.ncells / dt, iters=iters, u=u, operator=res.operator,
                              unit_diagonal=res.unit_diagonal, cell_shape=res.cell_shape,
                              asm_kernel_ms=float(np.median(asm_ms)), spmv_avg_ms=spmv_ms / max(spmv_n, 1),
-                             spmv_launches=spmv_n)
+                             spmv_launches=spmv_n, product=product, separate=separate)
         log(f"{name}: {dt * 1e3:.1f} ms/step, iters {iters[-1]}, assembly kernels {np.median(asm_ms):.3f} ms, "
             f"SpMV {spmv_ms / max(spmv_n, 1) * 1e3:.1f} us avg over {spmv_n} launches")
 
@@ -177,9 +183,9 @@ def main():
             r, _, _ = step(mode)
         torch.cuda.synchronize()
         dtc = (time.perf_counter() - t1) / args.steps
-        fa.set_tuning(K, time_kernels=1)
+        fa.set_tuning(K, time_kernels=1, cg_elems=8)   # (the separate kernels, whatever the size)
         _, _, ts = step(mode)
-        fa.set_tuning(K, lattice=0, cell_operator=0, elem_operator=0, time_kernels=0)
+        fa.set_tuning(K, cg_elems=0, lattice=0, cell_operator=0, elem_operator=0, time_kernels=0)
         log(f"{name}: {dtc * 1e3:.1f} ms/step, {r.iterations} iterations, operator {r.operator}, SpMV "
             f"{ts['spmv_ms'] / max(ts['spmv_launches'], 1) * 1e3:.1f} us")
         return {"cells_per_s": g.ncells / dtc, "ms_per_step": dtc * 1e3, "operator": r.operator,
@@ -210,8 +216,9 @@ def main():
     fa.assemble_global(fa.start_assemble(K, f), cv, colors, el, precision="fp64")
     fa.apply(K, f, ch)
 
-    # roofline of the dominant kernel: the FP32 SpMV of the mixed solver, algorithmic bytes of its
-    # operator form.  Cell form (z-marching): t = S and x read over the padded lattice, k_e over
+    # roofline of the mixed solver's separate FP32 SpMV (the launches of the step with cg_elems = 8;
+    # the timed steps run the resident CG instead where it fits, "resident_cg" below, which reads its
+    # operator from LDS and registers), algorithmic bytes of its operator form.  Cell form (z-marching): t = S and x read over the padded lattice, k_e over
     # it (one per cell origin row), y written over the marched planes.  Lattice planes: 14 FP32
     # value planes over the computed rows (13 with the unit diagonal, whose centre plane is not
     # read), x over the padded lattice, y over the computed rows; backward neighbours re-read
@@ -241,6 +248,7 @@ def main():
         SPMV32_KERNEL = "k_sell<float, float, 0, true, 8, false, true>"   # sliced ELL, u16 offsets, NT loads
         spmv_bytes = nnz * (4 + 4) + 4 * (nd + 1) + 4 * nd + 4 * nd
     spmv_gbs = spmv_bytes / (spmv_ms * 1e-3) / 1e9
+    resident = results["mixed"]["operator"] == "cells" and (n + 1) ** 3 <= 2.6e6   # what the bricks hold
     stream = same_size_stream(torch, npad)
     lat_kernel, lat_bytes, lat_gbs = lattice_roofline(mixed_lattice["unit_diagonal"], mixed_lattice["spmv_avg_ms"])
     spmv64_iso_ms = fa.spmv_bench(K, mixed=False, reps=50)
@@ -300,7 +308,18 @@ def main():
         "fp32_element_assembly": {"kernel_ms": asm32_ms, "K_rel_err_vs_fp64": kerr32,
                                   "u_rel_err_vs_fp64": uerr32},
         "dofs_per_s": dh.ndofs / (results["mixed"]["ms"] * 1e-3),
-        "roofline": {"bound": "hbm", "kernel": SPMV32_KERNEL,
+        # the kernel the timed mixed steps spend their time in (bricks of the cell form): its
+        # iterations are bound by the product's VALU work, then by the exchange of halo values
+        # between blocks, not by HBM (the operator and the vectors stay on chip)
+        "resident_cg": None if not resident else
+                       {"kernel": "k_resident_cells" if n >= 80 else "k_resident", "bound": "valu+exchange",
+                        "product_us": results["mixed"]["product"]["ms"] * 1e3 / max(results["mixed"]["product"]["n"], 1),
+                        "products": results["mixed"]["product"]["n"],
+                        "us_per_iteration": results["mixed"]["product"]["solve_ms"] * 1e3 /
+                                            max(results["mixed"]["product"]["its"], 1),
+                        "separate_kernels_us_per_iteration": results["mixed"]["separate"]["solve_ms"] * 1e3 /
+                                                             max(results["mixed"]["separate"]["its"], 1)},
+        "roofline": {"bound": "hbm", "kernel": SPMV32_KERNEL, "in_timed_steps": not resident,
                      "achieved": spmv_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": spmv_gbs / HBM_PEAK_GBS, "traffic": measured_traffic(SPMV32_KERNEL, n),
                      "bytes_per_launch": spmv_bytes, "avg_launch_ms": spmv_ms,
@@ -361,9 +380,10 @@ def distorted_run(args, fa, np, torch, g0, ip, cv, dh0, colors, k):
         torch.cuda.synchronize()
         dt = (time.perf_counter() - t1) / args.steps
         us[name] = fa.device.DeviceVector(K, 2).to_numpy()
-        fa.set_tuning(K, lattice=-1, cell_operator=-1, elem_operator=elem, time_kernels=1)
+        fa.set_tuning(K, lattice=-1, cell_operator=-1, elem_operator=elem, time_kernels=1, cg_elems=8)
         _ = step(mode)
         ts = fa.timings(K)
+        fa.set_tuning(K, time_kernels=0, cg_elems=0)
         spmv = ts["spmv_ms"] / max(ts["spmv_launches"], 1)
         out[name] = {"cells_per_s": g.ncells / dt, "ms_per_step": dt * 1e3, "operator": r.operator,
                      "cg_iterations": r.iterations, "relres": r.relres, "spmv_avg_ms": spmv,
