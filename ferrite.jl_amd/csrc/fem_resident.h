@@ -1,5 +1,5 @@
-// Resident CG (fem_resident.hip): one launch runs the whole recurrence between two hand-overs
-// with the operator's rows, the vectors and the scalars on chip.
+// Resident CG (fem_resident.hip): one launch runs a whole solve, or the recurrence between two
+// hand-overs, with the operator's rows, the vectors and the scalars on chip.
 #pragma once
 #include "fem_internal.h"
 
