@@ -124,6 +124,7 @@ int pattern_finish(fem_ctx* c, int64_t n, int64_t nnz, const int32_t* hcolptr) {
     if (dg[j] < 0) return set_error(c, FEM_ERR_ARG, "pattern lacks a diagonal entry");
   c->n = n; c->nnz = nnz;
   c->pattern_sym = -1;
+  c->nzval_out = false;                // (a new nzval array: addresses of the old one are void)
   c->max_row_nnz = 0;
   for (int64_t j = 0; j < n; ++j) c->max_row_nnz = std::max<int>(c->max_row_nnz, hcolptr[j + 1] - hcolptr[j]);
   free_solver(c);
@@ -387,10 +388,11 @@ int32_t fem_solution_upload(fem_ctx* c, const double* u) {
 int32_t fem_device_pointer(fem_ctx* c, int32_t which, void** ptr, int64_t* nelem) {
   if (!c || !ptr) return FEM_ERR_ARG;
   switch (which) {
-    case 0:   // writable: the solver's operator copies are rebuilt from nzval at the next solve
+    case 0:   // writable: every solve from now on reads K anew (fem_solve)
       *ptr = c->d_nzval;
       if (nelem) *nelem = c->nnz;
       ++c->nzval_version;
+      c->nzval_out = true;
       break;
     case 1: *ptr = c->d_f; if (nelem) *nelem = c->ndofs; break;
     case 2: *ptr = c->d_u; if (nelem) *nelem = c->ndofs; break;

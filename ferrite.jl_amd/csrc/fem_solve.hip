@@ -2753,6 +2753,14 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
   int rc = ensure_work(c, mixed);
   if (rc) return rc;
   SolverWork* w = c->solver;
+  if (c->nzval_out) {
+    // K may have been written in place since the last solve: no copy of it is kept, least of all the
+    // FP64 one the residual is formed from.  The stored element matrices stay in use: there
+    // the residual is formed from nzval, so a K that is not theirs ends in FEM_ERR_NOCONV.
+    const bool elements = c->ea_version == c->nzval_version;
+    ++c->nzval_version;
+    if (elements) c->ea_version = c->nzval_version;
+  }
   const int64_t n = c->n;
   const int maxit = cfg->maxit > 0 ? cfg->maxit : 100000;
   fem_solve_info out{};

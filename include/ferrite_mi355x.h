@@ -190,8 +190,11 @@ int32_t fem_matrix_upload(fem_ctx* ctx, const double* nzval, const double* f);
 int32_t fem_solution_download(fem_ctx* ctx, double* u);
 int32_t fem_solution_upload(fem_ctx* ctx, const double* u);
 /* Device address of a resident array (0 = nzval, 1 = f, 2 = u) for zero-copy wrapping.  Asking
- * for nzval marks K as changed: the solver rebuilds its operator copies at the next solve, so
- * a caller may write K in place between solves. */
+ * for nzval marks K as changed, and from then on (until a new pattern) every solve builds its
+ * operator copies from nzval as it is at the call: a caller may write K in place between solves
+ * through an address it asked for once.  Element matrices stored by an assembly (tuning
+ * elem_operator) do not follow such writes, and a solve on them then fails with
+ * FEM_ERR_NOCONV: ask for the address again after the assembly, which drops them. */
 int32_t fem_device_pointer(fem_ctx* ctx, int32_t which, void** ptr, int64_t* nelem);
 
 /* ---- launch-shape tuning (autotuner interface; no counterpart in the reference) ---- */

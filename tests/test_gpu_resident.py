@@ -6,6 +6,8 @@ more than 1,024 rows per block), lattices beyond that; every source of rows (K's
 9, 18 and 27 entries per row.  An explicit launch shape of the separate kernels (cg_elems)
 selects those.  Both solve to a true residual of 1e-12, so their u differ by a few times
 cond · 1e-12: 1e-8, the bar the other solver tests use."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -133,6 +135,40 @@ def test_hand_overs(nel, delta):
     assert one.outer_iterations >= (10 if delta == 0.5 else 3)
     assert np.linalg.norm(b - A @ one.u) <= 2e-12 * np.linalg.norm(b)
     assert abs(np.linalg.norm(b - A @ one.u) / np.linalg.norm(b) - one.relres) <= 1e-13
+
+
+class _InPlace:
+    """K.nzval for torch, through an address that is asked for once."""
+
+    def __init__(self, K):
+        p, n = ctypes.c_void_p(), ctypes.c_int64(0)
+        K.ctx.call("fem_device_pointer", 0, ctypes.byref(p), ctypes.byref(n))
+        self.__cuda_array_interface__ = dict(shape=(n.value,), typestr="<f8", data=(p.value, False), version=2)
+
+
+_FORMS = [((40, 31), dict(lattice=-1, cell_operator=-1)), ((40, 31), dict(cell_operator=-1)), ((40, 31), {}),
+          ((14, 13, 12), dict(lattice=-1, cell_operator=-1)), ((14, 13, 12), {})]
+
+
+@pytest.mark.parametrize("nel,forms,mode,cg_elems",
+                         [(*x, mode, e) for x in _FORMS for mode in ("mixed", "cg") for e in (0, 8)] +
+                         [((90, 84, 80), {}, "mixed", 0)])
+def test_K_written_in_place(nel, forms, mode, cg_elems):
+    """A caller keeps K's address and writes K in place between solves: every solve is of the K
+    that is there, on every form of the rows (the last case: bricks), resident or not."""
+    print("case resident K in place", nel, forms, mode, cg_elems, flush=True)
+    import torch
+    K, f = _poisson(nel, False, cg_elems=cg_elems, **forms)
+    nz = torch.as_tensor(_InPlace(K), device="cuda")
+    u = fa.solve(K, f, mode=mode, rtol=1e-12).u
+    for scale in (2.0, 0.25):
+        nz *= scale
+        torch.cuda.synchronize()
+        now = fa.solve(K, f, mode=mode, rtol=1e-12)
+        u = u / scale
+        A, b = K.to_scipy(), f.to_numpy()
+        assert np.linalg.norm(b - A @ now.u) <= 2e-12 * np.linalg.norm(b)
+        assert np.linalg.norm(now.u - u) <= 1e-8 * np.linalg.norm(u)
 
 
 @pytest.mark.parametrize("nel", [(1, 1, 1), (2, 1, 1), (3, 3, 2), (5, 4, 4), (60, 1, 1), (2, 30, 3), (11, 12, 11),
