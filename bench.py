@@ -163,7 +163,7 @@ def main():
         fa.set_tuning(K, time_kernels=0, cg_elems=0)
         spmv_ms, spmv_n = ts["spmv_ms"], ts["spmv_launches"]
         results[name] = dict(ms=dt * 1e3, cells_per_s=g.ncells / dt, iters=iters, u=u, operator=res.operator,
-                             unit_diagonal=res.unit_diagonal, cell_shape=res.cell_shape,
+                             unit_diagonal=res.unit_diagonal, cell_shape=res.cell_shape, kernels=res.kernels,
                              asm_kernel_ms=float(np.median(asm_ms)), spmv_avg_ms=spmv_ms / max(spmv_n, 1),
                              spmv_launches=spmv_n, product=product, separate=separate)
         log(f"{name}: {dt * 1e3:.1f} ms/step, iters {iters[-1]}, assembly kernels {np.median(asm_ms):.3f} ms, "
@@ -188,7 +188,7 @@ def main():
         fa.set_tuning(K, cg_elems=0, lattice=0, cell_operator=0, elem_operator=0, time_kernels=0)
         log(f"{name}: {dtc * 1e3:.1f} ms/step, {r.iterations} iterations, operator {r.operator}, SpMV "
             f"{ts['spmv_ms'] / max(ts['spmv_launches'], 1) * 1e3:.1f} us")
-        return {"cells_per_s": g.ncells / dtc, "ms_per_step": dtc * 1e3, "operator": r.operator,
+        return {"cells_per_s": g.ncells / dtc, "ms_per_step": dtc * 1e3, "operator": r.operator, "kernels": r.kernels,
                 "cg_iterations": r.iterations, "relres": r.relres,
                 "spmv_avg_ms": ts["spmv_ms"] / max(ts["spmv_launches"], 1), "unit_diagonal": r.unit_diagonal}
 
@@ -236,7 +236,7 @@ def main():
 
     spmv_ms = results["mixed"]["spmv_avg_ms"]               # inside the CG loop of the timed steps
     if results["mixed"]["operator"] == "cells" and results["mixed"]["cell_shape"]:
-        # the z-marching template the solver reports (MAP, ZN, KN, stages, rows per thread)
+        # the z-marching template of the separate kernels (MAP, ZN, KN, stages, rows per thread)
         SPMV32_KERNEL = "k_cell_spmv_z<float, {}, {}, {}, {}, {}>".format(*results["mixed"]["cell_shape"])
         spmv_bytes = 3 * 4 * npad + 4 * (px - 2) * px * px
     elif results["mixed"]["operator"] == "cells":
@@ -248,7 +248,8 @@ def main():
         SPMV32_KERNEL = "k_sell<float, float, 0, true, 8, false, true>"   # sliced ELL, u16 offsets, NT loads
         spmv_bytes = nnz * (4 + 4) + 4 * (nd + 1) + 4 * nd + 4 * nd
     spmv_gbs = spmv_bytes / (spmv_ms * 1e-3) / 1e9
-    resident = results["mixed"]["operator"] == "cells" and (n + 1) ** 3 <= 2.6e6   # what the bricks hold
+    resident = {"rows": "k_resident", "bricks": "k_resident_cells", "elements": "k_resident_elems"}.get(
+        results["mixed"]["kernels"])   # what the timed steps ran, None: the separate kernels
     stream = same_size_stream(torch, npad)
     lat_kernel, lat_bytes, lat_gbs = lattice_roofline(mixed_lattice["unit_diagonal"], mixed_lattice["spmv_avg_ms"])
     spmv64_iso_ms = fa.spmv_bench(K, mixed=False, reps=50)
@@ -281,10 +282,10 @@ def main():
                    "cells": g.ncells, "dofs": dh.ndofs, "nnz": nnz, "colors": len(colors),
                    "coloring": args.coloring, "seed": args.seed},
         "fp64": {"cells_per_s": results["fp64"]["cells_per_s"], "ms_per_step": results["fp64"]["ms"],
-                 "operator": results["fp64"]["operator"],
+                 "operator": results["fp64"]["operator"], "kernels": results["fp64"]["kernels"],
                  "cg_iterations": results["fp64"]["iters"][-1][0], "relres": results["fp64"]["iters"][-1][2]},
         "mixed": {"cells_per_s": results["mixed"]["cells_per_s"], "ms_per_step": results["mixed"]["ms"],
-                  "operator": results["mixed"]["operator"],
+                  "operator": results["mixed"]["operator"], "kernels": results["mixed"]["kernels"],
                   "cg_iterations": results["mixed"]["iters"][-1][0],
                   "refinements": results["mixed"]["iters"][-1][1], "relres": results["mixed"]["iters"][-1][2]},
         "mixed_speedup_vs_fp64": results["fp64"]["ms"] / results["mixed"]["ms"],
@@ -312,14 +313,14 @@ def main():
         # iterations are bound by the product's VALU work, then by the exchange of halo values
         # between blocks, not by HBM (the operator and the vectors stay on chip)
         "resident_cg": None if not resident else
-                       {"kernel": "k_resident_cells" if n >= 80 else "k_resident", "bound": "valu+exchange",
+                       {"kernel": resident, "bound": "valu+exchange",
                         "product_us": results["mixed"]["product"]["ms"] * 1e3 / max(results["mixed"]["product"]["n"], 1),
                         "products": results["mixed"]["product"]["n"],
                         "us_per_iteration": results["mixed"]["product"]["solve_ms"] * 1e3 /
                                             max(results["mixed"]["product"]["its"], 1),
                         "separate_kernels_us_per_iteration": results["mixed"]["separate"]["solve_ms"] * 1e3 /
                                                              max(results["mixed"]["separate"]["its"], 1)},
-        "roofline": {"bound": "hbm", "kernel": SPMV32_KERNEL, "in_timed_steps": not resident,
+        "roofline": {"bound": "hbm", "kernel": SPMV32_KERNEL, "in_timed_steps": resident is None,
                      "achieved": spmv_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": spmv_gbs / HBM_PEAK_GBS, "traffic": measured_traffic(SPMV32_KERNEL, n),
                      "bytes_per_launch": spmv_bytes, "avg_launch_ms": spmv_ms,
@@ -386,7 +387,7 @@ def distorted_run(args, fa, np, torch, g0, ip, cv, dh0, colors, k):
         fa.set_tuning(K, time_kernels=0, cg_elems=0)
         spmv = ts["spmv_ms"] / max(ts["spmv_launches"], 1)
         out[name] = {"cells_per_s": g.ncells / dt, "ms_per_step": dt * 1e3, "operator": r.operator,
-                     "cg_iterations": r.iterations, "relres": r.relres, "spmv_avg_ms": spmv,
+                     "kernels": r.kernels, "cg_iterations": r.iterations, "relres": r.relres, "spmv_avg_ms": spmv,
                      "assembly_kernel_ms": t_asm}
         log(f"distorted {name}: {dt * 1e3:.1f} ms/step, {r.iterations} iterations, operator {r.operator}, "
             f"SpMV {spmv * 1e3:.1f} us, assembly {t_asm:.3f} ms")

@@ -138,7 +138,7 @@ struct fem_batch {
   int32_t* d_rnode = nullptr;
   int res_state = 0;                // 1 planned, −1 not in use
   std::vector<double> last_times_ms;
-  std::vector<int> last_iters;
+  std::vector<int> last_iters, last_kernels;   // (kernels: 1 resident, 0 separate)
 };
 
 namespace fem {
@@ -1654,6 +1654,8 @@ int32_t fem_batch_run(fem_batch* B, const fem_batch_cfg* cfg, fem_batch_info* in
     if (done_ms[p] < 0) iters[p] = hs[p].iters;   // unconverged: iterations so far, completion -1
   B->last_times_ms = done_ms;
   B->last_iters = iters;
+  B->last_kernels.assign(np_, 0);
+  for (int p = 0; p < np_; ++p) B->last_kernels[p] = state[p] != 0;
   ++c->nzval_version;
   if (info) {
     info->assemble_ms = t_asm;
@@ -1685,6 +1687,12 @@ int32_t fem_batch_problem_stats(const fem_batch* B, double* completion_ms, int32
     if (completion_ms) completion_ms[p] = B->last_times_ms[p];
     if (iterations) iterations[p] = B->last_iters[p];
   }
+  return FEM_OK;
+}
+
+int32_t fem_batch_problem_kernels(const fem_batch* B, int32_t* kernels) {
+  if (!B || !kernels) return FEM_ERR_ARG;
+  std::copy(B->last_kernels.begin(), B->last_kernels.end(), kernels);
   return FEM_OK;
 }
 

@@ -187,6 +187,7 @@ struct fem_ctx {
 
   fem::DevError* d_err = nullptr;
   fem::SolverWork* solver = nullptr;
+  int solve_kernels = -1;              // of the last solve (fem_solve_kernels)
 
   fem_timings timings{};
   fem_tuning tune{};

@@ -2733,10 +2733,12 @@ static int cg_solve(fem_ctx* c, SolverWork* w, int jacobi, double bnorm2, double
     bool gave_up = false;
     if (w->res_op) rc = cg_run_rows<X>(c, w, bnorm2, tol2, hold_factor2, maxit, out, &gave_up);
     else rc = cg_run_stretches<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, out, &gave_up);
+    c->solve_kernels = w->res_op ? 1 : w->use_bricks ? 2 : 3;
     if (!gave_up) return rc;
     w->res_off = true;
     if ((rc = prepare_operator<X>(c, w, jacobi, &nv))) return rc;
   }
+  c->solve_kernels = 0;
   return cg_run<X>(c, w, vecs(), bnorm2, tol2, hold_factor2, maxit, sizeof(X) == 4 ? w->g32 : w->g64, out);
 }
 
@@ -2764,6 +2766,7 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
   const int64_t n = c->n;
   const int maxit = cfg->maxit > 0 ? cfg->maxit : 100000;
   fem_solve_info out{};
+  c->solve_kernels = -1;
   c->timings.spmv_ms = 0.0;
   c->timings.spmv_launches = 0;
 
@@ -2793,7 +2796,7 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
   out.outer_iterations = cg.handovers;
   out.operator_format = w->use_elem ? 4 : w->use_cells ? 3 : !w->use_lat ? 0
                         : (mixed ? w->lat.unit32 : w->lat.unit64) ? 2 : 1;
-  if (w->use_cells && w->cells.dim == 3) {   // the z-marching template that ran
+  if (w->use_cells && w->cells.dim == 3) {   // the z-marching template of the separate SpMV
     const int pi = mixed ? 0 : 1;
     const CellOp& cl = w->cells;
     const int grid = mixed ? cl.grid32 : cl.grid64;
@@ -2809,6 +2812,13 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
     snprintf(buf, sizeof buf, "CG did not converge: relres %.3e after %d iterations", out.relres, out.iterations);
     return set_error(c, FEM_ERR_NOCONV, buf);
   }
+  return FEM_OK;
+}
+
+extern "C" int32_t fem_solve_kernels(const fem_ctx* c, int32_t* kernels, int32_t* gave_up) {
+  if (!c) return FEM_ERR_ARG;
+  if (kernels) *kernels = c->solve_kernels;
+  if (gave_up) *gave_up = c->solver && c->solver->res_off ? 1 : 0;
   return FEM_OK;
 }
 

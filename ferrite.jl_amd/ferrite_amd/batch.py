@@ -28,7 +28,7 @@ from .values import CellValues
 
 
 class BatchResult:
-    def __init__(self, info, completion_ms, iterations):
+    def __init__(self, info, completion_ms, iterations, kernels):
         self.assemble_ms = info.assemble_ms
         self.apply_ms = info.apply_ms
         self.solve_ms = info.solve_ms
@@ -37,6 +37,8 @@ class BatchResult:
         self.total_iterations = info.total_iterations
         self.completion_ms = completion_ms
         self.iterations = iterations
+        # per problem: 1 solved in a launch that several share (the resident CG), 0 by the separate kernels
+        self.kernels = kernels
 
     def percentile(self, q):
         return float(np.percentile(self.completion_ms, q))
@@ -137,7 +139,9 @@ class BatchedPoisson:
         it = np.zeros(n, dtype=np.int32)
         L.lib().fem_batch_problem_stats(self._h, L.ptr(ms, C.c_double), L.ptr(it, C.c_int32))
         L.raise_for(rc, self._h, "fem_batch_run", batch=True)
-        return BatchResult(info, ms, it)
+        kernels = np.zeros(n, dtype=np.int32)
+        self._call("fem_batch_problem_kernels", L.ptr(kernels, C.c_int32))
+        return BatchResult(info, ms, it, kernels)
 
     def download(self, i):
         p = self.problems[i]

@@ -270,7 +270,7 @@ def apply_solution(K, ch, applyzero=False, download=True):
 
 
 class SolveResult:
-    def __init__(self, info, u):
+    def __init__(self, info, u, kernels, gave_up):
         self.iterations = info.iterations
         self.outer_iterations = info.outer_iterations
         self.relres = info.relres
@@ -278,7 +278,12 @@ class SolveResult:
         # or "cells" (per-cell coefficients times cell 0's unit-coefficient element matrix)
         self.operator = {1: "lattice", 2: "lattice", 3: "cells", 4: "elements"}.get(info.operator_format, "sell")
         self.unit_diagonal = info.operator_format == 2
-        # the 3D cell form's SpMV template (MAP, ZN, KN, stages, rows per thread), or None
+        # the kernels that ran: "separate" (an SpMV and a vector step per iteration), or one launch on
+        # the "rows" of the operator, on "bricks" of the cell form, on the Q2 "elements"; None: f = 0
+        self.kernels = {0: "separate", 1: "rows", 2: "bricks", 3: "elements"}.get(kernels)
+        # a one-launch solve was refused or stopped waiting: solves stay on the separate kernels
+        self.gave_up = bool(gave_up)
+        # the 3D cell form's separate SpMV template (MAP, ZN, KN, stages, rows per thread), or None
         sh = info.operator_shape
         self.cell_shape = None if sh <= 0 else (sh // 10000, sh // 1000 % 10, sh // 100 % 10, sh // 10 % 10, sh % 10)
         self.u = u
@@ -291,8 +296,10 @@ def solve(K, f, mode="cg", rtol=1e-10, maxit=0, precond="jacobi", inner_rtol=0.0
                      precond=1 if precond == "jacobi" else 0, reserved=0)
     info = L.SolveInfo()
     K.ctx.call("fem_solve", C.byref(cfg), C.byref(info))
+    kernels, gave_up = C.c_int32(0), C.c_int32(0)
+    K.ctx.call("fem_solve_kernels", C.byref(kernels), C.byref(gave_up))
     u = DeviceVector(K, 2).to_numpy() if download else None
-    return SolveResult(info, u)
+    return SolveResult(info, u, kernels.value, gave_up.value)
 
 
 def timings(K):

@@ -175,12 +175,22 @@ typedef struct {
                                 SpMV does not read the centre plane, 3 cell coefficients
                                 (tuning cell_operator), 4 the element matrices of the last
                                 assembly (tuning elem_operator) */
-  int32_t operator_shape;    /* the z-marching cell-form SpMV's template (format 3, 3D):
-                                MAP·10⁴ + ZN·10³ + KN·10² + stages·10 + rows per thread of
-                                k_cell_spmv_z<X, MAP, ZN, KN, stages, rows>; 0 otherwise */
+  int32_t operator_shape;    /* format 3, 3D: the template of the z-marching cell-form SpMV on this
+                                lattice, MAP·10⁴ + ZN·10³ + KN·10² + stages·10 + rows per thread of
+                                k_cell_spmv_z<X, MAP, ZN, KN, stages, rows>, which runs in the
+                                separate kernels and in fem_spmv_bench (fem_solve_kernels says
+                                whether the solve used them); 0 otherwise */
 } fem_solve_info;
 
 int32_t fem_solve(fem_ctx* ctx, const fem_solve_cfg* cfg, fem_solve_info* info);
+
+/* Which kernels ran the last fem_solve's recurrence: 0 the separate ones (an SpMV and a vector
+ * step per iteration), or in one launch (1: per solve; 2, 3: per stretch between two reliable
+ * updates) 1 the rows' entries, 2 bricks of the cell form, 3 the Q2 element matrices; -1 no solve
+ * yet, or f = 0.  *gave_up: 1 when a one-launch solve was refused by the device or stopped waiting
+ * for one of its blocks; solves then start over on the separate kernels, and stay on them
+ * until fem_set_tuning or a new mesh, dofs or pattern.  Either pointer may be NULL. */
+int32_t fem_solve_kernels(const fem_ctx* ctx, int32_t* kernels, int32_t* gave_up);
 
 /* ---- results ---- */
 int32_t fem_matrix_download(fem_ctx* ctx, double* nzval, double* f);

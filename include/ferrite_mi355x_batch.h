@@ -77,6 +77,10 @@ int32_t fem_batch_run(fem_batch* b, const fem_batch_cfg* cfg, fem_batch_info* in
  * iterations; arrays of length nproblems. */
 int32_t fem_batch_problem_stats(const fem_batch* b, double* completion_ms, int32_t* iterations);
 
+/* Per problem of the last run the kernels that solved it: 1 the launch that several problems
+ * share (the resident CG), 0 the separate kernels; array of length nproblems. */
+int32_t fem_batch_problem_kernels(const fem_batch* b, int32_t* kernels);
+
 /* Assembly only (zero + one launch per colour), timed with HIP events: *ms. */
 int32_t fem_batch_assemble_only(fem_batch* b, int32_t precision, int32_t cells_per_wg, int32_t chunk, double* ms);
 

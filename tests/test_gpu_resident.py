@@ -47,16 +47,16 @@ def _poisson(nel, distort, **tune):
     return K, f
 
 
-def _check(K, f, mode, operator):
+def _check(K, f, mode, operator, kernels):
     A, b = K.to_scipy(), f.to_numpy()
     one = fa.solve(K, f, mode=mode, rtol=1e-12)
     two = fa.solve(K, f, mode=mode, rtol=1e-12)
-    assert one.operator == operator
+    assert one.operator == operator and one.kernels == kernels and not one.gave_up
     assert np.array_equal(one.u, two.u) and one.iterations == two.iterations
     assert np.linalg.norm(b - A @ one.u) <= 2e-12 * np.linalg.norm(b)
     fa.set_tuning(K, cg_elems=8)
     sep = fa.solve(K, f, mode=mode, rtol=1e-12)
-    assert sep.operator == operator
+    assert sep.operator == operator and sep.kernels == "separate"
     assert np.linalg.norm(one.u - sep.u) <= 1e-8 * np.linalg.norm(sep.u)
 
 
@@ -65,10 +65,10 @@ def _check(K, f, mode, operator):
 def test_rows_of_K(nel):
     print("case resident rows of K", nel, flush=True)
     K, f = _poisson(nel, True, lattice=-1, cell_operator=-1)
-    _check(K, f, "cg", "sell")
+    _check(K, f, "cg", "sell", "rows")
     if len(nel) == 2 or nel[0] < 60:
         fa.set_tuning(K, cg_elems=0)
-        _check(K, f, "mixed", "sell")
+        _check(K, f, "mixed", "sell", "rows")
 
 
 @pytest.mark.parametrize("nel", [(15, 15), (24, 21), (71, 69), (7, 7, 7), (13, 12, 11), (40, 38, 36)])
@@ -79,7 +79,7 @@ def test_lattice_rows(nel, operator):
     K, f = _poisson(nel, operator == "lattice", **forms)
     for mode in ("mixed", "cg"):
         fa.set_tuning(K, cg_elems=0)
-        _check(K, f, mode, operator)
+        _check(K, f, mode, operator, "rows")
 
 
 @pytest.mark.parametrize("nel", [(90, 84, 80), (61, 140, 66), (200, 60, 50)])
@@ -88,7 +88,7 @@ def test_cell_bricks(nel):
     inhomogeneous prescribed rows on one side)."""
     print("case resident cell bricks", nel, flush=True)
     K, f = _poisson(nel, False)
-    _check(K, f, "mixed", "cells")
+    _check(K, f, "mixed", "cells", "bricks")
 
 
 @pytest.mark.parametrize("nel", [(11, 11), (40, 23), (130, 64)])
@@ -101,13 +101,13 @@ def test_vector_field(nel):
     f = fa.allocate_vector(K)
     cv = fa.CellValues(fa.QuadratureRule("RefQuadrilateral", 2), ip)
     fa.assemble_global(fa.start_assemble(K, f), cv, fa.create_coloring(g), fa.ElasticityElement(nu=0.3))
-    fa.add_point_load(K, f, [dh.ndofs], [-1.0])
+    fa.add_point_load(K, f, [int(dh.cell_dofs[nel[1] // 2 * nel[0] + nel[0] // 2, 1])], [-1.0])   # an inner node
     ch = fa.ConstraintHandler(dh)
     ch.add(fa.Dirichlet("u", g.facetsets["left"] + g.facetsets["right"], lambda x, t: [0.0, 0.0])).close()
     fa.apply(K, f, ch)
     for mode in ("cg", "mixed"):
         fa.set_tuning(K, cg_elems=0)
-        _check(K, f, mode, "sell")
+        _check(K, f, mode, "sell", "rows")
 
 
 @pytest.mark.parametrize("nel", [(40, 31), (14, 13, 12)])
@@ -121,7 +121,7 @@ def test_ends_without_convergence(nel, mode):
         fa.solve(K, f, mode=mode, rtol=1e-12, maxit=10)
     with pytest.raises(Exception, match="did not converge"):
         fa.solve(K, f, mode=mode, rtol=1e-19, maxit=20000)
-    _check(K, f, mode, "sell" if mode == "cg" else "lattice")
+    _check(K, f, mode, "sell" if mode == "cg" else "lattice", "rows")
 
 
 @pytest.mark.parametrize("nel", [(40, 31), (14, 13, 12)])
@@ -132,6 +132,7 @@ def test_hand_overs(nel, delta):
     K, f = _poisson(nel, False)
     A, b = K.to_scipy(), f.to_numpy()
     one = fa.solve(K, f, mode="mixed", rtol=1e-12, inner_rtol=delta)
+    assert one.kernels == "rows"
     assert one.outer_iterations >= (10 if delta == 0.5 else 3)
     assert np.linalg.norm(b - A @ one.u) <= 2e-12 * np.linalg.norm(b)
     assert abs(np.linalg.norm(b - A @ one.u) / np.linalg.norm(b) - one.relres) <= 1e-13
@@ -160,7 +161,9 @@ def test_K_written_in_place(nel, forms, mode, cg_elems):
     import torch
     K, f = _poisson(nel, False, cg_elems=cg_elems, **forms)
     nz = torch.as_tensor(_InPlace(K), device="cuda")
-    u = fa.solve(K, f, mode=mode, rtol=1e-12).u
+    one = fa.solve(K, f, mode=mode, rtol=1e-12)
+    assert one.kernels == ("separate" if cg_elems else "bricks" if nel == (90, 84, 80) else "rows")
+    u = one.u
     for scale in (2.0, 0.25):
         nz *= scale
         torch.cuda.synchronize()
@@ -196,7 +199,7 @@ def test_q2_elements(nel, precision):
     # separate kernels either, 8e-12 and 5e-10)
     for mode in ("cg",) if nel == (60, 1, 1) else ("cg", "mixed"):
         fa.set_tuning(K, cg_elems=0)
-        _check(K, f, mode, "elements")
+        _check(K, f, mode, "elements", "separate" if nel == (13, 11, 11) else "elements")
 
 
 @pytest.mark.parametrize("grids", [
@@ -223,7 +226,7 @@ def test_batch(grids):
     us = []
     for _ in range(2):
         res = b.run("mixed", rtol=1e-11)
-        assert res.converged == len(grids) and np.all(res.completion_ms > 0)
+        assert res.converged == len(grids) and np.all(res.completion_ms > 0) and np.all(res.kernels == 1)
         us.append([b.download(i) for i in range(len(grids))])
     for i, p in enumerate(b.problems):
         nz, f, u = us[0][i]
