@@ -1696,6 +1696,8 @@ int32_t fem_batch_problem_kernels(const fem_batch* B, int32_t* kernels) {
   return FEM_OK;
 }
 
+int32_t fem_batch_set_wait_limit(fem_batch* B, int32_t polls) { return B ? fem_set_wait_limit(B->c, polls) : FEM_ERR_ARG; }
+
 int32_t fem_batch_download(fem_batch* B, int32_t prob, double* nzval, double* f, double* u) {
   if (!B) return FEM_ERR_ARG;
   fem_ctx* c = B->c;

@@ -43,6 +43,8 @@ struct DevError {
 
 struct SolverWork;
 
+constexpr uint32_t kResPolls = 1u << 22;   // polls of a wait in a one-launch solve: some seconds, far above any real one
+
 // CG scalars of the scaled system (hat quantities): γ = r̂·r̂, δ = r̂·Â r̂.
 struct Scal {
   double rz;      // γ of the current residual
@@ -188,6 +190,7 @@ struct fem_ctx {
   fem::DevError* d_err = nullptr;
   fem::SolverWork* solver = nullptr;
   int solve_kernels = -1;              // of the last solve (fem_solve_kernels)
+  uint32_t res_polls = fem::kResPolls; // one-launch solves: polls of a wait (fem_set_wait_limit)
 
   fem_timings timings{};
   fem_tuning tune{};

@@ -23,7 +23,7 @@
 // they carry the number.  Two buffers alternate: a block writes exchange e + 2 only after it
 // holds every block's partials of e + 1, which they publish after reading all of e.  Partials
 // are summed in block order, so every block holds the same scalars and results are bitwise
-// reproducible.  Waits are bounded (kSpinLimit): a block that gives up reports it and stops
+// reproducible.  Waits are bounded (kResPolls): a block that gives up reports it and stops
 // publishing, so every other block gives up too, and the host runs the separate kernels.
 //
 // Measured, µs per iteration, separate kernels → here: 100×100 Q1 quads FP64 11.7 → 3.0 (21
@@ -520,7 +520,7 @@ struct ResArgs {
   ResState* st;
   uint32_t *wx, *wu, *rec;
   double in0[2], hold2;
-  uint32_t epoch;
+  uint32_t epoch, polls;
   int lim, time;
 };
 
@@ -540,6 +540,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
   __shared__ double red[2][2][kResWaves];    // wave sums, alternating
   __shared__ double tot[2][2][4];            // sums of 64 blocks' partials each
   __shared__ int gaveup;
+  __shared__ uint32_t polls;                 // what a wait may take (in LDS: scalar registers are short)
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int b = blockIdx.x;
   const int4 gr = a.grp[b];
@@ -559,8 +560,10 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
   const double tol2 = a.in ? a.in[2 * gr.x + 1] : a.in0[1];
   if (t == 0) {
     gaveup = 0;
+    polls = a.polls;
     rl[zero] = X(0);
   }
+  auto polls_left = [&]() { return (uint32_t)uniform((int)polls); };
 
   // operator rows
   X av[RRES][NZ];
@@ -666,7 +669,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
         for (int k = 0; k < H; ++k) {
           at[k] = wi + (uint32_t)hl[min(base + k * kResT + t, nh - 1)];   // (spare threads repeat the last row)
         }
-        for (uint32_t spin = 0;; ++spin) {
+        for (uint32_t left = polls_left();; --left) {
           asm volatile("" ::: "memory");
           bool ok = true;
           if (need) {
@@ -681,7 +684,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
             if (base + k * kResT < nh) ok = ok && LL<X>::ok(hv[k], ep);
           if (need) need = !(LL<double>::ok(q0, ep) && LL<double>::ok(q1, ep));
           if (ok) break;
-          if (spin >= kSpinLimit) { lost = true; break; }
+          if (left == 0) { lost = true; break; }
         }
 #pragma unroll
         for (int k = 0; k < H; ++k)
@@ -689,12 +692,12 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
       }
     }
     if (wave < (kResMaxBlocks + 63) / 64) {
-      for (uint32_t spin = 0; need; ++spin) {
+      for (uint32_t left = polls_left(); need; --left) {
         asm volatile("" ::: "memory");
         q0 = LL<double>::get(rr, rin);
         q1 = LL<double>::get(rr, rin + kResMaxBlocks);
         need = !(LL<double>::ok(q0, ep) && LL<double>::ok(q1, ep));
-        if (spin >= kSpinLimit) { lost = true; break; }
+        if (left == 0) { lost = true; break; }
       }
       const double s0 = wave_sum63(reader ? LL<double>::val(q0) : 0.0);
       const double s1 = wave_sum63(reader ? LL<double>::val(q1) : 0.0);
@@ -742,11 +745,11 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
     for (int h = tt; h < nh; h += kResT) {
       const uint32_t at = (uint32_t)hl[h];
       U4 q = {};
-      for (uint32_t spin = 0;; ++spin) {
+      for (uint32_t left = polls_left();; --left) {
         asm volatile("" ::: "memory");
         q = LL<double>::get(ru, at);
         if (LL<double>::ok(q, ep)) break;
-        if (spin >= kSpinLimit) { gaveup = 1; break; }
+        if (left == 0) { gaveup = 1; break; }
       }
       ul[nown + h] = LL<double>::val(q);
     }
@@ -1388,6 +1391,7 @@ int resident_run(fem_ctx* c, ResOp* o, const ResSource& s, const double* sc, con
   a.in0[1] = tol2;
   a.hold2 = hold_factor2;
   a.epoch = o->epoch + 1u;
+  a.polls = c->res_polls;
   a.lim = lim;
   a.time = c->tune.time_kernels;
   std::fill(o->st, o->st + o->ng, ResState{});

@@ -63,7 +63,7 @@ struct BrickArgs {
   Scal* s;
   uint32_t *wx, *rec;
   double hold2, tol2;
-  uint32_t epoch;
+  uint32_t epoch, polls;
   int restart, lim, time;
   CellKrefT<float> kr;
 };
@@ -89,6 +89,7 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
   __shared__ double red[2][2][kResWaves];
   __shared__ double tot[2][2][4];
   __shared__ int gaveup;
+  __shared__ uint32_t polls;                 // what a wait may take (in LDS: scalar registers are short)
   float* zl = reinterpret_cast<float*>(brick_lds);     // [bz + 2][by + 2][SX]
   float* kl = zl + a.zplane * (a.mz + 2);              // [bz + 1][by + 1][KX]
   float* xl = kl + a.kplane * (a.mz + 1);              // [BZ][kResT] x̂
@@ -105,7 +106,11 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
   const int cx = t % bx, cy = t / bx;
   const double rzp0 = a.s->rzp, rr0 = a.s->rr;
   const bool keep0 = !a.restart && !a.s->restart && rzp0 > 0.0;
-  if (t == 0) gaveup = 0;
+  if (t == 0) {
+    gaveup = 0;
+    polls = a.polls;
+  }
+  auto polls_left = [&]() { return (uint32_t)uniform((int)polls); };
   auto row_of = [&](int x, int y, int z) { return (x + 1) + a.px * (y + 1) + a.pxy * (z + 1); };   // padded row
 
   // coefficients of the cells whose first corner is one of (x0 − 1 .., y0 − 1 .., z0 − 1 ..)
@@ -224,7 +229,7 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
       uint32_t q[H];
 #pragma unroll
       for (int k = 0; k < H; ++k) q[k] = at + hq[t + k * kResT];
-      for (uint32_t spin = 0;; ++spin) {
+      for (uint32_t left = polls_left();; --left) {
         asm volatile("" ::: "memory");
         bool ok = true;
         if (need) {
@@ -239,19 +244,19 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
           if (there >> k & 1u) ok = ok && LL<float>::ok(hv[k], ep);
         if (need) need = !(LL<double>::ok(q0, ep) && LL<double>::ok(q1, ep));
         if (ok) break;
-        if (spin >= kSpinLimit) { lost = true; break; }
+        if (left == 0) { lost = true; break; }
       }
 #pragma unroll
       for (int k = 0; k < H; ++k)
         if (there >> k & 1u) hw[k] = LL<float>::val(hv[k]);
     }
     if (wave < (kResMaxBlocks + 63) / 64) {
-      for (uint32_t spin = 0; need; ++spin) {
+      for (uint32_t left = polls_left(); need; --left) {
         asm volatile("" ::: "memory");
         q0 = LL<double>::get(rr, rin);
         q1 = LL<double>::get(rr, rin + kResMaxBlocks);
         need = !(LL<double>::ok(q0, ep) && LL<double>::ok(q1, ep));
-        if (spin >= kSpinLimit) { lost = true; break; }
+        if (left == 0) { lost = true; break; }
       }
       const double s0 = wave_sum63(reader ? LL<double>::val(q0) : 0.0);
       const double s1 = wave_sum63(reader ? LL<double>::val(q1) : 0.0);
@@ -536,7 +541,7 @@ int brick_run(fem_ctx* c, BrickOp* o, const BrickSource& s, const double* res, c
   }
   BrickArgs a{o->n[0], o->n[1], o->n[2], o->cut[0], o->cut[1], o->cut[2], o->slots,
               kBrickSX * (o->most[1] + 2), kBrickKX * (o->most[1] + 1), o->most[2], s.px, s.pxy,
-              s.t, s.kc, s.dofp, res, sc, p, sv, u, scal, o->wx, o->rec, hold_factor2, tol2, o->epoch + 1u, restart,
+              s.t, s.kc, s.dofp, res, sc, p, sv, u, scal, o->wx, o->rec, hold_factor2, tol2, o->epoch + 1u, c->res_polls, restart,
               lim, c->tune.time_kernels, {}};
   for (int i = 0; i < 8; ++i) a.kr.f[i] = (float)s.f[i];
   o->epoch += need;

@@ -9,7 +9,6 @@ constexpr int kResT = 512;              // threads per block
 constexpr int kResWaves = kResT / 64;
 constexpr int kResMaxBlocks = 256;      // one per CU
 constexpr int kResCopies = 8;           // copies of a block's record
-constexpr uint32_t kSpinLimit = 1u << 22;
 constexpr size_t kRecWords = (size_t)2 * kResCopies * 2 * kResMaxBlocks * 4;
 
 typedef unsigned int U4 __attribute__((ext_vector_type(4)));

@@ -92,7 +92,7 @@ struct ElemsArgs {
   Scal* s;
   uint32_t *wx, *rec;
   double hold2, tol2;
-  uint32_t epoch;
+  uint32_t epoch, polls;
   int restart, lim, time;
 };
 
@@ -105,6 +105,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
   __shared__ double red[2][2][kResWaves];
   __shared__ double tot[2][2][4];
   __shared__ int gaveup;
+  __shared__ uint32_t polls;                 // what a wait may take (in LDS: scalar registers are short)
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int b = blockIdx.x;
   const double rzp0 = a.s->rzp, rr0 = a.s->rr;
@@ -140,7 +141,11 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
     if (a.isc && a.isc[d]) pd = (X)(a.sc[d] * a.sc[d] * a.nzval[a.diag[d]]);
   }
   for (int i = t; i < kElMost * ST + V; i += kResT) re[i] = yl[i] = X(0);
-  if (t == 0) gaveup = 0;
+  if (t == 0) {
+    gaveup = 0;
+    polls = a.polls;
+  }
+  auto polls_left = [&]() { return (uint32_t)uniform((int)polls); };
   res_barrier();
   auto spread = [&]() {                      // r̂ to the rows of the cells
 #pragma unroll
@@ -194,7 +199,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
     if (halo && widest > 0) {          // (spare reads repeat a slot that is published)
       const uint32_t wi = (ep & 1u) * (uint32_t)a.nslots;
       typename LL<X>::W hv[kElShare];
-      for (uint32_t spin = 0;; ++spin) {
+      for (uint32_t left = polls_left();; --left) {
         asm volatile("" ::: "memory");
         bool ok = true;
         if (need) {
@@ -209,7 +214,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
           if (k < widest) ok = ok && LL<X>::ok(hv[k], ep);
         if (need) need = !(LL<double>::ok(q0, ep) && LL<double>::ok(q1, ep));
         if (ok) break;
-        if (spin >= kSpinLimit) { lost = true; break; }
+        if (left == 0) { lost = true; break; }
       }
       X sum = X(0);
 #pragma unroll
@@ -218,12 +223,12 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
       if (nfrom > 0) w = sum;
     }
     if (wave < (kResMaxBlocks + 63) / 64) {
-      for (uint32_t spin = 0; need; ++spin) {
+      for (uint32_t left = polls_left(); need; --left) {
         asm volatile("" ::: "memory");
         q0 = LL<double>::get(rr, rin);
         q1 = LL<double>::get(rr, rin + kResMaxBlocks);
         need = !(LL<double>::ok(q0, ep) && LL<double>::ok(q1, ep));
-        if (spin >= kSpinLimit) { lost = true; break; }
+        if (left == 0) { lost = true; break; }
       }
       const double s0 = wave_sum63(reader ? LL<double>::val(q0) : 0.0);
       const double s1 = wave_sum63(reader ? LL<double>::val(q1) : 0.0);
@@ -508,7 +513,7 @@ int elems_run(fem_ctx* c, ElemsOp* o, const double* res, const double* sc, X* p,
   const X* val = sizeof(X) == 4 ? reinterpret_cast<const X*>(o->val32) : reinterpret_cast<const X*>(o->val64);
   ElemsArgs<X> a{o->nb, std::max(1, o->nslots), o->cell, o->dof, o->pos, o->slot, o->from, o->nfrom, val,
                  c->ea_constrained ? c->d_isc : nullptr, c->d_diag, c->d_nzval, res, sc, p, sv, u, s, o->wx, o->rec,
-                 hold_factor2, tol2, o->epoch + 1u, restart, lim, c->tune.time_kernels};
+                 hold_factor2, tol2, o->epoch + 1u, c->res_polls, restart, lim, c->tune.time_kernels};
   o->epoch += need;
   const void* k = (const void*)k_resident_elems<X>;
   void* args[] = {&a};

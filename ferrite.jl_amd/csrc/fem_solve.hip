@@ -2822,6 +2822,12 @@ extern "C" int32_t fem_solve_kernels(const fem_ctx* c, int32_t* kernels, int32_t
   return FEM_OK;
 }
 
+extern "C" int32_t fem_set_wait_limit(fem_ctx* c, int32_t polls) {
+  if (!c) return FEM_ERR_ARG;
+  c->res_polls = polls < 0 ? kResPolls : (uint32_t)polls;
+  return FEM_OK;
+}
+
 // Average duration (HIP events) of `reps` back-to-back launches of the solver's SpMV
 // w = Â x (sliced operator, FP64 or FP32 values and vectors).
 extern "C" int32_t fem_spmv_bench(fem_ctx* c, int32_t mixed, int32_t reps, double* avg_ms) {

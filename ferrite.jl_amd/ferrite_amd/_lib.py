@@ -111,6 +111,7 @@ SIGNATURES = {
     "fem_apply_solution": (I32, [P, I32]),
     "fem_solve": (I32, [P, C.POINTER(SolveCfg), C.POINTER(SolveInfo)]),
     "fem_solve_kernels": (I32, [P, PI32, PI32]),
+    "fem_set_wait_limit": (I32, [P, I32]),
     "fem_matrix_download": (I32, [P, PD, PD]),
     "fem_matrix_upload": (I32, [P, PD, PD]),
     "fem_solution_download": (I32, [P, PD]),
@@ -134,6 +135,7 @@ SIGNATURES = {
     "fem_batch_run": (I32, [P, C.POINTER(BatchCfg), C.POINTER(BatchInfo)]),
     "fem_batch_problem_stats": (I32, [P, PD, PI32]),
     "fem_batch_problem_kernels": (I32, [P, PI32]),
+    "fem_batch_set_wait_limit": (I32, [P, I32]),
     "fem_batch_download": (I32, [P, I32, PD, PD, PD]),
     "fem_batch_assemble_only": (I32, [P, I32, I32, I32, PD]),
 }

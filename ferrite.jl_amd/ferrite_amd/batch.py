@@ -143,6 +143,10 @@ class BatchedPoisson:
         self._call("fem_batch_problem_kernels", L.ptr(kernels, C.c_int32))
         return BatchResult(info, ms, it, kernels)
 
+    def set_wait_limit(self, polls=-1):
+        """device.set_wait_limit for the launches of this batch."""
+        self._call("fem_batch_set_wait_limit", int(polls))
+
     def download(self, i):
         p = self.problems[i]
         nz = np.zeros(p["nnz"])

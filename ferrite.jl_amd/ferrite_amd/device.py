@@ -302,6 +302,12 @@ def solve(K, f, mode="cg", rtol=1e-10, maxit=0, precond="jacobi", inner_rtol=0.0
     return SolveResult(info, u, kernels.value, gave_up.value)
 
 
+def set_wait_limit(K, polls=-1):
+    """Polls after which a block of a one-launch solve stops waiting for another (-1: the default); the
+    solve then starts over on the separate kernels."""
+    K.ctx.call("fem_set_wait_limit", int(polls))
+
+
 def timings(K):
     t = L.Timings()
     K.ctx.call("fem_get_timings", C.byref(t))

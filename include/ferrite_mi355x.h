@@ -191,6 +191,9 @@ int32_t fem_solve(fem_ctx* ctx, const fem_solve_cfg* cfg, fem_solve_info* info);
  * for one of its blocks; solves then start over on the separate kernels, and stay on them
  * until fem_set_tuning or a new mesh, dofs or pattern.  Either pointer may be NULL. */
 int32_t fem_solve_kernels(const fem_ctx* ctx, int32_t* kernels, int32_t* gave_up);
+/* How long a block of a one-launch solve waits for a value of another block before it gives up:
+ * this many polls after the first, about a microsecond each (negative: the default, 4 million). */
+int32_t fem_set_wait_limit(fem_ctx* ctx, int32_t polls);
 
 /* ---- results ---- */
 int32_t fem_matrix_download(fem_ctx* ctx, double* nzval, double* f);

@@ -80,6 +80,9 @@ int32_t fem_batch_problem_stats(const fem_batch* b, double* completion_ms, int32
 /* Per problem of the last run the kernels that solved it: 1 the launch that several problems
  * share (the resident CG), 0 the separate kernels; array of length nproblems. */
 int32_t fem_batch_problem_kernels(const fem_batch* b, int32_t* kernels);
+/* fem_set_wait_limit for the launches of a batch; a batch in which one gave up stays on the
+ * separate kernels. */
+int32_t fem_batch_set_wait_limit(fem_batch* b, int32_t polls);
 
 /* Assembly only (zero + one launch per colour), timed with HIP events: *ms. */
 int32_t fem_batch_assemble_only(fem_batch* b, int32_t precision, int32_t cells_per_wg, int32_t chunk, double* ms);

@@ -124,6 +124,31 @@ def test_ends_without_convergence(nel, mode):
     _check(K, f, mode, "sell" if mode == "cg" else "lattice", "rows")
 
 
+@pytest.mark.parametrize("nel,forms,mode,kernels", [
+    ((40, 31), dict(lattice=-1, cell_operator=-1), "cg", "rows"), ((14, 13, 12), {}, "mixed", "rows"),
+    ((63, 64, 65), {}, "cg", "rows"), ((90, 84, 80), {}, "mixed", "bricks")])
+def test_gives_up(nel, forms, mode, kernels):
+    """A wait that runs out (no poll beyond the first allowed): every block leaves, the solve starts over on
+    the separate kernels, which are used from then on until the tuning is set."""
+    print("case resident gives up", nel, mode, flush=True)
+    K, f = _poisson(nel, False, **forms)
+    fa.set_wait_limit(K, 0)
+    _gives_up(K, f, mode, kernels)
+
+
+def _gives_up(K, f, mode, kernels):
+    for _ in range(2):
+        lost = fa.solve(K, f, mode=mode, rtol=1e-12)
+        assert lost.kernels == "separate" and lost.gave_up
+        fa.set_wait_limit(K)
+    A, b = K.to_scipy(), f.to_numpy()
+    assert np.linalg.norm(b - A @ lost.u) <= 2e-12 * np.linalg.norm(b)
+    fa.set_tuning(K)
+    back = fa.solve(K, f, mode=mode, rtol=1e-12)
+    assert back.kernels == kernels and not back.gave_up and back.operator == lost.operator
+    assert np.linalg.norm(back.u - lost.u) <= 1e-8 * np.linalg.norm(lost.u)
+
+
 @pytest.mark.parametrize("nel", [(40, 31), (14, 13, 12)])
 @pytest.mark.parametrize("delta", [0.5, 1e-3])
 def test_hand_overs(nel, delta):
@@ -200,6 +225,10 @@ def test_q2_elements(nel, precision):
     for mode in ("cg",) if nel == (60, 1, 1) else ("cg", "mixed"):
         fa.set_tuning(K, cg_elems=0)
         _check(K, f, mode, "elements", "separate" if nel == (13, 11, 11) else "elements")
+        if nel == (5, 4, 4):
+            fa.set_tuning(K, cg_elems=0)
+            fa.set_wait_limit(K, 0)
+            _gives_up(K, f, mode, "elements")
 
 
 @pytest.mark.parametrize("grids", [
@@ -233,4 +262,27 @@ def test_batch(grids):
         A = sp.csc_matrix((nz, p["rowval"] - 1, p["colptr"] - 1), shape=(p["ndofs"], p["ndofs"]))
         assert np.linalg.norm(f - A @ u) <= 1e-11 * np.linalg.norm(f) * 1.0001
         assert np.array_equal(u, us[1][i][2])
+    b.close()
+
+
+def test_batch_gives_up():
+    """The 2D problems are of one block each and wait for nobody; a block of the 3D ones gives up, and
+    the separate kernels solve those."""
+    print("case resident batch gives up", flush=True)
+    import scipy.sparse as sp
+    grids = [("Quadrilateral", (9, 8)), ("Hexahedron", (30, 31, 32)), ("Quadrilateral", (7, 7)), ("Hexahedron", (9, 8, 7))]
+    b = BatchedPoisson(0)
+    for i, (ct, nel) in enumerate(grids):
+        k = np.exp(np.random.default_rng(i).normal(0.0, 0.5, int(np.prod(nel))))
+        b.add(*poisson_problem(ct, nel, k))
+    b.finalize()
+    b.set_wait_limit(0)
+    for kernels in ([1, 0, 1, 0], [0, 0, 0, 0]):
+        res = b.run("mixed", rtol=1e-11)
+        assert res.converged == len(grids) and list(res.kernels) == kernels
+        b.set_wait_limit()
+        for i, p in enumerate(b.problems):
+            nz, f, u = b.download(i)
+            A = sp.csc_matrix((nz, p["rowval"] - 1, p["colptr"] - 1), shape=(p["ndofs"], p["ndofs"]))
+            assert np.linalg.norm(f - A @ u) <= 1e-11 * np.linalg.norm(f) * 1.0001
     b.close()
