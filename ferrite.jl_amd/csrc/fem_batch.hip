@@ -1061,10 +1061,11 @@ int plan_resident(fem_batch* B) {
     }
   }
   int rc;
-  if ((rc = dev_alloc(c, &B->d_rnode, c->ndofs))) return rc;
+  if ((rc = dev_alloc(c, &B->d_rnode, c->ndofs))) return no_memory(c, rc) ? FEM_OK : rc;
   FEM_HIP(c, hipMemcpy(B->d_rnode, node.data(), 4 * node.size(), hipMemcpyHostToDevice));
   for (BResident& r : B->res) {
-    if ((rc = dev_alloc(c, &r.d_prob, r.prob.size())) || (rc = dev_alloc(c, &r.d_in, 2 * r.prob.size()))) return rc;
+    if ((rc = dev_alloc(c, &r.d_prob, r.prob.size())) || (rc = dev_alloc(c, &r.d_in, 2 * r.prob.size())))
+      return no_memory(c, rc) ? FEM_OK : rc;
     FEM_HIP(c, hipMemcpy(r.d_prob, r.prob.data(), 4 * r.prob.size(), hipMemcpyHostToDevice));
   }
   B->res_state = 1;
@@ -1697,6 +1698,14 @@ int32_t fem_batch_problem_kernels(const fem_batch* B, int32_t* kernels) {
 }
 
 int32_t fem_batch_set_wait_limit(fem_batch* B, int32_t polls) { return B ? fem_set_wait_limit(B->c, polls) : FEM_ERR_ARG; }
+
+int32_t fem_batch_set_copy_limit(fem_batch* B, int64_t bytes) {
+  if (!B) return FEM_ERR_ARG;
+  FEM_HIP(B->c, hipStreamSynchronize(B->c->stream));
+  for (BResident& r : B->res) resident_free(&r.op);
+  B->c->copy_limit = bytes < 0 ? -1 : bytes;
+  return FEM_OK;
+}
 
 int32_t fem_batch_download(fem_batch* B, int32_t prob, double* nzval, double* f, double* u) {
   if (!B) return FEM_ERR_ARG;

@@ -190,6 +190,7 @@ struct fem_ctx {
   fem::DevError* d_err = nullptr;
   fem::SolverWork* solver = nullptr;
   int solve_kernels = -1;              // of the last solve (fem_solve_kernels)
+  int64_t copy_limit = -1;             // ... bytes of a buffer they may take (fem_set_copy_limit), −1: any
   uint32_t res_polls = fem::kResPolls; // one-launch solves: polls of a wait (fem_set_wait_limit)
 
   fem_timings timings{};

@@ -29,6 +29,21 @@ struct ResSource {
 
 struct ResOp;
 
+// Device memory of a one-launch solve.  It is optional: without it the separate kernels solve, so
+// what prepares one answers "does not fit" (no_memory) instead of failing.
+template <class T>
+int copy_alloc(fem_ctx* c, T** p, size_t n) {
+  if (c->copy_limit >= 0 && n * sizeof(T) > (size_t)c->copy_limit)
+    return set_error(c, FEM_ERR_OOM, "over the limit of fem_set_copy_limit");
+  return dev_alloc(c, p, n);
+}
+inline bool no_memory(fem_ctx* c, int rc) {
+  if (rc != FEM_ERR_OOM) return false;
+  (void)hipGetLastError();       // (of the hipMalloc)
+  c->err.clear();
+  return true;
+}
+
 // What the launch did for one system.
 struct ResState {
   double rr;                     // square of the true residual of u
@@ -46,7 +61,8 @@ int resident_blocks(int64_t rows, int widest, bool fp32);
 int resident_most_blocks(const fem_ctx* c);
 
 // Ready to run on `s` in FP32 or FP64 (structure once per pattern, values when K or the scaling
-// changed); *ok = false when the rows do not fit (the caller keeps the separate kernels).
+// changed); *ok = false when the rows do not fit, or memory for them is not to be had (the caller keeps
+// the separate kernels).
 int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok);
 
 // The whole solve K u = f from u = 0: the recurrence and its hand-overs (u, the FP64 residual, the

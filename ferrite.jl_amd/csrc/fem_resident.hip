@@ -1153,14 +1153,14 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
           node[d] = c->h_cell_nodes[e * npc + at[a]];
         }
       }
-    if ((rc = dev_alloc(c, &w.node, n))) return rc;
+    if ((rc = copy_alloc(c, &w.node, n))) return rc;
     FEM_HIP(c, hipMemcpy(w.node, node.data(), 4 * n, hipMemcpyHostToDevice));
     g.node = w.node;
     g.dim = c->sdim;
     for (int d = 0; d < 3; ++d) g.x[d] = c->d_x[d];
   }
   std::vector<double> geom(10 * ng);
-  if ((rc = dev_alloc(c, &w.geom, 10 * ng)) || (rc = dev_alloc(c, &w.sys, ng))) return rc;
+  if ((rc = copy_alloc(c, &w.geom, 10 * ng)) || (rc = copy_alloc(c, &w.sys, ng))) return rc;
   FEM_HIP(c, hipMemcpyAsync(w.sys, sys.data(), sizeof(ResSystem) * ng, hipMemcpyHostToDevice, c->stream));
   k_res_geom<<<ng, 1024, 0, c->stream>>>(g, rows, w.sys, nz, w.geom);
   FEM_HIP(c, hipGetLastError());
@@ -1195,11 +1195,11 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   o->nb = nb;
   const int grid = (int)std::min<int64_t>(2048, (n + 255) / 256);
   const int gridy = (int)std::max<int64_t>(1, std::min<int64_t>(2048 / ng, (longest + 255) / 256));
-  if ((rc = dev_alloc(c, &w.part, n)) || (rc = dev_alloc(c, &w.hist, (size_t)kResBins * nb)) ||
-      (rc = dev_alloc(c, &w.flag, n)) || (rc = dev_alloc(c, &w.size, 2 * nb)) || (rc = dev_alloc(c, &w.rank, n)) ||
-      (rc = dev_alloc(c, &w.cnt, nb)) || (rc = dev_alloc(c, &w.slab, nb)) || (rc = dev_alloc(c, &o->grp, nb)) ||
-      (rc = dev_alloc(c, &o->oofs, nb + 1)) || (rc = dev_alloc(c, &o->pofs, nb + 1)) ||
-      (rc = dev_alloc(c, &o->hoff, nb + 1)))
+  if ((rc = copy_alloc(c, &w.part, n)) || (rc = copy_alloc(c, &w.hist, (size_t)kResBins * nb)) ||
+      (rc = copy_alloc(c, &w.flag, n)) || (rc = copy_alloc(c, &w.size, 2 * nb)) || (rc = copy_alloc(c, &w.rank, n)) ||
+      (rc = copy_alloc(c, &w.cnt, nb)) || (rc = copy_alloc(c, &w.slab, nb)) || (rc = copy_alloc(c, &o->grp, nb)) ||
+      (rc = copy_alloc(c, &o->oofs, nb + 1)) || (rc = copy_alloc(c, &o->pofs, nb + 1)) ||
+      (rc = copy_alloc(c, &o->hoff, nb + 1)))
     return rc;
   FEM_HIP(c, hipMemcpyAsync(w.sys, sys.data(), sizeof(ResSystem) * ng, hipMemcpyHostToDevice, c->stream));
   FEM_HIP(c, hipMemcpyAsync(o->grp, grp.data(), sizeof(int4) * nb, hipMemcpyHostToDevice, c->stream));
@@ -1244,7 +1244,7 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   while (pow2 < o->Rmax) pow2 *= 2;
   o->Rp = (o->Rmax + 63) / 64 * 64;
   FEM_HIP(c, hipMemcpyAsync(o->oofs, off.data(), 4 * (nb + 1), hipMemcpyHostToDevice, c->stream));
-  if ((rc = dev_alloc(c, &o->orow, off[nb]))) return rc;
+  if ((rc = copy_alloc(c, &o->orow, off[nb]))) return rc;
   k_res_gather<<<grid, 256, 0, c->stream>>>(n, w.part, w.flag, o->oofs, w.size + nb, o->orow);
   k_res_sort<<<nb, 1024, 4 * pow2, c->stream>>>(pow2, o->oofs, o->orow, w.rank, w.cnt);
   FEM_HIP(c, hipGetLastError());
@@ -1268,16 +1268,17 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   o->nlocmax += o->nlocmax & 1;             // keeps what follows r̂ and its zero slot apart
   if (o->nlocmax > 65535) return FEM_OK;    // positions are 16 bits (and byte offsets: res_lds_rows)
   const int nz2 = (nz + 1) / 2;
-  if ((rc = dev_alloc(c, &o->hrow, hof[nb])) || (rc = dev_alloc(c, &o->hslot, hof[nb])) ||
-      (rc = dev_alloc(c, &o->ai, (size_t)nb * nz2 * o->Rp)) || (rc = dev_alloc(c, &o->wx, (size_t)8 * o->nslots)) ||
-      (rc = dev_alloc(c, &o->wu, (size_t)4 * o->nslots)) || (rc = dev_alloc(c, &o->rec, kRecWords)))
+  if ((rc = copy_alloc(c, &o->hrow, hof[nb])) || (rc = copy_alloc(c, &o->hslot, hof[nb])) ||
+      (rc = copy_alloc(c, &o->ai, (size_t)nb * nz2 * o->Rp)) || (rc = copy_alloc(c, &o->wx, (size_t)8 * o->nslots)) ||
+      (rc = copy_alloc(c, &o->wu, (size_t)4 * o->nslots)) || (rc = copy_alloc(c, &o->rec, kRecWords)))
     return rc;
   FEM_HIP(c, hipMemcpyAsync(o->pofs, pub.data(), 4 * (nb + 1), hipMemcpyHostToDevice, c->stream));
   FEM_HIP(c, hipMemcpyAsync(o->hoff, hof.data(), 4 * (nb + 1), hipMemcpyHostToDevice, c->stream));
   FEM_HIP(c, hipMemsetAsync(o->wx, 0, (size_t)32 * o->nslots, c->stream));
   FEM_HIP(c, hipMemsetAsync(o->wu, 0, (size_t)16 * o->nslots, c->stream));
   FEM_HIP(c, hipMemsetAsync(o->rec, 0, 4 * kRecWords, c->stream));
-  FEM_HIP(c, hipHostMalloc((void**)&o->st, sizeof(ResState) * ng, hipHostMallocDefault));
+  if (hipHostMalloc((void**)&o->st, sizeof(ResState) * ng, hipHostMallocDefault) != hipSuccess)
+    return set_error(c, FEM_ERR_OOM, "hipHostMalloc failed");
   k_res_fill<<<nb, 256, lds, c->stream>>>(rows, nz, o->Rp, words, w.sys, o->grp, w.part, w.rank, o->oofs, o->orow,
                                           o->pofs, o->hoff, o->hrow, o->hslot, o->ai);
   FEM_HIP(c, hipGetLastError());
@@ -1296,10 +1297,7 @@ static int res_lds_rows(const ResOp* o, bool fp32, int maxlds) {
   return base + rest * per > cap ? -1 : rest;
 }
 
-int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok) {
-  *ok = false;
-  if (!*op) *op = new ResOp();
-  ResOp* o = *op;
+static int res_prepare(fem_ctx* c, ResOp* o, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok) {
   if (o->state == -1) return FEM_OK;
   ResRows rows{s.src, s.dim, s.n, s.npad, s.px, s.pxy, c->d_colptr, c->d_rowval, s.dofp, s.map, c->d_nzval, sc, s.kc, s.val,
                s.t, {}};
@@ -1323,8 +1321,8 @@ int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* s
     return FEM_OK;
   const int pi = fp32 ? 0 : 1;
   const size_t len = (size_t)o->nb * o->nz * o->Rp;
-  if (fp32 && !o->val32 && ((rc = dev_alloc(c, &o->val32, len)) || (rc = dev_alloc(c, &o->raw, len)))) return rc;
-  if (!fp32 && !o->val64 && (rc = dev_alloc(c, &o->val64, len))) return rc;
+  if (fp32 && !o->val32 && ((rc = copy_alloc(c, &o->val32, len)) || (rc = copy_alloc(c, &o->raw, len)))) return rc;
+  if (!fp32 && !o->val64 && (rc = copy_alloc(c, &o->val64, len))) return rc;
   if (o->ver[pi] != c->nzval_version + 1 || o->aux[pi] != c->aux_version + 1 || o->jac[pi] != jacobi ||
       o->vsrc[pi] != s.src) {
     const int g = (int)std::min<int64_t>(8192, ((int64_t)o->nb * o->Rp + 255) / 256);
@@ -1339,6 +1337,17 @@ int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* s
     o->vsrc[pi] = s.src;
   }
   *ok = true;
+  return FEM_OK;
+}
+
+int resident_prepare(fem_ctx* c, ResOp** op, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok) {
+  *ok = false;
+  if (!*op) *op = new ResOp();
+  const int rc = res_prepare(c, *op, s, sc, jacobi, fp32, ok);
+  if (!no_memory(c, rc)) return rc;
+  resident_free(op);
+  *op = new ResOp();
+  (*op)->state = -1;
   return FEM_OK;
 }
 

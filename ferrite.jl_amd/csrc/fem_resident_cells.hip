@@ -500,10 +500,7 @@ bool brick_cut(int nx, int ny, int nz, int most, int maxlds, int* cut) {
   return best < 1e300;
 }
 
-int brick_prepare(fem_ctx* c, BrickOp** op, int nx, int ny, int nz, bool* ok) {
-  *ok = false;
-  if (!*op) *op = new BrickOp();
-  BrickOp* o = *op;
+static int brick_build(fem_ctx* c, BrickOp* o, int nx, int ny, int nz, bool* ok) {
   if (o->state == 0) {
     o->state = -1;
     int ncu = 0, maxlds = 0, coop = 0;
@@ -521,13 +518,24 @@ int brick_prepare(fem_ctx* c, BrickOp** op, int nx, int ny, int nz, bool* ok) {
     o->slots = 2 * bx * by + bz * (2 * bx + 2 * by);
     o->lds = brick_lds_bytes(by, bz);
     int rc;
-    if ((rc = dev_alloc(c, &o->wx, (size_t)4 * o->nb * o->slots)) || (rc = dev_alloc(c, &o->rec, kRecWords))) return rc;
+    if ((rc = copy_alloc(c, &o->wx, (size_t)4 * o->nb * o->slots)) || (rc = copy_alloc(c, &o->rec, kRecWords))) return rc;
     FEM_HIP(c, hipMemsetAsync(o->wx, 0, (size_t)16 * o->nb * o->slots, c->stream));
     FEM_HIP(c, hipMemsetAsync(o->rec, 0, 4 * kRecWords, c->stream));
     o->epoch = 0;
     o->state = 1;
   }
   *ok = o->state == 1;
+  return FEM_OK;
+}
+
+int brick_prepare(fem_ctx* c, BrickOp** op, int nx, int ny, int nz, bool* ok) {
+  *ok = false;
+  if (!*op) *op = new BrickOp();
+  const int rc = brick_build(c, *op, nx, ny, nz, ok);
+  if (!no_memory(c, rc)) return rc;
+  brick_free(op);
+  *op = new BrickOp();
+  (*op)->state = -1;
   return FEM_OK;
 }
 

@@ -456,10 +456,10 @@ static int elems_build(fem_ctx* c, ElemsOp* o) {
         for (int k = 0; k < kElShare; ++k) from[((size_t)b * kElShare + k) * kResT + tt] = std::max(any, 0);
   }
   int rc;
-  if ((rc = dev_alloc(c, &o->cell, cell.size())) || (rc = dev_alloc(c, &o->dof, len)) ||
-      (rc = dev_alloc(c, &o->pos, pos.size())) || (rc = dev_alloc(c, &o->slot, len)) ||
-      (rc = dev_alloc(c, &o->from, from.size())) || (rc = dev_alloc(c, &o->nfrom, len)) ||
-      (rc = dev_alloc(c, &o->wx, (size_t)8 * nslots + 8)) || (rc = dev_alloc(c, &o->rec, kRecWords)))
+  if ((rc = copy_alloc(c, &o->cell, cell.size())) || (rc = copy_alloc(c, &o->dof, len)) ||
+      (rc = copy_alloc(c, &o->pos, pos.size())) || (rc = copy_alloc(c, &o->slot, len)) ||
+      (rc = copy_alloc(c, &o->from, from.size())) || (rc = copy_alloc(c, &o->nfrom, len)) ||
+      (rc = copy_alloc(c, &o->wx, (size_t)8 * nslots + 8)) || (rc = copy_alloc(c, &o->rec, kRecWords)))
     return rc;
   FEM_HIP(c, hipMemcpy(o->cell, cell.data(), 4 * cell.size(), hipMemcpyHostToDevice));
   FEM_HIP(c, hipMemcpy(o->dof, dof.data(), 4 * len, hipMemcpyHostToDevice));
@@ -476,16 +476,13 @@ static int elems_build(fem_ctx* c, ElemsOp* o) {
   return FEM_OK;
 }
 
-int elems_prepare(fem_ctx* c, ElemsOp** op, const double* sc, bool fp32, bool* ok) {
-  *ok = false;
-  if (!*op) *op = new ElemsOp();
-  ElemsOp* o = *op;
+static int elems_values(fem_ctx* c, ElemsOp* o, const double* sc, bool fp32, bool* ok) {
   int rc;
   if (o->state == 0 && (rc = elems_build(c, o))) return rc;
   if (o->state != 1) return FEM_OK;
   const size_t len = (size_t)o->nb * 81 * kResT;
-  if (fp32 && !o->val32 && (rc = dev_alloc(c, &o->val32, len))) return rc;
-  if (!fp32 && !o->val64 && (rc = dev_alloc(c, &o->val64, len))) return rc;
+  if (fp32 && !o->val32 && (rc = copy_alloc(c, &o->val32, len))) return rc;
+  if (!fp32 && !o->val64 && (rc = copy_alloc(c, &o->val64, len))) return rc;
   const uint8_t* isc = c->ea_constrained ? c->d_isc : nullptr;
   const dim3 g(o->nb, 3);
   if (fp32 && c->ea_fp64)
@@ -498,6 +495,17 @@ int elems_prepare(fem_ctx* c, ElemsOp** op, const double* sc, bool fp32, bool* o
     k_elems_vals<double, float><<<g, kResT, 0, c->stream>>>(o->cell, c->d_q2cnode, c->d_keq32, sc, isc, o->val64);
   FEM_HIP(c, hipGetLastError());
   *ok = true;
+  return FEM_OK;
+}
+
+int elems_prepare(fem_ctx* c, ElemsOp** op, const double* sc, bool fp32, bool* ok) {
+  *ok = false;
+  if (!*op) *op = new ElemsOp();
+  const int rc = elems_values(c, *op, sc, fp32, ok);
+  if (!no_memory(c, rc)) return rc;
+  elems_free(op);
+  *op = new ElemsOp();
+  (*op)->state = -1;
   return FEM_OK;
 }
 

@@ -2828,6 +2828,14 @@ extern "C" int32_t fem_set_wait_limit(fem_ctx* c, int32_t polls) {
   return FEM_OK;
 }
 
+extern "C" int32_t fem_set_copy_limit(fem_ctx* c, int64_t bytes) {
+  if (!c) return FEM_ERR_ARG;
+  FEM_HIP(c, hipStreamSynchronize(c->stream));
+  c->copy_limit = bytes < 0 ? -1 : bytes;
+  free_solver(c);
+  return FEM_OK;
+}
+
 // Average duration (HIP events) of `reps` back-to-back launches of the solver's SpMV
 // w = Â x (sliced operator, FP64 or FP32 values and vectors).
 extern "C" int32_t fem_spmv_bench(fem_ctx* c, int32_t mixed, int32_t reps, double* avg_ms) {

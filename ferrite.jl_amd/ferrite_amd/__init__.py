@@ -10,7 +10,7 @@ from .batch import BatchedPoisson, batch_sizes, make_batch
 from .constraints import (AffineConstraint, ConformityConstraint, ConstraintHandler, Dirichlet, PeriodicDirichlet,
                           collect_periodic_facets)
 from .device import (MI355XCSC, Context, ElasticityElement, PoissonElement, add_point_load, allocate_matrix,
-                     allocate_vector, apply, apply_solution, apply_traction, apply_zero, compliance_gradient, simp_modulus, assemble_global, get_tuning, set_cell_parameters, set_tuning, set_wait_limit, solve,
+                     allocate_vector, apply, apply_solution, apply_traction, apply_zero, compliance_gradient, simp_modulus, assemble_global, get_tuning, set_cell_parameters, set_copy_limit, set_tuning, set_wait_limit, solve,
                      spmv_bench, start_assemble, timings)
 from .dofs import DofHandler, add, add_constraint_entries, close, create_coloring, create_sparsity_pattern
 from .mesh import Grid, Hexahedron, NonConformingGrid, Quadrilateral, generate_grid
@@ -27,7 +27,7 @@ __all__ = [
     "add_constraint_entries", "apply_solution", "MI355XCSC", "Context", "ElasticityElement", "PoissonElement",
     "allocate_matrix", "allocate_vector", "apply", "apply_traction", "add_point_load", "compliance_gradient",
     "simp_modulus", "apply_zero", "assemble_global", "set_cell_parameters",
-    "solve", "spmv_bench", "set_tuning", "get_tuning", "set_wait_limit", "start_assemble", "timings", "DofHandler", "add", "close", "create_coloring",
+    "solve", "spmv_bench", "set_tuning", "get_tuning", "set_copy_limit", "set_wait_limit", "start_assemble", "timings", "DofHandler", "add", "close", "create_coloring",
     "create_sparsity_pattern", "Grid", "Hexahedron", "NonConformingGrid", "Quadrilateral", "generate_grid",
     "FacetQuadratureRule",
     "Lagrange", "QuadratureRule", "RefHexahedron", "RefLine", "RefQuadrilateral", "VectorizedInterpolation",

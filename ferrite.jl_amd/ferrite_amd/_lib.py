@@ -112,6 +112,7 @@ SIGNATURES = {
     "fem_solve": (I32, [P, C.POINTER(SolveCfg), C.POINTER(SolveInfo)]),
     "fem_solve_kernels": (I32, [P, PI32, PI32]),
     "fem_set_wait_limit": (I32, [P, I32]),
+    "fem_set_copy_limit": (I32, [P, I64]),
     "fem_matrix_download": (I32, [P, PD, PD]),
     "fem_matrix_upload": (I32, [P, PD, PD]),
     "fem_solution_download": (I32, [P, PD]),
@@ -136,6 +137,7 @@ SIGNATURES = {
     "fem_batch_problem_stats": (I32, [P, PD, PI32]),
     "fem_batch_problem_kernels": (I32, [P, PI32]),
     "fem_batch_set_wait_limit": (I32, [P, I32]),
+    "fem_batch_set_copy_limit": (I32, [P, I64]),
     "fem_batch_download": (I32, [P, I32, PD, PD, PD]),
     "fem_batch_assemble_only": (I32, [P, I32, I32, I32, PD]),
 }

@@ -147,6 +147,10 @@ class BatchedPoisson:
         """device.set_wait_limit for the launches of this batch."""
         self._call("fem_batch_set_wait_limit", int(polls))
 
+    def set_copy_limit(self, nbytes=-1):
+        """device.set_copy_limit for the launches of this batch."""
+        self._call("fem_batch_set_copy_limit", int(nbytes))
+
     def download(self, i):
         p = self.problems[i]
         nz = np.zeros(p["nnz"])

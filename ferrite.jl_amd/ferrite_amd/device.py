@@ -308,6 +308,12 @@ def set_wait_limit(K, polls=-1):
     K.ctx.call("fem_set_wait_limit", int(polls))
 
 
+def set_copy_limit(K, nbytes=-1):
+    """Largest device buffer a one-launch solve may take for its copy of the operator (-1: any); past it
+    the separate kernels solve."""
+    K.ctx.call("fem_set_copy_limit", int(nbytes))
+
+
 def timings(K):
     t = L.Timings()
     K.ctx.call("fem_get_timings", C.byref(t))

@@ -194,6 +194,10 @@ int32_t fem_solve_kernels(const fem_ctx* ctx, int32_t* kernels, int32_t* gave_up
 /* How long a block of a one-launch solve waits for a value of another block before it gives up:
  * this many polls after the first, about a microsecond each (negative: the default, 4 million). */
 int32_t fem_set_wait_limit(fem_ctx* ctx, int32_t polls);
+/* Bytes of the largest device buffer a one-launch solve may take for its copy of the operator
+ * (negative: any, the default).  Where the limit or the device's memory does not allow them, the
+ * separate kernels solve.  Drops the solver's copies, as fem_set_tuning does. */
+int32_t fem_set_copy_limit(fem_ctx* ctx, int64_t bytes);
 
 /* ---- results ---- */
 int32_t fem_matrix_download(fem_ctx* ctx, double* nzval, double* f);

@@ -83,6 +83,8 @@ int32_t fem_batch_problem_kernels(const fem_batch* b, int32_t* kernels);
 /* fem_set_wait_limit for the launches of a batch; a batch in which one gave up stays on the
  * separate kernels. */
 int32_t fem_batch_set_wait_limit(fem_batch* b, int32_t polls);
+/* fem_set_copy_limit for them. */
+int32_t fem_batch_set_copy_limit(fem_batch* b, int64_t bytes);
 
 /* Assembly only (zero + one launch per colour), timed with HIP events: *ms. */
 int32_t fem_batch_assemble_only(fem_batch* b, int32_t precision, int32_t cells_per_wg, int32_t chunk, double* ms);

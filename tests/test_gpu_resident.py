@@ -149,6 +149,28 @@ def _gives_up(K, f, mode, kernels):
     assert np.linalg.norm(back.u - lost.u) <= 1e-8 * np.linalg.norm(lost.u)
 
 
+@pytest.mark.parametrize("nel,mode,kernels,limit", [
+    ((40, 31), "cg", "rows", 0), ((14, 13, 12), "cg", "rows", 200_000), ((14, 13, 12), "mixed", "rows", 0),
+    ((14, 13, 12), "mixed", "rows", 200_000), ((90, 84, 80), "mixed", "bricks", 2_000_000)])
+def test_no_memory(nel, mode, kernels, limit):
+    """Memory for the copy of the operator is not to be had (none, or its tables but not its values): the
+    solve takes the separate kernels instead of failing, or bricks where those do fit."""
+    print("case resident no memory", nel, mode, limit, flush=True)
+    K, f = _poisson(nel, False)
+    _no_memory(K, f, mode, kernels, limit)
+
+
+def _no_memory(K, f, mode, kernels, limit):
+    A, b = K.to_scipy(), f.to_numpy()
+    small = "bricks" if mode == "mixed" and limit == 200_000 else "separate"
+    for nbytes, ran in ((limit, small), (-1, kernels)):
+        fa.set_copy_limit(K, nbytes)
+        for _ in range(2):
+            one = fa.solve(K, f, mode=mode, rtol=1e-12)
+            assert one.kernels == ran and not one.gave_up
+            assert np.linalg.norm(b - A @ one.u) <= 2e-12 * np.linalg.norm(b)
+
+
 @pytest.mark.parametrize("nel", [(40, 31), (14, 13, 12)])
 @pytest.mark.parametrize("delta", [0.5, 1e-3])
 def test_hand_overs(nel, delta):
@@ -227,6 +249,8 @@ def test_q2_elements(nel, precision):
         _check(K, f, mode, "elements", "separate" if nel == (13, 11, 11) else "elements")
         if nel == (5, 4, 4):
             fa.set_tuning(K, cg_elems=0)
+            for limit in (0, 500_000):
+                _no_memory(K, f, mode, "elements", limit)
             fa.set_wait_limit(K, 0)
             _gives_up(K, f, mode, "elements")
 
@@ -266,8 +290,8 @@ def test_batch(grids):
 
 
 def test_batch_gives_up():
-    """The 2D problems are of one block each and wait for nobody; a block of the 3D ones gives up, and
-    the separate kernels solve those."""
+    """A launch that is not to be had: no memory for it, or a block of it gives up (the 2D problems
+    are of one block each and wait for nobody).  The separate kernels solve its problems."""
     print("case resident batch gives up", flush=True)
     import scipy.sparse as sp
     grids = [("Quadrilateral", (9, 8)), ("Hexahedron", (30, 31, 32)), ("Quadrilateral", (7, 7)), ("Hexahedron", (9, 8, 7))]
@@ -276,11 +300,13 @@ def test_batch_gives_up():
         k = np.exp(np.random.default_rng(i).normal(0.0, 0.5, int(np.prod(nel))))
         b.add(*poisson_problem(ct, nel, k))
     b.finalize()
-    b.set_wait_limit(0)
-    for kernels in ([1, 0, 1, 0], [0, 0, 0, 0]):
+    # memory for the 2D rows but not for the 3D ones; then the wait limit
+    for limit, polls, kernels in ((200_000, -1, [1, 0, 1, 0]), (0, -1, [0, 0, 0, 0]), (-1, -1, [1, 1, 1, 1]),
+                                  (-1, 0, [1, 0, 1, 0]), (-1, -1, [0, 0, 0, 0])):
+        b.set_copy_limit(limit)
+        b.set_wait_limit(polls)
         res = b.run("mixed", rtol=1e-11)
         assert res.converged == len(grids) and list(res.kernels) == kernels
-        b.set_wait_limit()
         for i, p in enumerate(b.problems):
             nz, f, u = b.download(i)
             A = sp.csc_matrix((nz, p["rowval"] - 1, p["colptr"] - 1), shape=(p["ndofs"], p["ndofs"]))
