@@ -21,7 +21,7 @@
 // every iteration is two launches for all problems, the short ones waiting at each hand-over for a
 // round trip of the host.
 // Those take the problems that do not fit a launch (more than 256 × 0.85 × 4096 rows in 2D,
-// 2048 in 3D; more than 27 entries per row) or stall in it.  There a problem stops updating once
+// 2048 in 3D; more than 27 entries per row), or stall in it, or whose launch cannot be prepared.  There a problem stops updating once
 // its FP64 residual meets its tolerance, and its completion time is taken from the batch boundary
 // at which that happened.  Their FP32 operator is a sliced ELL copy whose slices (≤ 64 rows, one
 // wave) never cross a reduction segment, so one block per segment runs its slices and sums its
@@ -1017,8 +1017,10 @@ int ensure_cg_graph(fem_batch* B, int width) {
   return FEM_OK;
 }
 
-// The problems shared out over launches of the resident CG: 2D and 3D apart (their rows have 9
-// and 27 entries), the largest first, as many as a launch holds.
+// The problems shared out over launches of the resident CG, the largest first, as many as a launch
+// holds: 2D and 3D apart (their rows have 9 and 27 entries), and those of a dimension together at
+// the room its widest rows need (9, 18 or 27 entries), except that what fits a launch only at
+// less goes into one of its own.  A problem with wider rows, or too large for a launch, is left out.
 int plan_resident(fem_batch* B) {
   fem_ctx* c = B->c;
   const int np_ = (int)B->probs.size();
@@ -1033,31 +1035,38 @@ int plan_resident(fem_batch* B) {
   }
   for (int dim = 2; dim <= 3; ++dim) {
     std::vector<int> left;
-    int widest = 0;
+    std::vector<int> widest(np_, 0);
     for (int p = 0; p < np_; ++p) {
       const BProblemHost& P = B->probs[p];
       if (P.dim != dim) continue;
       left.push_back(p);
-      for (int64_t j = 0; j < P.ndofs; ++j) widest = std::max(widest, P.colptr[j + 1] - P.colptr[j]);
+      for (int64_t j = 0; j < P.ndofs; ++j) widest[p] = std::max(widest[p], P.colptr[j + 1] - P.colptr[j]);
     }
     std::stable_sort(left.begin(), left.end(),
                      [&](int a, int b) { return B->probs[a].ndofs > B->probs[b].ndofs; });
-    for (size_t at = 0; at < left.size();) {
+    for (int room : {27, 18, 9}) {
+      if (std::none_of(left.begin(), left.end(), [&](int p) { return widest[p] <= room && widest[p] > room - 9; })) continue;
+      auto need = [&](int p) { return resident_blocks(B->probs[p].ndofs, room, true); };
+      auto fits = [&](int p) { return widest[p] <= room && need(p) <= resident_most_blocks(c); };
+      int blocks = 0;
       BResident r;
       r.dim = dim;
-      r.widest = widest;
-      int blocks = 0;
-      for (; at < left.size(); ++at) {
-        const int p = left[at], need = resident_blocks(B->probs[p].ndofs, widest, true);
-        if (need == 0) return FEM_OK;   // too large, or too many entries per row
-        if (blocks + need > resident_most_blocks(c)) break;
-        blocks += need;
+      r.widest = room;
+      for (int p : left) {
+        if (!fits(p)) continue;
+        if (blocks + need(p) > resident_most_blocks(c)) {
+          B->res.push_back(r);
+          r.prob.clear();
+          r.rows.clear();
+          blocks = 0;
+        }
+        blocks += need(p);
         r.prob.push_back(p);
         r.rows.push_back((int32_t)d0[p]);
         r.rows.push_back((int32_t)d0[p + 1]);
       }
-      if (r.prob.empty()) return FEM_OK;
-      B->res.push_back(r);
+      if (!r.prob.empty()) B->res.push_back(r);
+      left.erase(std::remove_if(left.begin(), left.end(), fits), left.end());
     }
   }
   int rc;

@@ -312,3 +312,38 @@ def test_batch_gives_up():
             A = sp.csc_matrix((nz, p["rowval"] - 1, p["colptr"] - 1), shape=(p["ndofs"], p["ndofs"]))
             assert np.linalg.norm(f - A @ u) <= 1e-11 * np.linalg.norm(f) * 1.0001
     b.close()
+
+
+def _fan(m):
+    """m quadrilaterals around one node, whose column has 2 m + 1 entries; u = 0 on two facets."""
+    ang = np.arange(2 * m) * (np.pi / m)
+    rad = np.where(np.arange(2 * m) % 2, 1.1, 1.0)
+    nodes = np.vstack([[0.0, 0.0], np.stack([rad * np.cos(ang), rad * np.sin(ang)], axis=1)])
+    cells = np.array([[1, 2 + 2 * i, 3 + 2 * i, 2 + (2 * i + 2) % (2 * m)] for i in range(m)])
+    g = fa.Grid("Quadrilateral", cells, nodes, {"edge": [(1, 2), (m // 2, 3)]})
+    dh = fa.DofHandler(g).add("u", fa.Lagrange(g.refshape, 1)).close()
+    ch = fa.ConstraintHandler(dh)
+    ch.add(fa.Dirichlet("u", g.facetsets["edge"], lambda x, t: 0.0)).close()
+    return g, dh, fa.create_coloring(g), ch, 1.0 + np.arange(m) / m
+
+
+def test_batch_of_which_some_do_not_fit():
+    """One problem with a column of 29 entries and one of 895 k rows among problems that fit: only those
+    two take the separate kernels.  One of 13 entries shares the launch of the 2D problems."""
+    print("case resident batch of which some do not fit", flush=True)
+    import scipy.sparse as sp
+    b = BatchedPoisson(0)
+    setups = [_fan(14)]
+    for ct, nel in (("Quadrilateral", (950, 940)), ("Quadrilateral", (40, 41)), ("Hexahedron", (9, 8, 7))):
+        setups.append(poisson_problem(ct, nel, np.exp(np.random.default_rng(1).normal(0.0, 0.3, int(np.prod(nel))))))
+    setups.append(_fan(6))
+    for s in setups:
+        b.add(*s)
+    b.finalize()
+    res = b.run("fp64", rtol=1e-9)
+    assert res.converged == 5 and list(res.kernels) == [0, 0, 1, 1, 1]
+    for i, p in enumerate(b.problems):
+        nz, f, u = b.download(i)
+        A = sp.csc_matrix((nz, p["rowval"] - 1, p["colptr"] - 1), shape=(p["ndofs"], p["ndofs"]))
+        assert np.linalg.norm(f) > 0 and np.linalg.norm(f - A @ u) <= 1e-9 * np.linalg.norm(f) * 1.0001
+    b.close()
