@@ -2611,7 +2611,7 @@ static int cg_run(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, double bnorm2, 
     Scal ht{};
     if ((rc = read_scal(c, w, &ht))) return rc;
     if (ht.rr <= tol2) { converged = true; break; }
-    stall = ht.rr > 0.81 * prev_true ? stall + 1 : 0;
+    stall = ht.rr <= 0.81 * prev_true ? 0 : stall + 1;   // (a NaN stalls)
     if (stall >= kMaxStall) break;
     prev_true = std::min(prev_true, ht.rr);
     reseed<X>(c, w, v, w->res, hold_factor2, tol2, 0);
@@ -2807,7 +2807,7 @@ extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_inf
   out.relres = std::sqrt(cg.rr / bnorm2);
   c->timings.solve_ms = cg.ms;
   if (info) *info = out;
-  if (out.relres > cfg->rtol * 1.0000001) {
+  if (!(out.relres <= cfg->rtol * 1.0000001)) {   // (a NaN did not converge)
     char buf[160];
     snprintf(buf, sizeof buf, "CG did not converge: relres %.3e after %d iterations", out.relres, out.iterations);
     return set_error(c, FEM_ERR_NOCONV, buf);

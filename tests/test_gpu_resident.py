@@ -172,6 +172,26 @@ def _no_memory(K, f, mode, kernels, limit):
 
 
 @pytest.mark.parametrize("nel", [(40, 31), (14, 13, 12)])
+@pytest.mark.parametrize("mode", ["cg", "mixed"])
+@pytest.mark.parametrize("cg_elems", [0, 8])
+@pytest.mark.parametrize("where,value", [("K", np.nan), ("K", np.inf), ("f", np.nan), ("f", np.inf)])
+def test_no_numbers(nel, mode, cg_elems, where, value):
+    """A NaN or an infinity in K or f: the solve ends and says that it did not converge."""
+    print("case resident no numbers", nel, mode, cg_elems, where, value, flush=True)
+    K, f = _poisson(nel, True, cg_elems=cg_elems)
+    if where == "K":
+        nz = K.nzval()
+        nz[K.nnz // 2] = value
+        K.set_nzval(nz)
+    else:
+        b = f.to_numpy()
+        b[len(b) // 2] = value
+        K.ctx.call("fem_matrix_upload", None, b.ctypes.data_as(ctypes.POINTER(ctypes.c_double)))
+    with pytest.raises(fa.FemConvergenceError, match="did not converge"):
+        fa.solve(K, f, mode=mode, rtol=1e-10, maxit=3200)
+
+
+@pytest.mark.parametrize("nel", [(40, 31), (14, 13, 12)])
 @pytest.mark.parametrize("delta", [0.5, 1e-3])
 def test_hand_overs(nel, delta):
     """Many hand-overs (δ = 0.5) and few."""
