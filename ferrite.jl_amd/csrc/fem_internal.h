@@ -67,7 +67,8 @@ struct Scal {
   // adds it)
   double xa0, xa1, pend;
   double rz0;     // γ at the last reseed (the host's batch-length choice)
-  // resident CG: products run, and (time_kernels) the 100 MHz clock ticks block 0 spent in them
+  // resident CG: products run, and (time_kernels) the 100 MHz clock ticks the largest brick spent
+  // in them (element matrices: the first block, whose products take as long as any)
   long long prod_ticks;
   int prods, pad2;
 };

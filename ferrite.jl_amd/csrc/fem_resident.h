@@ -52,7 +52,7 @@ struct ResState {
   int lost;                      // 1: a block gave up waiting for another one
   int prods;                     // products with Â run
   uint32_t epoch;                // exchange numbers used up to here
-  long long ticks, begin, end;   // 100 MHz clock: in block 0's products (time), the system's first and last
+  long long ticks, begin, end;   // 100 MHz clock: in the largest part's products (time), the system's first and last
 };
 
 // Fewest blocks that hold a system of several in a launch (0: its rows have too many entries), and

@@ -47,7 +47,7 @@ struct ResOp {
   // parts: one block each; own rows (those other parts read first, each class ascending),
   // coupled rows (ascending), published slots
   int nb = 0, ng = 0, Rmax = 0, Rp = 0, nz = 0, nlocmax = 0, nhmax = 0, nslots = 0;
-  int4* grp = nullptr;                  // [nb] system of each part, its first part, how many, 0
+  int4* grp = nullptr;                  // [nb] system of each part, its first part, how many, its largest
   int32_t* oofs = nullptr;              // [nb + 1] ranges of orow
   int32_t* orow = nullptr;              // own rows of each part
   int32_t* pofs = nullptr;              // [nb + 1] published slots: one per row other parts read
@@ -955,11 +955,11 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
     o->handovers = handovers;
     o->status = status;
     o->prods = prods;
-    o->ticks = ticks;
     o->begin = begin;
     o->end = wall_clock64();
     o->epoch = ep;
   }
+  if (b == z.grp[b].w && t == 0) o->ticks = ticks;
 }
 
 // ---- host ---------------------------------------------------------------------------------
@@ -1188,7 +1188,7 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   std::vector<int4> grp;
   for (int i = 0; i < ng; ++i) {
     const int m = cut[3 * i] * cut[3 * i + 1] * cut[3 * i + 2];
-    for (int k = 0; k < m; ++k) grp.push_back(make_int4(i, nb, m, 0));
+    for (int k = 0; k < m; ++k) grp.push_back(make_int4(i, nb, m, nb));
     if (m > 1 && !coop) return FEM_OK;
     nb += m;
   }
@@ -1202,7 +1202,6 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
       (rc = copy_alloc(c, &o->hoff, nb + 1)))
     return rc;
   FEM_HIP(c, hipMemcpyAsync(w.sys, sys.data(), sizeof(ResSystem) * ng, hipMemcpyHostToDevice, c->stream));
-  FEM_HIP(c, hipMemcpyAsync(o->grp, grp.data(), sizeof(int4) * nb, hipMemcpyHostToDevice, c->stream));
   FEM_HIP(c, hipMemsetAsync(w.part, 0xff, 4 * n, c->stream));
   FEM_HIP(c, hipMemsetAsync(w.flag, 0, n, c->stream));
   FEM_HIP(c, hipMemsetAsync(w.size, 0, 8 * nb, c->stream));
@@ -1238,7 +1237,10 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   for (int b = 0; b < nb; ++b) {
     off[b + 1] = off[b] + h[b];
     o->Rmax = std::max(o->Rmax, h[b]);
+    if (h[b] > h[grp[grp[b].y].w]) grp[grp[b].y].w = b;
   }
+  for (int b = 0; b < nb; ++b) grp[b].w = grp[grp[b].y].w;
+  FEM_HIP(c, hipMemcpyAsync(o->grp, grp.data(), sizeof(int4) * nb, hipMemcpyHostToDevice, c->stream));
   if (o->Rmax > 8192) return FEM_OK;
   int pow2 = 2;
   while (pow2 < o->Rmax) pow2 *= 2;

@@ -463,8 +463,8 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
     o->pend = 0.0;
     o->iters += it;
     o->prods += prods;
-    o->prod_ticks += ticks;
   }
+  if (b == nb - 1 && t == 0) z.s->prod_ticks += ticks;   // of the largest brick: the last along each axis
 }
 
 // LDS of bricks of at most by nodes along y and bz along z.

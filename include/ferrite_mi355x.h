@@ -229,7 +229,8 @@ typedef struct {
                                         spmv_launches): separate kernels are launched directly (no
                                         graph replay) with HIP events around every SpMV; where the
                                         whole recurrence runs in one launch, its products are timed
-                                        on the device's clock and counted */
+                                        on the device's clock, in the block with the most rows,
+                                        and counted */
   int32_t sell_unroll;               /* sliced-ELL SpMV: entries loaded per lane before their x
                                         gathers, 4 / 8 / 16 (0 = default: 8 FP32, 4 FP64) */
   int32_t sell_map;                  /* solver SpMV rows to blocks: 1 = grid-stride, 2 = contiguous,
