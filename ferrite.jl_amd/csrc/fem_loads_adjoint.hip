@@ -39,7 +39,8 @@ __device__ __forceinline__ void cross3(const double* u, const double* v, double*
 // point q, then lane I sums its entry over the points.  With one lane per facet a boundary of 728 Q2
 // facets was 728 lanes in a chain of 9 × 81 read-modify-writes of memory: 265 µs, now 25.
 constexpr int kFacetBlock = 128;
-__global__ __launch_bounds__(kFacetBlock) void k_facet_fe(const int32_t* __restrict__ fnum,
+constexpr int64_t kFacetGrid = 1 << 16;   // most blocks: a launch holds fewer than 2³² threads
+__global__ __launch_bounds__(kFacetBlock) void k_facet_fe(int64_t nf, const int32_t* __restrict__ fnum,
                                                           const int32_t* __restrict__ fnodes,
                                                           const double* __restrict__ X0,
                                                           const double* __restrict__ X1,
@@ -49,47 +50,49 @@ __global__ __launch_bounds__(kFacetBlock) void k_facet_fe(const int32_t* __restr
                                                           const double* __restrict__ tw, double t0, double t1,
                                                           double t2, int vdim, double* __restrict__ fe_out) {
   __shared__ double sdG[kMaxNFQ];
-  const int64_t k = blockIdx.x;
-  const int32_t fc = fnum[k];
-  for (int q = threadIdx.x; q < nfq; q += kFacetBlock) {
-    const int tq = fc * nfq + q;
-    double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-    for (int a = 0; a < ngeo; ++a) {
-      const int32_t nd = fnodes[k * ngeo + a];
-      const double x[3] = {X0[nd], X1[nd], sdim == 3 ? X2[nd] : 0.0};
-      for (int i = 0; i < sdim; ++i)
-        for (int j = 0; j < sdim; ++j) J[i][j] += x[i] * tdM[(tq * ngeo + a) * sdim + j];
-    }
-    double nrm;
-    if (sdim == 2) {
-      // facet_integrals.jl:122-131
-      double n0, n1;
-      switch (fc) {
-        case 0: n0 = J[1][0]; n1 = -J[0][0]; break;
-        case 1: n0 = J[1][1]; n1 = -J[0][1]; break;
-        case 2: n0 = -J[1][0]; n1 = J[0][0]; break;
-        default: n0 = -J[1][1]; n1 = J[0][1]; break;
+  for (int64_t k = blockIdx.x; k < nf; k += gridDim.x) {
+    const int32_t fc = fnum[k];
+    for (int q = threadIdx.x; q < nfq; q += kFacetBlock) {
+      const int tq = fc * nfq + q;
+      double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+      for (int a = 0; a < ngeo; ++a) {
+        const int32_t nd = fnodes[k * ngeo + a];
+        const double x[3] = {X0[nd], X1[nd], sdim == 3 ? X2[nd] : 0.0};
+        for (int i = 0; i < sdim; ++i)
+          for (int j = 0; j < sdim; ++j) J[i][j] += x[i] * tdM[(tq * ngeo + a) * sdim + j];
       }
-      nrm = sqrt(n0 * n0 + n1 * n1);
-    } else {
-      // facet_integrals.jl:191-202: column pairs (2,1) (1,3) (2,3) (3,1) (3,2) (1,2)
-      const int pa[6] = {1, 0, 1, 2, 2, 0}, pb[6] = {0, 2, 2, 0, 1, 1};
-      const double ca[3] = {J[0][pa[fc]], J[1][pa[fc]], J[2][pa[fc]]};
-      const double cb[3] = {J[0][pb[fc]], J[1][pb[fc]], J[2][pb[fc]]};
-      double n[3];
-      cross3(ca, cb, n);
-      nrm = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+      double nrm;
+      if (sdim == 2) {
+        // facet_integrals.jl:122-131
+        double n0, n1;
+        switch (fc) {
+          case 0: n0 = J[1][0]; n1 = -J[0][0]; break;
+          case 1: n0 = J[1][1]; n1 = -J[0][1]; break;
+          case 2: n0 = -J[1][0]; n1 = J[0][0]; break;
+          default: n0 = -J[1][1]; n1 = J[0][1]; break;
+        }
+        nrm = sqrt(n0 * n0 + n1 * n1);
+      } else {
+        // facet_integrals.jl:191-202: column pairs (2,1) (1,3) (2,3) (3,1) (3,2) (1,2)
+        const int pa[6] = {1, 0, 1, 2, 2, 0}, pb[6] = {0, 2, 2, 0, 1, 1};
+        const double ca[3] = {J[0][pa[fc]], J[1][pa[fc]], J[2][pa[fc]]};
+        const double cb[3] = {J[0][pb[fc]], J[1][pb[fc]], J[2][pb[fc]]};
+        double n[3];
+        cross3(ca, cb, n);
+        nrm = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
+      }
+      sdG[q] = nrm * tw[tq];
     }
-    sdG[q] = nrm * tw[tq];
-  }
-  __syncthreads();
-  const int ndpc = nbf * vdim;
-  for (int I = threadIdx.x; I < ndpc; I += kFacetBlock) {
-    const int a = I / vdim, d = I - a * vdim;
-    const double t = d == 0 ? t0 : d == 1 ? t1 : t2;
-    double fe = 0.0;
-    for (int q = 0; q < nfq; ++q) fe += t * tN[(fc * nfq + q) * nbf + a] * sdG[q];
-    fe_out[k * ndpc + I] = fe;
+    __syncthreads();
+    const int ndpc = nbf * vdim;
+    for (int I = threadIdx.x; I < ndpc; I += kFacetBlock) {
+      const int a = I / vdim, d = I - a * vdim;
+      const double t = d == 0 ? t0 : d == 1 ? t1 : t2;
+      double fe = 0.0;
+      for (int q = 0; q < nfq; ++q) fe += t * tN[(fc * nfq + q) * nbf + a] * sdG[q];
+      fe_out[k * ndpc + I] = fe;
+    }
+    __syncthreads();   // sdG was read
   }
 }
 
@@ -312,8 +315,9 @@ int32_t fem_facet_traction(fem_ctx* c, int64_t nfacets, const int64_t* facets, i
   const int32_t *dnodes = dnum + nfacets, *ddof = dnodes + nfacets * ngeo, *dptr = ddof + nd, *dsrc = dptr + nd + 1;
   double* dfe = c->d_facet + up / 8;
   const double t0 = traction[0], t1 = sdim > 1 ? traction[1] : 0.0, t2 = sdim > 2 ? traction[2] : 0.0;
-  k_facet_fe<<<(unsigned)nfacets, kFacetBlock, 0, st>>>(dnum, dnodes, c->d_x[0], c->d_x[1], c->d_x[2], sdim, nfq, nbf,
-                                                        ngeo, dN, dN + nN, dN + nN + ndM, t0, t1, t2, vdim, dfe);
+  k_facet_fe<<<(unsigned)std::min(nfacets, kFacetGrid), kFacetBlock, 0, st>>>(
+      nfacets, dnum, dnodes, c->d_x[0], c->d_x[1], c->d_x[2], sdim, nfq, nbf, ngeo, dN, dN + nN, dN + nN + ndM, t0, t1, t2,
+      vdim, dfe);
   k_facet_gather<<<(unsigned)((nd + 255) / 256), 256, 0, st>>>(nd, ddof, dptr, dsrc, dfe, c->d_f);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(st);

@@ -248,3 +248,30 @@ def test_torch_autograd_function():
     J2, dth, dx, _ = prob.compliance(theta, g.nodes.copy())
     assert np.allclose(th.grad.numpy(), 2 * dth, rtol=1e-14, atol=0)
     assert np.allclose(X.grad.numpy(), 2 * dx, rtol=1e-14, atol=0)
+
+
+@pytest.mark.parametrize("extra", [0, 77])
+def test_traction_on_more_facets_than_blocks(extra):
+    """65,536 facets and some more (a launch's blocks take several): the boundary of a small mesh over and
+    over, which must give that many times its traction."""
+    print("case traction on many facets", extra, flush=True)
+    g = fa.generate_grid("Quadrilateral", (12, 9), (0.0, 0.0), (2.0, 1.0))
+    ip = fa.Lagrange("RefQuadrilateral", 1) ** 2
+    dh = fa.DofHandler(g).add("u", ip).close()
+    K = fa.allocate_matrix(fa.MI355XCSC, dh)
+    f = fa.allocate_vector(K)
+    cv = fa.CellValues(fa.QuadratureRule("RefQuadrilateral", 2), ip)
+    fv = fa.FacetValues(fa.FacetQuadratureRule("RefQuadrilateral", 2), ip)
+    colors = fa.create_coloring(g)
+    edge = [x for n in ("left", "right", "bottom", "top") for x in g.facetsets[n]]
+
+    def load(facets):
+        fa.assemble_global(fa.start_assemble(K, f), cv, colors, fa.ElasticityElement(nu=0.3))
+        fa.apply_traction(K, f, fv, facets, (0.3, -1.0))
+        return f.to_numpy()
+
+    n = (1 << 16) + extra
+    whole, rest = n // len(edge), n % len(edge)
+    want = whole * load(edge) + load(edge[:rest])
+    got = load(edge * whole + edge[:rest])
+    assert np.linalg.norm(want) > 0 and _rel(got, want) <= 1e-11
