@@ -1116,7 +1116,7 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   }
   const int words = (int)((longest + 31) / 32);
   const int lds = 4 * (words + (words + 7) / 8);
-  if (lds > maxlds - 1024) return FEM_OK;   // a bitmap of the rows (more than a million): far too many anyway
+  if (lds > maxlds - kStaticLds) return FEM_OK;   // a bitmap of the rows (more than a million): far too many anyway
 
   struct Scratch {                          // freed on every way out
     int32_t *node = nullptr, *part = nullptr, *hist = nullptr, *size = nullptr, *rank = nullptr, *cnt = nullptr;
@@ -1255,8 +1255,8 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
   FEM_HIP(c, hipStreamSynchronize(c->stream));
   for (int b = 0; b < nb; ++b) pub[b + 1] = pub[b] + h[b];
   o->nslots = pub[nb];
-  (void)hipFuncSetAttribute((const void*)k_res_count, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * words);
-  (void)hipFuncSetAttribute((const void*)k_res_fill, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  (void)res_dynamic_lds((const void*)k_res_count, maxlds);
+  (void)res_dynamic_lds((const void*)k_res_fill, maxlds);
   k_res_count<<<nb, 256, 4 * words, c->stream>>>(rows, nz, words, w.sys, o->grp, w.part, o->oofs, o->orow, w.cnt);
   FEM_HIP(c, hipGetLastError());
   FEM_HIP(c, hipMemcpyAsync(h.data(), w.cnt, 4 * nb, hipMemcpyDeviceToHost, c->stream));
@@ -1293,7 +1293,7 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
 // Rows whose entries LDS holds: those beyond the register rows; −1 when they do not fit.
 static int res_lds_rows(const ResOp* o, bool fp32, int maxlds) {
   const size_t xb = fp32 ? 4 : 8, base = res_lds_bytes(o, xb, 0), per = o->nz * xb + 4 * ((o->nz + 1) / 2 | 1);
-  const size_t cap = (size_t)maxlds - 1024;
+  const size_t cap = (size_t)maxlds - kStaticLds;
   if (base > cap || (o->nlocmax + 1) * xb > 65536) return -1;   // 16-bit byte offsets into r̂
   const int rest = std::max(0, o->Rmax - res_register_rows(o->nz, fp32));
   return base + rest * per > cap ? -1 : rest;
@@ -1408,7 +1408,7 @@ int resident_run(fem_ctx* c, ResOp* o, const ResSource& s, const double* sc, con
   std::fill(o->st, o->st + o->ng, ResState{});
   const void* k = res_kernel<X>(o->nz, o->Rmax);
   const size_t lds = res_lds_bytes(o, sizeof(X), nl);
-  FEM_HIP(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  FEM_HIP(c, res_dynamic_lds(k, maxlds));
   void* args[] = {&a};
   const hipError_t e = o->nb == o->ng ? hipLaunchKernel(k, dim3(o->nb), dim3(kResT), args, lds, c->stream)
                                       : hipLaunchCooperativeKernel(k, dim3(o->nb), dim3(kResT), args, (unsigned)lds,

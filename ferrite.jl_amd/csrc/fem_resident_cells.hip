@@ -490,7 +490,7 @@ bool brick_cut(int nx, int ny, int nz, int most, int maxlds, int* cut) {
         if (lo[0] < 2 || lo[1] < 2 || lo[2] < 2) continue;
         if (hi[0] > kBrickX || hi[0] * hi[1] > kResT || hi[2] > kBrickZ) continue;
         const int around = 2 * (hi[0] + 2) * (hi[1] + 2) + (2 * (hi[0] + 2) + 2 * hi[1]) * hi[2];
-        if (around > kBrickH * kResT || brick_lds_bytes(hi[1], hi[2]) > maxlds - 1024) continue;
+        if (around > kBrickH * kResT || brick_lds_bytes(hi[1], hi[2]) > maxlds - kStaticLds) continue;
         const double cost = (double)((hi[0] * hi[1] + 63) / 64) * hi[2] * 1e4 + around;
         if (cost < best) {
           best = cost;
@@ -554,7 +554,9 @@ int brick_run(fem_ctx* c, BrickOp* o, const BrickSource& s, const double* res, c
   for (int i = 0; i < 8; ++i) a.kr.f[i] = (float)s.f[i];
   o->epoch += need;
   const void* k = (const void*)k_resident_cells;
-  FEM_HIP(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, o->lds));
+  int maxlds = 0;
+  FEM_HIP(c, hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
+  FEM_HIP(c, res_dynamic_lds(k, maxlds));
   void* args[] = {&a};
   const hipError_t e =
       hipLaunchCooperativeKernel(k, dim3(o->nb), dim3(kResT), args, (unsigned)o->lds, c->stream);

@@ -9,7 +9,14 @@ constexpr int kResT = 512;              // threads per block
 constexpr int kResWaves = kResT / 64;
 constexpr int kResMaxBlocks = 256;      // one per CU
 constexpr int kResCopies = 8;           // copies of a block's record
+constexpr int kStaticLds = 1024;        // left for a kernel's static LDS; the rest of the device's limit may be dynamic
 constexpr size_t kRecWords = (size_t)2 * kResCopies * 2 * kResMaxBlocks * 4;
+
+// Lets a kernel take all the dynamic LDS there is.  The attribute belongs to the kernel, not to a
+// launch: a value per launch would let one host thread lower it under the launch of another.
+inline hipError_t res_dynamic_lds(const void* kernel, int maxlds) {
+  return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, maxlds - kStaticLds);
+}
 
 typedef unsigned int U4 __attribute__((ext_vector_type(4)));
 typedef unsigned int U2 __attribute__((ext_vector_type(2)));

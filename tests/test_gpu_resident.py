@@ -334,6 +334,25 @@ def test_batch_gives_up():
     b.close()
 
 
+def test_contexts_on_threads():
+    """Contexts on host threads of their own, whose one-launch solves want different amounts of LDS of
+    the same kernels: each gets the u it gets alone, by the same kernels."""
+    print("case resident contexts on threads", flush=True)
+    from concurrent.futures import ThreadPoolExecutor
+    systems = [(_poisson(nel, False), mode) for nel, mode in (
+        ((24, 20, 17), "cg"), ((60, 58, 56), "cg"), ((47, 43, 41), "mixed"), ((14, 13, 12), "mixed"))]
+    alone = [fa.solve(K, f, mode=mode, rtol=1e-11).u for (K, f), mode in systems]
+
+    def repeat(i):
+        (K, f), mode = systems[i]
+        return [fa.solve(K, f, mode=mode, rtol=1e-11) for _ in range(20)]
+
+    with ThreadPoolExecutor(len(systems)) as pool:
+        for i, results in enumerate(pool.map(repeat, range(len(systems)))):
+            for r in results:
+                assert r.kernels == "rows" and not r.gave_up and np.array_equal(r.u, alone[i])
+
+
 def _fan(m):
     """m quadrilaterals around one node, whose column has 2 m + 1 entries; u = 0 on two facets."""
     ang = np.arange(2 * m) * (np.pi / m)
