@@ -38,7 +38,7 @@ struct DevError {
   int detj_cell;     // cell id (0-based) with det(J) <= 0, INT_MAX if none
   int pattern_cell;  // cell id with a nonzero value for a missing pattern entry
   int pattern_entry; // local entry (col * nb + row) of that cell (valid when pattern_cell set)
-  int pad;        // 1: the resident CG gave up waiting for another block
+  int pad;
 };
 
 struct SolverWork;
@@ -61,7 +61,7 @@ struct Scal {
   int restart;    // breakdown happened: the next reseed restarts p = r̂
   int fresh;      // p, s = Â p and α were just set by a reseed: the next step only moves x̂, r̂
   int sfresh;     // (record written by k_cg_scal) the step k_cg_move runs now is such a step
-  int pad;        // 1: the resident CG gave up waiting for another block
+  int gave_up;    // 1: a block of a one-launch stretch stopped waiting for another one
   // x̂ moves every other step: k_cg_move adds xa0 p_old + xa1 p_new (both 0: x̂ is not touched
   // and α p of this step is pending); pend = the α whose step's p is not yet in x̂ (k_fold
   // adds it)

@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
   }
   const BrickArgs& z = *reinterpret_cast<const BrickArgs*>(res_kernargs());
   if (!ok) {
-    if (t == 0) z.s->pad = 1;
+    if (t == 0) z.s->gave_up = 1;
     return;
   }
   if (mine) {
@@ -448,7 +448,7 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
     }
   }
   if (b == 0 && t == 0) {
-    Scal* o = z.s;                // all but pad, which a block that gave up sets
+    Scal* o = z.s;                // all but gave_up
     o->rz = rz;
     o->rz0 = rz0;
     o->rzp = rzp;

@@ -328,7 +328,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
     res_barrier();
   }
   if (!ok) {
-    if (t == 0) a.s->pad = 1;
+    if (t == 0) a.s->gave_up = 1;
     return;
   }
   if (own) {
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
     a.u[d] += a.sc[d] * (double)x;
   }
   if (b == 0 && t == 0) {
-    Scal* o = a.s;                // all but pad, which a block that gave up sets
+    Scal* o = a.s;                // all but gave_up
     o->rz = rz;
     o->rz0 = rz0;
     o->rzp = rzp;

@@ -27,11 +27,12 @@
 //
 // Reductions are fence-free and fixed-order: blocks write partials that the next kernel
 // sums (by default one block, k_cg_scal), in the same order every time, so results are
-// bitwise reproducible and the host never sits in the iteration.  Systems whose rows fit the
-// chip's registers and LDS run the whole recurrence in one launch per hand-over instead
-// (fem_resident.hip).  Otherwise a batch of iterations is
-// captured once into a hipGraph and replayed; kernels launched past a hand-over return at
-// once on the device flag.
+// bitwise reproducible and the host never sits in the iteration.  Systems that fit the
+// chip's registers and LDS run the recurrence without launches in between: on the rows' entries
+// the whole solve, hand-overs included, is one launch (fem_resident.hip); bricks of the cell form
+// (fem_resident_cells.hip) and Q2 element matrices (fem_resident_elems.hip) take one launch per
+// stretch between two hand-overs.  Otherwise a batch of iterations is captured once into a
+// hipGraph and replayed; kernels launched past a hand-over return at once on the device flag.
 #include <cmath>
 #include <cstring>
 
@@ -2693,7 +2694,7 @@ static int cg_run_stretches(fem_ctx* c, SolverWork* w, const CgVecs<X>& v, doubl
     residual(c, w);
     FEM_HIP(c, hipGetLastError());
     if ((rc = read_scal(c, w, &h))) return rc;
-    if (h.pad) {
+    if (h.gave_up) {
       *gave_up = true;
       return FEM_OK;
     }
