@@ -27,9 +27,10 @@
 // publishing, so every other block gives up too, and the host runs the separate kernels.
 //
 // Measured, µs per iteration, separate kernels → here: 100×100 Q1 quads FP64 11.7 → 3.0 (21
-// blocks); 24×20×17 distorted hexes FP64 17.4 → 3.6 (24); 64³ hexes FP64 33 → 6.4 (250); 512×256
-// Q1² quads FP64 26.5 → 4.0 (180); 301×227 Q1 quads FP32 cell form 13.3 → 3.75 and 47×53×61 hexes
-// FP32 planes 16.2 → 5.9 (both with their hand-overs).  At 100×100 an iteration is about 0.25 µs of
+// blocks); 24×20×17 distorted hexes FP64 17.4 → 3.6 (24); 64³ hexes FP64 33 → 6.3 (216); 512×256
+// Q1² quads FP64 26.5 → 4.0 (180); 301×227 Q1 quads FP32 cell form 13.3 → 3.6 (140) and 47×53×61
+// hexes FP32 planes 16.2 → 5.9 (both with their hand-overs).  Vector units busy 25% (64³) to 34%
+// (301×227), LDS 25% and 9%: the exchange's latency is what is left.  At 100×100 an iteration is about 0.25 µs of
 // products, 0.3 µs of sums inside the block, 1.3 µs until the other blocks' values are there and
 // 0.5 µs of scalars and vector moves.
 #include <algorithm>

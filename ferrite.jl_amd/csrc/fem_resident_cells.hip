@@ -10,11 +10,12 @@
 // planes below carried in registers, as in k_cell_spmv_z.  A node on the brick's surface is
 // published as soon as the march has it, so most values have arrived when the march ends.
 //
-// What bounds it: at 128³ (252 bricks of up to 22 × 22 × 19 nodes) an iteration takes 11.3 µs, 5 of
-// them the march (60 vector instructions a node, four cycles each without packed FP32, on two
-// waves per SIMD; 13 LDS words a node, with bank conflicts where a wave's columns wrap to the next
-// row of the brick), about 4 until the values of the other blocks are there (2,900 published values
-// of 8 bytes a block), the rest sums, scalars and vector moves.  No vector or coefficient is read
+// What bounds it: at 128³ (252 bricks of up to 22 × 22 × 19 nodes) an iteration takes 11 µs, 4.4 of
+// them the march (four cycles a vector instruction without packed FP32, on two waves per SIMD; 13
+// LDS words a node, with bank conflicts where a wave's columns wrap to the next row of the brick),
+// about 4 until the values of the other blocks are there (2,900 published values of 8 bytes a
+// block), the rest sums, scalars and vector moves.  Counters over a solve: 104 vector instructions per
+// 64 nodes and iteration in all, vector units busy 58%, LDS 42% (42% of that bank conflicts).  No vector or coefficient is read
 // from memory between two hand-overs.  The separate kernels (k_cell_spmv_z and k_cg_move_scal)
 // took 24–27 µs; whole mixed solve at 128³ 17.4 → 7.1 ms, at 90×84×80 8.9 → 3.85 ms.
 // Measured on the way: plane loads issued in the step that uses them 18.6 µs an iteration, one step

@@ -1,4 +1,4 @@
-"""Batched assembly + solve (one persistent work-queue kernel, batched mixed CG) vs the oracle.
+"""Batched assembly + solve (one launch per colour; mixed CG, several problems a launch) vs the oracle.
 
 Every problem of a batch must match the oracle's serial loop for that problem alone
 (heat_equation.jl:186-218 with per-cell k): FP64 element path K and f within 1e-12
