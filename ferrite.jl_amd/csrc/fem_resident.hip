@@ -964,9 +964,9 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
 }
 
 // ---- host ---------------------------------------------------------------------------------
-// Most rows per block of the instantiated kernels (FP64 with 27 entries: what LDS holds besides).
+// Most rows per block of the instantiated kernels (FP64 with 27 entries: LDS holds fewer, about 1,400).
 static int res_most_rows(int nz, bool fp32) {
-  return fp32 ? (nz == 9 ? 4096 : nz == 18 ? 2560 : 2048) : (nz == 9 ? 2048 : nz == 18 ? 1536 : 1400);
+  return fp32 ? (nz == 9 ? 4096 : nz == 18 ? 2560 : 2048) : (nz == 9 ? 2048 : 1536);
 }
 
 static int res_entries(int widest) { return widest <= 9 ? 9 : widest <= 18 ? 18 : 27; }
@@ -1300,6 +1300,23 @@ static int res_lds_rows(const ResOp* o, bool fp32, int maxlds) {
   return base + rest * per > cap ? -1 : rest;
 }
 
+// Whether `rows` rows may fit in this precision: the fullest block has at least its share of them,
+// and, in a mesh with little boundary (26 of 27 entries per row on average), no fewer coupled rows than
+// a cube.
+static bool res_may_fit(const fem_ctx* c, int64_t rows, int nz, bool fp32, bool one) {
+  const int blocks = resident_most_blocks(c);
+  if (rows > (int64_t)blocks * res_most_rows(nz, fp32)) return false;
+  if (!one || nz != 27 || c->nnz < 26 * rows) return true;
+  int maxlds = 0;
+  (void)hipDeviceGetAttribute(&maxlds, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device);
+  ResOp e;
+  e.nz = nz;
+  e.Rmax = (int)((rows + blocks - 1) / blocks);
+  e.nhmax = (int)(std::pow(std::cbrt((double)e.Rmax) + 2.0, 3.0) - e.Rmax);
+  e.nlocmax = e.Rmax + e.nhmax;
+  return res_lds_rows(&e, fp32, maxlds) >= 0;
+}
+
 static int res_prepare(fem_ctx* c, ResOp* o, const ResSource& s, const double* sc, int jacobi, bool fp32, bool* ok) {
   if (o->state == -1) return FEM_OK;
   ResRows rows{s.src, s.dim, s.n, s.npad, s.px, s.pxy, c->d_colptr, c->d_rowval, s.dofp, s.map, c->d_nzval, sc, s.kc, s.val,
@@ -1308,11 +1325,12 @@ static int res_prepare(fem_ctx* c, ResOp* o, const ResSource& s, const double* s
   int rc;
   if (o->state == 0) {
     const int widest = s.widest;
-    const int nz = res_entries(widest), most = res_most_rows(nz, fp32);
-    int64_t all = s.nsys > 0 ? 0 : s.n;
+    const int nz = res_entries(widest);
+    int64_t all = s.nsys > 0 ? 0 : c->n;    // (s.n counts a lattice's padding too)
     for (int i = 0; i < s.nsys; ++i) all += s.sys[2 * i + 1] - s.sys[2 * i];
-    // clearly too large in this precision (lattice rows include some padding): nothing is built
-    if (widest > 27 || all < 1 || all > (int64_t)kResMaxBlocks * most * 5 / 4) return FEM_OK;
+    // too large in this precision: nothing is built, which would take about 5 ms at 0.4 M rows (first
+    // FP64 solves that then took the separate kernels: 72³ hexes 10.8 → 6.2 ms, 724² quads 33.4 → 28.6)
+    if (widest > 27 || all < 1 || !res_may_fit(c, all, nz, fp32, s.nsys == 0)) return FEM_OK;
     o->state = -1;
     if ((rc = res_build(c, o, s, rows, nz, res_most_rows(nz, true)))) return rc;
     if (o->state == -1) return FEM_OK;

@@ -71,6 +71,18 @@ def test_rows_of_K(nel):
         _check(K, f, "mixed", "sell", "rows")
 
 
+@pytest.mark.parametrize("nel,kernels", [((71, 71, 71), "rows"), ((71, 71, 72), "separate"), ((72, 72, 72), "separate"),
+                                         ((715, 715), "rows"), ((724, 724), "separate")])
+def test_largest_rows_in_fp64(nel, kernels):
+    """Meshes about as large as the rows of K may be in FP64, and larger ones."""
+    print("case resident largest rows", nel, flush=True)
+    K, f = _poisson(nel, False)
+    A, b = K.to_scipy(), f.to_numpy()
+    one = fa.solve(K, f, mode="cg", rtol=1e-8)
+    assert one.kernels == kernels and one.operator == "sell"
+    assert np.linalg.norm(b - A @ one.u) <= 1.01e-8 * np.linalg.norm(b)
+
+
 @pytest.mark.parametrize("nel", [(15, 15), (24, 21), (71, 69), (7, 7, 7), (13, 12, 11), (40, 38, 36)])
 @pytest.mark.parametrize("operator", ["lattice", "cells"])
 def test_lattice_rows(nel, operator):
