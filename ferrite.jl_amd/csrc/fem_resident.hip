@@ -1143,6 +1143,7 @@ static int res_build(fem_ctx* c, ResOp* o, const ResSource& s, const ResRows& ro
     const int64_t nc = c->ncells, nd = c->ndpc, npc = c->npc;
     if (nd <= 0 || npc <= 0 || (int64_t)c->h_cell_dofs.size() != nc * nd || (int64_t)c->h_cell_nodes.size() != nc * npc)
       return FEM_OK;
+    if (c->ndofs != n) return FEM_OK;         // dofs uploaded after the pattern: not those of its rows
     std::vector<int32_t> node(n, 0), at(nd);
     std::vector<uint8_t> seen(n, 0);
     for (int64_t a = 0; a < nd; ++a) at[a] = (int32_t)(a * npc / nd);

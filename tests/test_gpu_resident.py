@@ -94,6 +94,22 @@ def test_lattice_rows(nel, operator):
         _check(K, f, mode, operator, "rows")
 
 
+def test_dofs_uploaded_after_the_pattern():
+    """The context's dofs are no longer those of K's rows (more of them): positions of the rows are not to
+    be had, and the separate kernels solve."""
+    print("case resident dofs uploaded after the pattern", flush=True)
+    K, _ = _poisson((12, 9), False, lattice=-1, cell_operator=-1)
+    A, n = K.to_scipy(), K.n
+    dofs = np.ascontiguousarray(2 * K.dh.cell_dofs, dtype=np.int64)
+    K.ctx.call("fem_dofs_upload", 2 * n, 4, dofs.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)))
+    b, u = np.ones(2 * n), np.zeros(2 * n)
+    pd = ctypes.POINTER(ctypes.c_double)
+    K.ctx.call("fem_matrix_upload", None, b.ctypes.data_as(pd))
+    assert fa.solve(K, None, mode="cg", rtol=1e-12, download=False).kernels == "separate"
+    K.ctx.call("fem_solution_download", u.ctypes.data_as(pd))
+    assert np.linalg.norm(b[:n] - A @ u[:n]) <= 2e-12 * np.linalg.norm(b[:n])
+
+
 @pytest.mark.parametrize("nel", [(90, 84, 80), (61, 140, 66), (200, 60, 50)])
 def test_cell_bricks(nel):
     """More rows than the entries of which fit on chip: bricks of the cell form (uneven cuts,
