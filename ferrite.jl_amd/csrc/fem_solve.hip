@@ -2750,6 +2750,7 @@ using namespace fem;
 extern "C" int32_t fem_solve(fem_ctx* c, const fem_solve_cfg* cfg, fem_solve_info* info) {
   if (!c || !cfg) return FEM_ERR_ARG;
   if (c->nnz == 0 || !c->d_f) return set_error(c, FEM_ERR_STATE, "assemble a system first");
+  if (c->n > c->ndofs) return set_error(c, FEM_ERR_STATE, "K has more rows than there are dofs: upload its pattern again");
   if (!(cfg->precond == 0 || cfg->precond == 1)) return set_error(c, FEM_ERR_ARG, "precond must be 0 or 1");
   FEM_HIP(c, hipSetDevice(c->device));
   const bool mixed = cfg->mode == FEM_SOLVE_IR_MIXED;

@@ -108,6 +108,12 @@ def test_dofs_uploaded_after_the_pattern():
     assert fa.solve(K, None, mode="cg", rtol=1e-12, download=False).kernels == "separate"
     K.ctx.call("fem_solution_download", u.ctypes.data_as(pd))
     assert np.linalg.norm(b[:n] - A @ u[:n]) <= 2e-12 * np.linalg.norm(b[:n])
+    # fewer dofs than K has rows: f and u are too short
+    few = np.minimum(K.dh.cell_dofs, n // 2)
+    few = np.ascontiguousarray(few, dtype=np.int64)
+    K.ctx.call("fem_dofs_upload", n // 2, 4, few.ctypes.data_as(ctypes.POINTER(ctypes.c_int64)))
+    with pytest.raises(fa.FemError, match="more rows than"):
+        fa.solve(K, None, mode="cg", download=False)
 
 
 @pytest.mark.parametrize("nel", [(90, 84, 80), (61, 140, 66), (200, 60, 50)])
