@@ -564,7 +564,6 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
     polls = a.polls;
     rl[zero] = X(0);
   }
-  auto polls_left = [&]() { return (uint32_t)uniform((int)polls); };
 
   // operator rows
   X av[RRES][NZ];
@@ -631,6 +630,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
       red[par][0][wave] = v0;
       red[par][1][wave] = v1;
     }
+    const uint32_t in_lds = polls;                  // (read before the barrier, which waits for it anyway)
     res_barrier();
     if (nb == 1) {
       irz = 1.0 / rzp;
@@ -646,6 +646,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
     }
     // the block's record: its two sums, one copy per group of readers (blocks ≡ b mod 8), so
     // that the reads of all blocks spread over the memory channels
+    const uint32_t most = (uint32_t)uniform((int)in_lds);
     const uint32_t rec = (uint32_t)(par * kResCopies * 2 * kResMaxBlocks);
     if (t < 2 * kResCopies) {
       double sum = 0.0;
@@ -670,7 +671,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
         for (int k = 0; k < H; ++k) {
           at[k] = wi + (uint32_t)hl[min(base + k * kResT + t, nh - 1)];   // (spare threads repeat the last row)
         }
-        for (uint32_t left = polls_left();; --left) {
+        for (uint32_t left = most;; --left) {
           asm volatile("" ::: "memory");
           bool ok = true;
           if (need) {
@@ -693,7 +694,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
       }
     }
     if (wave < (kResMaxBlocks + 63) / 64) {
-      for (uint32_t left = polls_left(); need; --left) {
+      for (uint32_t left = most; need; --left) {
         asm volatile("" ::: "memory");
         q0 = LL<double>::get(rr, rin);
         q1 = LL<double>::get(rr, rin + kResMaxBlocks);
@@ -746,7 +747,7 @@ __global__ __launch_bounds__(kResT) void k_resident(ResArgs<X> a) {
     for (int h = tt; h < nh; h += kResT) {
       const uint32_t at = (uint32_t)hl[h];
       U4 q = {};
-      for (uint32_t left = polls_left();; --left) {
+      for (uint32_t left = (uint32_t)uniform((int)polls);; --left) {
         asm volatile("" ::: "memory");
         q = LL<double>::get(ru, at);
         if (LL<double>::ok(q, ep)) break;

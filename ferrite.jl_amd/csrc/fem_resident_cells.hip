@@ -111,7 +111,6 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
     gaveup = 0;
     polls = a.polls;
   }
-  auto polls_left = [&]() { return (uint32_t)uniform((int)polls); };
   auto row_of = [&](int x, int y, int z) { return (x + 1) + a.px * (y + 1) + a.pxy * (z + 1); };   // padded row
 
   // coefficients of the cells whose first corner is one of (x0 − 1 .., y0 − 1 .., z0 − 1 ..)
@@ -197,7 +196,9 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
       red[par][0][wave] = v0;
       red[par][1][wave] = v1;
     }
+    const uint32_t in_lds = polls;                  // (read before the barrier, which waits for it anyway)
     res_barrier();
+    const uint32_t most = (uint32_t)uniform((int)in_lds);
     const uint32_t rec = (uint32_t)(par * kResCopies * 2 * kResMaxBlocks);
     if (t < 2 * kResCopies) {
       double sum = 0.0;
@@ -230,7 +231,7 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
       uint32_t q[H];
 #pragma unroll
       for (int k = 0; k < H; ++k) q[k] = at + hq[t + k * kResT];
-      for (uint32_t left = polls_left();; --left) {
+      for (uint32_t left = most;; --left) {
         asm volatile("" ::: "memory");
         bool ok = true;
         if (need) {
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(kResT) void k_resident_cells(BrickArgs a) {
         if (there >> k & 1u) hw[k] = LL<float>::val(hv[k]);
     }
     if (wave < (kResMaxBlocks + 63) / 64) {
-      for (uint32_t left = polls_left(); need; --left) {
+      for (uint32_t left = most; need; --left) {
         asm volatile("" ::: "memory");
         q0 = LL<double>::get(rr, rin);
         q1 = LL<double>::get(rr, rin + kResMaxBlocks);

@@ -145,7 +145,6 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
     gaveup = 0;
     polls = a.polls;
   }
-  auto polls_left = [&]() { return (uint32_t)uniform((int)polls); };
   res_barrier();
   auto spread = [&]() {                      // r̂ to the rows of the cells
 #pragma unroll
@@ -168,6 +167,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
       red[par][0][wave] = v0;
       red[par][1][wave] = v1;
     }
+    const uint32_t in_lds = polls;                  // (read before the barrier, which waits for it anyway)
     res_barrier();
     if (a.nb == 1) {
       irz = 1.0 / rzp;
@@ -181,6 +181,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
       ++ep;
       return true;
     }
+    const uint32_t most = (uint32_t)uniform((int)in_lds);
     const uint32_t rec = (uint32_t)(par * kResCopies * 2 * kResMaxBlocks);
     if (t < 2 * kResCopies) {
       double sum = 0.0;
@@ -199,7 +200,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
     if (halo && widest > 0) {          // (spare reads repeat a slot that is published)
       const uint32_t wi = (ep & 1u) * (uint32_t)a.nslots;
       typename LL<X>::W hv[kElShare];
-      for (uint32_t left = polls_left();; --left) {
+      for (uint32_t left = most;; --left) {
         asm volatile("" ::: "memory");
         bool ok = true;
         if (need) {
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(kResT) void k_resident_elems(ElemsArgs<X> a) {
       if (nfrom > 0) w = sum;
     }
     if (wave < (kResMaxBlocks + 63) / 64) {
-      for (uint32_t left = polls_left(); need; --left) {
+      for (uint32_t left = most; need; --left) {
         asm volatile("" ::: "memory");
         q0 = LL<double>::get(rr, rin);
         q1 = LL<double>::get(rr, rin + kResMaxBlocks);
